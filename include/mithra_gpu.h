@@ -343,8 +343,10 @@ int mithra_dev_set_reorder_interval(mithra_dev* dev, int interval);
 int mithra_dev_set_deterministic(mithra_dev* dev, int on);
 
 /* Tile shapes of the two marched field kernels (interior update, E/B evaluation): variant v
- * has `rows` x-rows of 64 y-nodes per workgroup and marches `planes` z-planes; variants 7-9
- * stage the interior update's A^n planes in LDS.  When no TF/SF seed is injected, the interior
+ * has `rows` x-rows of 64 y-nodes per workgroup and marches `planes` z-planes; variant 0 lays
+ * its rows end to end over the plane and marches fewer planes (at most eight, fewer on small
+ * meshes); variants 7-9 stage the interior update's A^n planes in LDS.  A domain starts with the
+ * shapes that suit its mesh and precision.  When no TF/SF seed is injected, the interior
  * update of every shape also updates the Mur y faces, which the boundary pass then skips.
  * Every shape computes identical values; only the speed differs. */
 #define MITHRA_TILE_VARIANTS 10
@@ -547,7 +549,8 @@ int mithra_dev_step_pipelined(mithra_dev* dev, double time, const mithra_seed* s
 /* 1 while a pipelined run is pending (the last step had more = 1 and was pipelined), else 0. */
 int mithra_dev_pipeline_pending(const mithra_dev* dev);
 /* Tile shapes of the pipelined step's fused kernel: `rows` x-rows of 64 y-nodes, `planes`
- * z-planes per workgroup; every shape computes identical values.  autotune_fused times each
+ * z-planes per workgroup (variant 0 on meshes under 5 million nodes: as variant 0 above); every
+ * shape computes identical values.  autotune_fused times each
  * (reps launches after one warm-up, ms[v] the mean) on the handle's current levels, keeps the
  * fastest and restores the level and the E/B array it writes.  No counterpart in the reference. */
 #define MITHRA_FUSED_TILE_VARIANTS 4

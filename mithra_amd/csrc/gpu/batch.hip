@@ -150,9 +150,9 @@ int build_tables(mithra_batch* b) {
     table(b->t_int[s], [&](int i, const BatchView& v) {
       if (v.nsfd == s) add(i, (long)v.tilesJ * v.tilesI * v.chunks * v.ncomp);
     });
-  table(b->t_eval, [&](int i, const BatchView& v) { add(i, (long)v.tilesJ * v.tilesI * v.chunks); });
+  table(b->t_eval, [&](int i, const BatchView& v) { add(i, (long)v.tilesJ * v.tilesI * v.echunks); });
   table(b->t_faces, [&](int i, const BatchView& v) {
-    add(i, v.ncomp * ((mur_face_count(v.N0, v.N1, v.N2, v.yfaces) + 255) / 256));
+    add(i, v.ncomp * ((mur_face_count(v.N0, v.N1, v.N2, v.faces) + 255) / 256));
   });
   table(b->t_edges, [&](int i, const BatchView& v) {
     const long ne = 4L * ((v.N2 - 2) + (v.N0 - 2) + (v.N1 - 2));
@@ -245,20 +245,38 @@ int upload_views(mithra_batch* b) {  // the host copies may change right after: 
   return MITHRA_OK;
 }
 
-void set_tile_geometry(BatchView& v, int variant) {
-  const int TI = kTileShapes[variant][0], K = kTileShapes[variant][1];
-  v.tilesJ = (v.N1 + 63) / 64;
-  v.tilesI = (v.N0 - 2 + TI - 1) / TI;
-  v.chunks = (v.N2 - 2 + K - 1) / K;
-  // without a TF/SF write between them, the interior kernels take the y faces
-  v.yfaces = v.seeded ? 0 : yface_mask(variant, v.N1);
+void set_tile_geometry(mithra_batch* b, int variant) {
+  long tile_planes[2] = {0, 0};  // shape 0: of the interior update and the E/B evaluation
+  for (const BatchView& v : b->hv) {
+    const long t = (long)flat_tiles(v.N0, v.N1) * (v.N2 - 2);
+    tile_planes[0] += t * v.ncomp;
+    tile_planes[1] += t;
+  }
+  for (BatchView& v : b->hv) {
+    if (variant == 0) {
+      v.planes = flat_planes(tile_planes[0]);
+      v.eplanes = flat_planes(tile_planes[1]);
+      v.tilesJ = 1;
+      v.tilesI = flat_tiles(v.N0, v.N1);
+    } else {
+      const int TI = kTileShapes[variant][0];
+      v.planes = v.eplanes = kTileShapes[variant][1];
+      v.tilesJ = (v.N1 + 63) / 64;
+      v.tilesI = (v.N0 - 2 + TI - 1) / TI;
+    }
+    v.chunks = (v.N2 - 2 + v.planes - 1) / v.planes;
+    v.echunks = (v.N2 - 2 + v.eplanes - 1) / v.eplanes;
+    // without a TF/SF write between them, the interior kernels take the Mur y faces
+    v.faces = v.seeded ? 0 : faces_mask(variant, v.N1);
+  }
 }
 
 int prepare(mithra_batch* b) {
   b->dep_lds = 0;
-  for (int i = 0; i < b->n; ++i) {
+  for (int i = 0; i < b->n; ++i)
     if (!b->ready[i]) return MITHRA_E_STATE;
-    set_tile_geometry(b->hv[i], b->variant);
+  set_tile_geometry(b, b->variant);
+  for (int i = 0; i < b->n; ++i) {
     const BatchView& v = b->hv[i];
     b->dep_lds = std::max(b->dep_lds, deposit_lds_bytes(v.ncomp, v.dTI, v.N1));
   }
@@ -544,7 +562,7 @@ int mithra_batch_autotune(mithra_batch* b, int reps, int* chosen, float* ms) {
   float best_ms = 0.0f;
   for (int v = 0; v < kTileVariants && !rc; ++v) {
     b->variant = v;
-    for (int i = 0; i < b->n; ++i) set_tile_geometry(b->hv[i], v);
+    set_tile_geometry(b, v);
     rc = upload_views(b);
     if (!rc) rc = build_tables(b);
     float total = 0.0f;
@@ -583,7 +601,7 @@ int mithra_batch_autotune(mithra_batch* b, int reps, int* chosen, float* ms) {
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   b->variant = rc ? keep : best;
-  for (int i = 0; i < b->n; ++i) set_tile_geometry(b->hv[i], b->variant);
+  set_tile_geometry(b, b->variant);
   if (!rc && chosen) *chosen = best;
   return rc;
 }

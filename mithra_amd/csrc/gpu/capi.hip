@@ -243,6 +243,9 @@ int mithra_dev_create(const mithra_grid* grid, const mithra_coeffs* coeffs, int 
   d->nodes = d->N1N0 * grid->N2;
   d->i_np1 = 0; d->i_n = 1; d->i_nm1 = 2;
   d->sort_interval = kDefaultSortInterval;
+  d->tile_interior = default_tile(d, 0);
+  d->tile_eval = default_tile(d, 1);
+  d->tile_fused = default_tile(d, 2);
   d->pk_lo = 1;
   d->pk_hi = 0;
   d->vk = -1;

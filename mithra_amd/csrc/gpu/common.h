@@ -52,18 +52,20 @@ struct MurCoeffs {
   double bB[5], cB[5], dB[5], eE[5], fE[5], gE[5], hC[17];
 };
 
-// Mur y faces (j = 0 and j = N1-1) that the interior kernels (every tile shape) update together
-// with the interior when no TF/SF write comes between the two: bit 0 the j = 0 face, bit 1 the
-// j = N1-1 face, the latter only when node N1-2 shares its 64-node tile row.
-__host__ __device__ inline int yface_mask(int, int N1) {
+// Mur y faces that the interior kernels update together with the interior when no TF/SF write
+// comes between the two: bit 0 the j = 0 face, bit 1 the j = N1-1 face.  The flat form (shape 0)
+// takes both when they have inward neighbours of their own, the tiled forms j = N1-1 only when
+// node N1-2 shares its 64-node tile row.
+__host__ __device__ inline int faces_mask(int variant, int N1) {
+  if (variant == 0) return N1 >= 4 ? 3 : 0;
   if (N1 < 3) return 0;
   return 1 | ((N1 - 1) % 64 != 0 ? 2 : 0);
 }
 
-// Face nodes the Mur face kernel updates: both x faces, the y faces not in `ymask`, both z faces.
-__host__ __device__ inline long mur_face_count(int N0, int N1, int N2, int ymask) {
+// Face nodes the Mur face kernel updates: both x faces, the y faces not in `mask`, both z faces.
+__host__ __device__ inline long mur_face_count(int N0, int N1, int N2, int mask) {
   const long ny = (long)(N0 - 2) * (N2 - 2);
-  return 2L * (long)(N1 - 2) * (N2 - 2) + ((ymask & 1) ? 0 : ny) + ((ymask & 2) ? 0 : ny) +
+  return 2L * (long)(N1 - 2) * (N2 - 2) + ((mask & 1) ? 0 : ny) + ((mask & 2) ? 0 : ny) +
          2L * (long)(N0 - 2) * (N1 - 2);
 }
 
@@ -225,7 +227,7 @@ struct Domain {
   int zrange_valid;         // zrange describes the current particle positions
   int pk_lo, pk_hi;         // power planes' cells (pk_lo > pk_hi: none)
   int zero_pending;         // the A^{n+1} buffer is logically zero (current_reset), not yet written
-  int yfaces_pending;       // Mur y faces the last interior launch updated (yface_mask bits)
+  int faces_pending;        // Mur y faces the last interior launch updated (faces_mask bits)
   double und_dist0;         // undulator[0].dist of the uploaded table (the emission flag's entry test)
   int sort_interval;        // deposits between reorders of the particle arrays (0: never)
   long sort_count;          // deposits since the particles were set
@@ -303,8 +305,10 @@ struct BatchView {
   int seeded;
   FieldSet lvl[3];
   float* eb;
-  int tilesJ, tilesI, chunks;  // interior / E-B tiles of the batch's tile shape
-  int yfaces;               // Mur y faces the interior kernels update (yface_mask of the tile shape)
+  int tilesJ, tilesI, chunks;  // interior / E-B tiles of the batch's tile shape (shape 0: tilesJ = 1)
+  int echunks;              // chunks of the E-B tiles
+  int planes, eplanes;      // shape 0: planes per interior / E-B entry
+  int faces;                // Mur y faces the interior kernels update (faces_mask of the tile shape)
   double a[6], alpha, beta;
   MurCoeffs mur;
   EvalConst ev;
@@ -349,9 +353,16 @@ struct BatchView {
 inline double* particle_array(Domain* d, int which) { return d->part + (size_t)which * d->cap; }
 
 // Launch helpers implemented in field.hip, particles.hip and power.hip.
-// fuse_yfaces: no TF/SF write follows, so the LDS-staged variants may update the Mur y faces
-// too; launch_boundaries then leaves them alone.
-hipError_t launch_interior(Domain* d, bool fuse_yfaces);
+// fuse_faces: no TF/SF write follows, so the interior update may take the Mur y faces (faces_mask)
+// with it; launch_boundaries then leaves them alone.
+hipError_t launch_interior(Domain* d, bool fuse_faces);
+// Workgroups over one plane of the flat form (shape 0), and its planes per workgroup given its
+// workgroups times planes.
+int flat_tiles(int N0, int N1);
+// Shape a domain starts with of the interior update (kernel 0), the E/B evaluation (1) and the
+// fused kernel of the pipelined step (2).
+int default_tile(const Domain* d, int kernel);
+int flat_planes(long tile_planes);
 hipError_t launch_tfsf(Domain* d, double time, const mithra_seed* seed);
 hipError_t launch_boundaries(Domain* d);
 hipError_t launch_eval_eb(Domain* d);

@@ -29,6 +29,9 @@ __device__ inline int xcd_logical_block(int b, int nblk) {
   return base + local;
 }
 
+template <typename PT>
+__device__ inline double rd(PT p, long m) { return (double)p[m]; }
+
 struct Plane5 {  // one z plane of a column and its four transverse neighbours
   double c, xp, xm, yp, ym;
 };
@@ -265,6 +268,132 @@ __global__ __launch_bounds__(kTileJ* TI) void k_interior_lds(
   interior_lds_body<R, NSFD, TI, K, FACES>(an_set, anm1_set, anp1_set, ncomp, N0, N1, N2, tilesJ, tilesI, chunks,
                                            a0, a1, a2, a3, a4, a5, alpha, beta,
                                            xcd_logical_block(blockIdx.x, gridDim.x), yf);
+}
+
+// ---- flat forms (tile shape 0) ---------------------------------------------------------------
+// Lanes run over the nodes of rows 1 .. N0-2 of a plane as one contiguous range (flat index
+// p = N1 i + j), so a mesh whose N1 is no multiple of 64 wastes only its two boundary columns of
+// lanes, and a workgroup marches only as many planes as leave the GPU its waves (flat_planes).
+// The transverse neighbours are other lanes' nodes, served by L1/L2; the z neighbours ride in
+// registers.  Same expressions, in the same order, as the tiled forms.
+//
+// What bounds the tiled forms on all but the largest meshes is the serial march of their 32-128
+// planes by too few workgroups, and lanes past N1; here it is HBM (71 x 71 x 397 nodes and up).
+// Interior update / E/B evaluation against the 4 x 64 tiles, us: 32 x 32 x 128 with phi, FP32
+// 56 / 74 -> 8 / 7; 71 x 71 x 397 FP32 82 / 123 -> 26 / 31, FP64 108 / 114 -> 41 / 45;
+// 128 x 128 x 1024 FP32 241 / 223 -> 163 / 218; 211 x 211 x 1531 FP64 1851 / 1610 -> 1528 / 1367.
+constexpr int kFlatThreads = 256;
+
+// A plane of a column and its transverse neighbours in the storage type.
+template <typename R>
+struct RawPlane {
+  R c, xp, xm, yp, ym;
+  __device__ inline Plane5 wide() const { return {(double)c, (double)xp, (double)xm, (double)yp, (double)ym}; }
+};
+
+template <typename R, typename PT>
+__device__ inline RawPlane<R> raw_plane(PT a, long m, long N1) {
+  return {a[m], a[m + N1], a[m - N1], a[m + 1], a[m - 1]};
+}
+
+// Tile, chunk and flat node of a flat workgroup; false for lanes without an interior node.
+struct FlatNode {
+  int kb, ke;    // planes
+  int i, j;
+  long m;        // node at plane kb
+};
+
+__device__ inline bool flat_node(int tile, int kc, int K, int klo, int khi, int N0, int N1, FlatNode& f) {
+  f.kb = klo + kc * K;
+  f.ke = min(f.kb + K, khi + 1);
+  const int p = N1 + tile * kFlatThreads + (int)threadIdx.x;
+  f.i = p / N1;
+  f.j = p - f.i * N1;
+  f.m = (long)N1 * N0 * f.kb + p;
+  return f.kb < f.ke && f.i <= N0 - 2 && f.j >= 1 && f.j <= N1 - 2;
+}
+
+// FACES: the threads of nodes j = 1 and j = N1-2 also update the Mur y face node beside them (mur_face
+// below with t along x, u along z).  Such a thread holds its own new value and A^{n-1} and all
+// of A^n that the face takes but two values; those and the face's A^{n-1} are loaded with the
+// prefetch, so that no load of the current plane's waits behind it.  Valid only when nothing writes
+// A^{n+1} between the interior update and the boundaries, and with N1 >= 4.
+template <typename R, bool NSFD, bool FACES>
+__device__ inline void interior_flat_body(FieldSet an_set, FieldSet anm1_set, FieldSet anp1_set, int ncomp, int N0,
+                                          int N1, int N2, int tiles, int chunks, int K, double a0, double a1,
+                                          double a2, double a3, double a4, double a5, double alpha, double beta,
+                                          int lb, const MurYFace& yf) {
+  const int tile = lb % tiles;
+  lb /= tiles;
+  const int kc = lb % chunks;
+  const int comp = lb / chunks;
+  FlatNode f;
+  if (comp >= ncomp || !flat_node(tile, kc, K, 1, N2 - 2, N0, N1, f)) return;
+  const bool face = FACES && (f.j == 1 || f.j == N1 - 2);
+  const int fs = f.j == 1 ? -1 : 1;  // offset of the face node
+  const gptr<const R> an = G((const R*)component(an_set, comp));
+  const gptr<const R> anm1 = G((const R*)component(anm1_set, comp));
+  const gptr<R> anp1 = G((R*)component(anp1_set, comp));
+  const double as = comp < 3 ? a4 : a5;
+  const long N1N0 = (long)N1 * N0;
+  long m = f.m;
+  // in the storage type until used: a conversion right after a load would wait for it there
+  RawPlane<R> pm = raw_plane<R>(an, m - N1N0, N1), p0 = raw_plane<R>(an, m, N1), pp = raw_plane<R>(an, m + N1N0, N1);
+  R v1 = ld_stream(anm1, m), src = ld_stream((gptr<const R>)anp1, m);
+  R fm = 0, fxp = 0, fxm = 0;  // the face node's A^{n-1} and its A^n neighbours along x
+  if (face) {
+    fm = anm1[m + fs];
+    fxp = an[m + fs + N1];
+    fxm = an[m + fs - N1];
+  }
+  for (int k = f.kb; k < f.ke; ++k, m += N1N0) {
+    RawPlane<R> pn = {};
+    R v1n = 0, srcn = 0, fmn = 0, fxpn = 0, fxmn = 0;
+    if (k + 1 < f.ke) {  // the next plane's loads go out before this plane's store
+      pn = raw_plane<R>(an, m + 2 * N1N0, N1);
+      v1n = ld_stream(anm1, m + N1N0);
+      srcn = ld_stream((gptr<const R>)anp1, m + N1N0);
+      if (face) {
+        fmn = anm1[m + N1N0 + fs];
+        fxpn = an[m + N1N0 + fs + N1];
+        fxmn = an[m + N1N0 + fs - N1];
+      }
+    }
+    const Plane5 qm = pm.wide(), q0 = p0.wide(), qp = pp.wide();
+    double r;
+    if (NSFD) {
+      const double tx = q0.xp + q0.xm + beta * (qp.xp + qm.xp + qp.xm + qm.xm);
+      const double ty = q0.yp + q0.ym + beta * (qp.yp + qm.yp + qp.ym + qm.ym);
+      r = a0 * q0.c - (double)v1 + alpha * (a1 * tx + a2 * ty) + a3 * (qp.c + qm.c) + as * (double)src;
+    } else {
+      r = a0 * q0.c - (double)v1 + a1 * (q0.xp + q0.xm) + a2 * (q0.yp + q0.ym) + a3 * (qp.c + qm.c) + as * (double)src;
+    }
+    st_stream(anp1, m, (R)r);
+    if (face) {
+      const double* B = yf.B;
+      const bool lo = fs < 0;
+      const double c = lo ? q0.ym : q0.yp, cp = lo ? qp.ym : qp.yp, cm = lo ? qm.ym : qm.yp;
+      anp1[m + fs] = (R)(B[0] * ((double)fm + (double)(R)r) + B[1] * (double)v1 + B[2] * (c + q0.c) +
+                         B[3] * (q0.xp + q0.xm + (double)fxp + (double)fxm) + B[4] * (qp.c + qm.c + cp + cm));
+    }
+    pm = p0;
+    p0 = pp;
+    pp = pn;
+    v1 = v1n;
+    src = srcn;
+    fm = fmn;
+    fxp = fxpn;
+    fxm = fxmn;
+  }
+}
+
+template <typename R, bool NSFD, bool FACES>
+__global__ __launch_bounds__(kFlatThreads) void k_interior_flat(FieldSet an, FieldSet anm1, FieldSet anp1, int ncomp,
+                                                                int N0, int N1, int N2, int tiles, int chunks, int K,
+                                                                double a0, double a1, double a2, double a3, double a4,
+                                                                double a5, double alpha, double beta, MurYFace yf) {
+  interior_flat_body<R, NSFD, FACES>(an, anm1, anp1, ncomp, N0, N1, N2, tiles, chunks, K, a0, a1, a2, a3, a4, a5,
+                                     alpha, beta, xcd_logical_block(blockIdx.x, gridDim.x), yf);
 }
 
 // ---- analytic seed (Signal::self src/classes.cpp:534-575, Seed::fields :740-855) --------
@@ -554,9 +683,6 @@ __global__ void k_seed_eval(mithra_seed s, const double* __restrict__ r, const d
 // node, o1 and o2 are the two inward offsets and w the offset along the edge.  For a corner,
 // sx, sy, sz are the three inward offsets.
 
-template <typename PT>
-__device__ inline double rd(PT p, long m) { return (double)p[m]; }
-
 template <typename TP, typename TN>
 __device__ inline double mur_face(const double* B, TP P, TN N, TN M, long m, long s, long t, long u) {
   return B[0] * (rd(M, m) + rd(P, m + s)) + B[1] * rd(M, m + s) + B[2] * (rd(N, m) + rd(N, m + s)) +
@@ -585,14 +711,14 @@ __device__ inline double mur_corner(const double* h, TP P, TN N, TN M, long m, l
 
 
 // All six faces in one launch: x faces (j, k), y faces (i, k), z faces (i, j), each min/max.
-// The y faces in `ymask` (yface_mask) were updated by the interior kernel and are skipped.
+// The faces in `mask` (faces_mask) were updated by the interior kernel and are skipped.
 template <typename R>
 __device__ inline void mur_faces_body(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2,
-                                      const MurCoeffs& c, long t, int comp, int ymask) {
+                                      const MurCoeffs& c, long t, int comp, int mask) {
   const long N1N0 = (long)N1 * N0;
   const long X = N1, Y = 1, Z = N1N0;
   const long nx = (long)(N1 - 2) * (N2 - 2), ny = (long)(N0 - 2) * (N2 - 2), nz = (long)(N0 - 2) * (N1 - 2);
-  const long nylo = (ymask & 1) ? 0 : ny, nyhi = (ymask & 2) ? 0 : ny;
+  const long nylo = (mask & 1) ? 0 : ny, nyhi = (mask & 2) ? 0 : ny;
   if (comp >= ncomp) return;
   const gptr<const R> pn = G((const R*)component(N, comp));
   const gptr<const R> pm = G((const R*)component(M, comp));
@@ -630,8 +756,8 @@ __device__ inline void mur_faces_body(FieldSet P, FieldSet N, FieldSet M, int nc
 
 template <typename R>
 __global__ void k_mur_faces(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2, MurCoeffs c,
-                           int ymask) {
-  mur_faces_body<R>(P, N, M, ncomp, N0, N1, N2, c, (long)blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, ymask);
+                           int mask) {
+  mur_faces_body<R>(P, N, M, ncomp, N0, N1, N2, c, (long)blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, mask);
 }
 
 // The twelve edges (second-order Mur only).
@@ -716,21 +842,10 @@ __device__ inline bool lazy_needed(int kb, int ke, const int* zr, int pb0, int p
 // Each thread owns one (i, j) column and marches K planes; the z neighbours of A_x and A_y (and
 // phi) at both time levels ride in a three-plane register queue, the transverse neighbours are
 // the centres of neighbouring lanes and rows.  Planes outside [klo, khi] are skipped.
-template <typename R, bool SC, int TI, int K>
-__device__ inline void eval_body(FieldSet An, FieldSet Ap, float* __restrict__ eb, int N0, int N1, int N2,
-                                 int tilesJ, int tilesI, int klo, int khi, const EvalConst& q,
-                                 const int* __restrict__ zr, int pb0, int pb1, int lb) {
+template <typename R, bool SC>
+__device__ inline void eval_march(FieldSet An, FieldSet Ap, float* __restrict__ eb, int N0, int N1, int N2, int kb,
+                                  int ke, long m, const EvalConst& q) {
   const gptr<f2> ebg = G(reinterpret_cast<f2*>(eb));
-  const int tj = lb % tilesJ;
-  lb /= tilesJ;
-  const int ti = lb % tilesI;
-  const int kc = lb / tilesI;
-  const int j = tj * kTileJ + (threadIdx.x % kTileJ);
-  const int i = 1 + ti * TI + (threadIdx.x / kTileJ);
-  const int kb = klo + kc * K;
-  const int ke = min(kb + K, khi + 1);
-  if (zr && !lazy_needed(kb, ke, zr, pb0, pb1)) return;
-  if (i > N0 - 2 || j < 1 || j > N1 - 2 || kb >= ke) return;
   const long N1N0 = (long)N1 * N0;
   const gptr<const R> n0 = G((const R*)An.c[0]);
   const gptr<const R> n1 = G((const R*)An.c[1]);
@@ -744,7 +859,6 @@ __device__ inline void eval_body(FieldSet An, FieldSet Ap, float* __restrict__ e
   auto dx_ = [&](double x) { return div_rn(x, dx2, q.rdx2); };
   auto dy_ = [&](double x) { return div_rn(x, dy2, q.rdy2); };
   auto dz_ = [&](double x) { return div_rn(x, dz2, q.rdz2); };
-  long m = N1N0 * kb + (long)N1 * i + j;
   // queue: [0] plane k-1, [1] plane k, [2] plane k+1
   double qn0[3], qn1[3], qp0[3], qp1[3], qf[3];
   for (int t = 0; t < 2; ++t) {
@@ -783,6 +897,44 @@ __device__ inline void eval_body(FieldSet An, FieldSet Ap, float* __restrict__ e
     qn0[1] = qn0[2]; qn1[1] = qn1[2]; qp0[1] = qp0[2]; qp1[1] = qp1[2];
     if (SC) { qf[0] = qf[1]; qf[1] = qf[2]; }
   }
+}
+
+template <typename R, bool SC, int TI, int K>
+__device__ inline void eval_body(FieldSet An, FieldSet Ap, float* __restrict__ eb, int N0, int N1, int N2,
+                                 int tilesJ, int tilesI, int klo, int khi, const EvalConst& q,
+                                 const int* __restrict__ zr, int pb0, int pb1, int lb) {
+  const int tj = lb % tilesJ;
+  lb /= tilesJ;
+  const int ti = lb % tilesI;
+  const int kc = lb / tilesI;
+  const int j = tj * kTileJ + (threadIdx.x % kTileJ);
+  const int i = 1 + ti * TI + (threadIdx.x / kTileJ);
+  const int kb = klo + kc * K;
+  const int ke = min(kb + K, khi + 1);
+  if (zr && !lazy_needed(kb, ke, zr, pb0, pb1)) return;
+  if (i > N0 - 2 || j < 1 || j > N1 - 2 || kb >= ke) return;
+  eval_march<R, SC>(An, Ap, eb, N0, N1, N2, kb, ke, (long)N1 * N0 * kb + (long)N1 * i + j, q);
+}
+
+// The flat form (see interior_flat_body).
+template <typename R, bool SC>
+__device__ inline void eval_flat_body(FieldSet An, FieldSet Ap, float* __restrict__ eb, int N0, int N1, int N2,
+                                      int tiles, int K, int klo, int khi, const EvalConst& q,
+                                      const int* __restrict__ zr, int pb0, int pb1, int lb) {
+  const int tile = lb % tiles, kc = lb / tiles;
+  FlatNode f;
+  if (!flat_node(tile, kc, K, klo, khi, N0, N1, f)) return;
+  if (zr && !lazy_needed(f.kb, f.ke, zr, pb0, pb1)) return;
+  eval_march<R, SC>(An, Ap, eb, N0, N1, N2, f.kb, f.ke, f.m, q);
+}
+
+template <typename R, bool SC>
+__global__ __launch_bounds__(kFlatThreads) void k_eval_flat(FieldSet An, FieldSet Ap, float* __restrict__ eb, int N0,
+                                                            int N1, int N2, int tiles, int K, int klo, int khi,
+                                                            EvalConst q, const int* __restrict__ zr, int pb0,
+                                                            int pb1) {
+  eval_flat_body<R, SC>(An, Ap, eb, N0, N1, N2, tiles, K, klo, khi, q, zr, pb0, pb1,
+                        xcd_logical_block(blockIdx.x, gridDim.x));
 }
 
 template <typename R, bool SC, int TI, int K>
@@ -1159,6 +1311,110 @@ __global__ __launch_bounds__(kTileJ* TI, SC ? 3 : kStencilWaves) void k_stencil_
   }
 }
 
+// The flat form of the fused kernel (see interior_flat_body): A^{n+1}'s three planes and their
+// neighbours in registers, A^n's transverse neighbours from L1/L2.
+template <typename R, bool NSFD, bool SC>
+__global__ __launch_bounds__(kFlatThreads) void k_stencil_eb_flat(FieldSet An1, FieldSet An, FieldSet X,
+                                                                  float* __restrict__ eb, int N0, int N1, int N2,
+                                                                  int tiles, int K, StencilConst s, EvalConst q,
+                                                                  const int* __restrict__ zr, int pb0, int pb1) {
+  constexpr int NC = SC ? 4 : 3;
+  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  FlatNode f;
+  if (!flat_node(lb % tiles, lb / tiles, K, 1, N2 - 2, N0, N1, f)) return;
+  const bool ebneed = !zr || lazy_needed(f.kb, f.ke, zr, pb0, pb1);
+  const gptr<f2> ebg = G(reinterpret_cast<f2*>(eb));
+  const long N1N0 = (long)N1 * N0;
+  gptr<const R> p[NC], n[NC];
+  gptr<R> x[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    p[c] = G((const R*)component(An1, c));
+    n[c] = G((const R*)component(An, c));
+    x[c] = G((R*)component(X, c));
+  }
+  const double mdt = q.mdt, dx2 = q.dx2, dy2 = q.dy2, dz2 = q.dz2;
+  auto dt_ = [&](double v) { return div_rn(v, mdt, q.rmdt); };
+  auto dx_ = [&](double v) { return div_rn(v, dx2, q.rdx2); };
+  auto dy_ = [&](double v) { return div_rn(v, dy2, q.rdy2); };
+  auto dz_ = [&](double v) { return div_rn(v, dz2, q.rdz2); };
+  long m = f.m;
+  RawPlane<R> rm[NC], r0[NC], rp[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    rm[c] = raw_plane<R>(p[c], m - N1N0, N1);
+    r0[c] = raw_plane<R>(p[c], m, N1);
+  }
+  // A^n_x, A^n_y (and phi^n) at planes k-1, k, k+1
+  double qx[3], qy[3], qf[3];
+  qx[0] = rd(n[0], m - N1N0); qx[1] = rd(n[0], m);
+  qy[0] = rd(n[1], m - N1N0); qy[1] = rd(n[1], m);
+  if (SC) { qf[0] = rd(n[NC - 1], m - N1N0); qf[1] = rd(n[NC - 1], m); }
+  for (int k = f.kb; k < f.ke; ++k, m += N1N0) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) rp[c] = raw_plane<R>(p[c], m + N1N0, N1);
+    qx[2] = rd(n[0], m + N1N0);
+    qy[2] = rd(n[1], m + N1N0);
+    if (SC) qf[2] = rd(n[NC - 1], m + N1N0);
+    const double qz = rd(n[2], m);
+    const double v1[4] = {qx[1], qy[1], qz, SC ? qf[1] : 0.0};
+    Plane5 pm[NC], p0[NC], pp[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      pm[c] = rm[c].wide();
+      p0[c] = r0[c].wide();
+      pp[c] = rp[c].wide();
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      double r;
+      if (NSFD) {
+        const double tx = p0[c].xp + p0[c].xm + s.beta * (pp[c].xp + pm[c].xp + pp[c].xm + pm[c].xm);
+        const double ty = p0[c].yp + p0[c].ym + s.beta * (pp[c].yp + pm[c].yp + pp[c].ym + pm[c].ym);
+        r = s.a0 * p0[c].c - v1[c] + s.alpha * (s.a1 * tx + s.a2 * ty) + s.a3 * (pp[c].c + pm[c].c);
+      } else {
+        r = s.a0 * p0[c].c - v1[c] + s.a1 * (p0[c].xp + p0[c].xm) + s.a2 * (p0[c].yp + p0[c].ym) +
+            s.a3 * (pp[c].c + pm[c].c);
+      }
+      st_stream(x[c], m, (R)r);
+    }
+    if (ebneed) {
+      double ex = dt_(p0[0].c) - dt_(qx[1]);
+      double ey = dt_(p0[1].c) - dt_(qy[1]);
+      float ez = (float)dt_(p0[2].c);
+      ez = (float)((double)ez - dt_(qz));
+      if (SC) {  // minus the gradient of phi^n
+        ex = ex - dx_(rd(n[NC - 1], m + N1) - rd(n[NC - 1], m - N1));
+        ey = ey - dy_(rd(n[NC - 1], m + 1) - rd(n[NC - 1], m - 1));
+        ez = (float)((double)ez - dz_(qf[2] - qf[0]));
+      }
+      const float bx = (float)(0.5 * (dy_(rd(n[2], m + 1) - rd(n[2], m - 1)) - dz_(qy[2] - qy[0]) +
+                                      dy_(p0[2].yp - p0[2].ym) - dz_(pp[1].c - pm[1].c)));
+      const float by = (float)(0.5 * (dz_(qx[2] - qx[0]) - dx_(rd(n[2], m + N1) - rd(n[2], m - N1)) +
+                                      dz_(pp[0].c - pm[0].c) - dx_(p0[2].xp - p0[2].xm)));
+      const float bz = (float)(0.5 * (dx_(rd(n[1], m + N1) - rd(n[1], m - N1)) - dy_(rd(n[0], m + 1) - rd(n[0], m - 1)) +
+                                      dx_(p0[1].xp - p0[1].xm) - dy_(p0[0].yp - p0[0].ym)));
+      const f2 v0 = {(float)ex, (float)ey}, vv1 = {ez, bx}, v2 = {by, bz};
+      auto put = [&](long node) {
+        st_stream(ebg, kEBPairs * node, v0);
+        st_stream(ebg, kEBPairs * node + 1, vv1);
+        st_stream(ebg, kEBPairs * node + 2, v2);
+      };
+      put(m);
+      if (k == 1) put(m - N1N0);
+      if (k == N2 - 2) put(m + N1N0);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      rm[c] = r0[c];
+      r0[c] = rp[c];
+    }
+    qx[0] = qx[1]; qx[1] = qx[2];
+    qy[0] = qy[1]; qy[1] = qy[2];
+    if (SC) { qf[0] = qf[1]; qf[1] = qf[2]; }
+  }
+}
+
 // ---- batched forms: persistent workgroups walking a table of (instance, local tile) ---------
 // Workgroup b takes entries r * G + l(b), r = 0, 1, ..., where l gives every XCD a contiguous
 // run of entries, so neighbouring tiles of one instance meet in one L2.
@@ -1175,14 +1431,14 @@ __global__ __launch_bounds__(kTileJ* TI) void kb_interior(const BatchView* __res
       if constexpr (LDS) {
         MurYFace yf;  // a local copy: stores to the potentials cannot alias it
         for (int q = 0; q < 5; ++q) yf.B[q] = v.mur.cB[q];
-        yf.mask = v.yfaces;
+        yf.mask = v.faces;
         interior_lds_body<R, NSFD, TI, K, true>(v.lvl[v.i_n], v.lvl[v.i_nm1], v.lvl[v.i_np1], v.ncomp, v.N0, v.N1,
                                                 v.N2, v.tilesJ, v.tilesI, v.chunks, v.a[0], v.a[1], v.a[2], v.a[3],
                                                 v.a[4], v.a[5], v.alpha, v.beta, e.y, yf);
       } else {
         MurYFace yf;
         for (int q = 0; q < 5; ++q) yf.B[q] = v.mur.cB[q];
-        yf.mask = v.yfaces;
+        yf.mask = v.faces;
         interior_body<R, NSFD, TI, K, true>(v.lvl[v.i_n], v.lvl[v.i_nm1], v.lvl[v.i_np1], v.ncomp, v.N0, v.N1, v.N2,
                                             v.tilesJ, v.tilesI, v.chunks, v.a[0], v.a[1], v.a[2], v.a[3], v.a[4],
                                             v.a[5], v.alpha, v.beta, e.y, yf);
@@ -1221,6 +1477,47 @@ __global__ __launch_bounds__(kTileJ* TI) void kb_eval(const BatchView* __restric
   }
 }
 
+// The flat forms: v.tilesI tiles of a plane, v.planes / v.eplanes planes per entry.
+template <typename R, bool NSFD>
+__global__ __launch_bounds__(kFlatThreads) void kb_interior_flat(const BatchView* __restrict__ V, BatchTiles T) {
+  for (int r = 0;; ++r) {
+    const int t = batch_entry(r);
+    if (t >= T.n) break;
+    const int2 e = T.t[t];
+    const BatchView& v = V[e.x];
+    if (!v.active) continue;
+    MurYFace yf;  // a local copy: stores to the potentials cannot alias it
+    for (int q = 0; q < 5; ++q) yf.B[q] = v.mur.cB[q];
+    yf.mask = v.faces;
+    if (v.faces)
+      interior_flat_body<R, NSFD, true>(v.lvl[v.i_n], v.lvl[v.i_nm1], v.lvl[v.i_np1], v.ncomp, v.N0, v.N1, v.N2,
+                                        v.tilesI, v.chunks, v.planes, v.a[0], v.a[1], v.a[2], v.a[3], v.a[4], v.a[5],
+                                        v.alpha, v.beta, e.y, yf);
+    else
+      interior_flat_body<R, NSFD, false>(v.lvl[v.i_n], v.lvl[v.i_nm1], v.lvl[v.i_np1], v.ncomp, v.N0, v.N1, v.N2,
+                                         v.tilesI, v.chunks, v.planes, v.a[0], v.a[1], v.a[2], v.a[3], v.a[4], v.a[5],
+                                         v.alpha, v.beta, e.y, yf);
+  }
+}
+
+template <typename R>
+__global__ __launch_bounds__(kFlatThreads) void kb_eval_flat(const BatchView* __restrict__ V, BatchTiles T) {
+  for (int r = 0;; ++r) {
+    const int t = batch_entry(r);
+    if (t >= T.n) break;
+    const int2 e = T.t[t];
+    const BatchView& v = V[e.x];
+    if (!v.active) continue;
+    const EvalConst q = v.ev;  // a local copy: stores to eb cannot alias it
+    if (v.ncomp == 4)
+      eval_flat_body<R, true>(v.lvl[v.i_n], v.lvl[v.i_np1], v.eb, v.N0, v.N1, v.N2, v.tilesI, v.eplanes, 1, v.N2 - 2,
+                              q, nullptr, 0, -1, e.y);
+    else
+      eval_flat_body<R, false>(v.lvl[v.i_n], v.lvl[v.i_np1], v.eb, v.N0, v.N1, v.N2, v.tilesI, v.eplanes, 1, v.N2 - 2,
+                               q, nullptr, 0, -1, e.y);
+  }
+}
+
 // TF/SF injection of the seeded instances, one axis per launch (the reference's order);
 // entry .y = block of 256 lines of the axis.
 template <typename R>
@@ -1248,10 +1545,10 @@ __global__ __launch_bounds__(256) void kb_mur(const BatchView* __restrict__ V, B
     if (!v.active) continue;
     const FieldSet P = v.lvl[v.i_np1], N = v.lvl[v.i_n], M = v.lvl[v.i_nm1];
     if (WHICH == 0) {
-      const long nf = mur_face_count(v.N0, v.N1, v.N2, v.yfaces);
+      const long nf = mur_face_count(v.N0, v.N1, v.N2, v.faces);
       const int nb = (int)((nf + 255) / 256);
       mur_faces_body<R>(P, N, M, v.ncomp, v.N0, v.N1, v.N2, v.mur, (long)(e.y % nb) * 256 + threadIdx.x, e.y / nb,
-                        v.yfaces);
+                        v.faces);
     } else if (WHICH == 1) {
       const long ne = 4L * ((v.N2 - 2) + (v.N0 - 2) + (v.N1 - 2));
       const int nb = (int)((ne + 255) / 256);
@@ -1272,9 +1569,72 @@ __global__ void k_fill_zero_bytes(unsigned char* p, size_t n) {
   if (t < n) p[t] = 0;
 }
 
+// Planes per workgroup of the flat forms for `tile_planes` workgroup-planes: eight, the fastest
+// from 64 x 64 x 512 nodes to 211 x 211 x 1531 (four and sixteen are within 4 %; thirty-two is
+// 20-50 % slower at 71 x 71 x 397), fewer while that leaves under 1024 workgroups, four for a CU:
+// 32 x 32 x 128 takes 9.9 us with eight planes and 7.7 with two, 45 x 45 x 203 13.4 and 12.1.
+int flat_planes_for(long tile_planes) {
+  int K = 8;
+  while (K > 1 && tile_planes / K < 1024) K /= 2;
+  return K;
+}
+
+EvalConst eval_const(const mithra_grid& g) {
+  EvalConst q;
+  q.mdt = -g.dt; q.dx2 = 2.0 * g.dx; q.dy2 = 2.0 * g.dy; q.dz2 = 2.0 * g.dz;
+  q.rmdt = 1.0 / q.mdt; q.rdx2 = 1.0 / q.dx2; q.rdy2 = 1.0 / q.dy2; q.rdz2 = 1.0 / q.dz2;
+  return q;
+}
+
+template <typename R, bool NSFD>
+hipError_t interior_flat_launch(Domain* d, int mask) {
+  const mithra_grid& g = d->g;
+  const int tiles = flat_tiles(g.N0, g.N1), K = flat_planes_for((long)tiles * (g.N2 - 2) * d->ncomp);
+  const int chunks = (g.N2 - 2 + K - 1) / K;
+  const dim3 grid((unsigned)((long)tiles * chunks * d->ncomp));
+  const double* a = d->co.a;
+  MurYFace yf;
+  for (int q = 0; q < 5; ++q) yf.B[q] = d->co.cB[q];
+  yf.mask = mask;
+  if (mask)
+    hipLaunchKernelGGL((k_interior_flat<R, NSFD, true>), grid, dim3(kFlatThreads), 0, d->stream, d->lvl[d->i_n],
+                       d->lvl[d->i_nm1], d->lvl[d->i_np1], d->ncomp, g.N0, g.N1, g.N2, tiles, chunks, K, a[0], a[1],
+                       a[2], a[3], a[4], a[5], d->co.alpha, d->co.beta, yf);
+  else
+    hipLaunchKernelGGL((k_interior_flat<R, NSFD, false>), grid, dim3(kFlatThreads), 0, d->stream, d->lvl[d->i_n],
+                       d->lvl[d->i_nm1], d->lvl[d->i_np1], d->ncomp, g.N0, g.N1, g.N2, tiles, chunks, K, a[0], a[1],
+                       a[2], a[3], a[4], a[5], d->co.alpha, d->co.beta, yf);
+  return hipGetLastError();
+}
+
+template <typename R, bool SC>
+hipError_t eval_flat_launch(Domain* d, int klo, int khi, const int* zr, int pb0, int pb1) {
+  const mithra_grid& g = d->g;
+  const int planes = khi - klo + 1, tiles = flat_tiles(g.N0, g.N1), K = flat_planes_for((long)tiles * planes);
+  const int chunks = (planes + K - 1) / K;
+  hipLaunchKernelGGL((k_eval_flat<R, SC>), dim3((unsigned)((long)tiles * chunks)), dim3(kFlatThreads), 0, d->stream,
+                     d->lvl[d->i_n], d->lvl[d->i_np1], d->eb, g.N0, g.N1, g.N2, tiles, K, klo, khi, eval_const(g), zr,
+                     pb0, pb1);
+  return hipGetLastError();
+}
+
+template <typename R, bool NSFD, bool SC>
+hipError_t stencil_eb_flat_launch(Domain* d, const int* zr, int pb0, int pb1) {
+  const mithra_grid& g = d->g;
+  const int tiles = flat_tiles(g.N0, g.N1), K = flat_planes_for((long)tiles * (g.N2 - 2));
+  const int chunks = (g.N2 - 2 + K - 1) / K;
+  const double* a = d->co.a;
+  const StencilConst s = {a[0], a[1], a[2], a[3], d->co.alpha, d->co.beta};
+  hipLaunchKernelGGL((k_stencil_eb_flat<R, NSFD, SC>), dim3((unsigned)((long)tiles * chunks)), dim3(kFlatThreads), 0,
+                     d->stream, d->lvl[d->i_np1], d->lvl[d->i_n], d->lvl[d->i_nm1], d->eb, g.N0, g.N1, g.N2, tiles, K,
+                     s, eval_const(g), zr, pb0, pb1);
+  return hipGetLastError();
+}
+
 // Tile shapes of the marched field kernels: rows of x per workgroup (one wavefront of 64 y
-// nodes per row) and z planes per workgroup.  Every shape computes the same values; the
-// autotuner (capi) picks the fastest per domain.
+// nodes per row) and z planes per workgroup.  Shape 0, the default, is the flat form: its four
+// wavefronts lie end to end over the plane, and it marches at most eight planes.  Every shape
+// computes the same values; the autotuner (capi) picks the fastest per domain.
 template <typename R, bool NSFD, int TI, int K, bool LDS = false>
 hipError_t interior_launch(Domain* d, int ymask) {
   const mithra_grid& g = d->g;
@@ -1314,9 +1674,7 @@ hipError_t eval_launch(Domain* d, int klo, int khi, const int* zr, int pb0, int 
   const int tilesI = (g.N0 - 2 + TI - 1) / TI;
   const int chunks = (khi - klo + 1 + K - 1) / K;
   const long nblk = (long)tilesJ * tilesI * chunks;
-  EvalConst q;
-  q.mdt = -g.dt; q.dx2 = 2.0 * g.dx; q.dy2 = 2.0 * g.dy; q.dz2 = 2.0 * g.dz;
-  q.rmdt = 1.0 / q.mdt; q.rdx2 = 1.0 / q.dx2; q.rdy2 = 1.0 / q.dy2; q.rdz2 = 1.0 / q.dz2;
+  const EvalConst q = eval_const(g);
   if constexpr (LDS)
     hipLaunchKernelGGL((k_eval_lds<R, SC, TI, K>), dim3((unsigned)nblk), dim3(kTileJ * TI), 0, d->stream,
                        d->lvl[d->i_n], d->lvl[d->i_np1], d->eb, g.N0, g.N1, g.N2, tilesJ, tilesI, klo, khi, q, zr, pb0, pb1);
@@ -1334,7 +1692,7 @@ hipError_t field_variant(Domain* d, int kernel, int v, int klo, int khi, const i
   case idx:                                                                                    \
     return kernel == 0 ? interior_launch<R, FLAG, TI, K>(d, ymask) : eval_launch<R, FLAG, TI, K>(d, klo, khi, zr, pb0, pb1);
   switch (v) {
-    MITHRA_VARIANT(0, 4, 64)
+    case 0: return kernel == 0 ? interior_flat_launch<R, FLAG>(d, ymask) : eval_flat_launch<R, FLAG>(d, klo, khi, zr, pb0, pb1);
     MITHRA_VARIANT(1, 2, 64)
     MITHRA_VARIANT(2, 4, 32)
     MITHRA_VARIANT(3, 4, 128)
@@ -1353,6 +1711,14 @@ hipError_t field_variant(Domain* d, int kernel, int v, int klo, int khi, const i
   return hipErrorInvalidValue;
 }
 
+// Below this many nodes the flat forms are the faster ones in FP64 too.  The tiled forms with LDS
+// planes read a node's neighbours once from L2 but march serially; they win once the
+// levels no longer fit the 256 MB last-level cache and the workgroups suffice.  us, flat against
+// tiled: fused kernel 32 x 32 x 128 with phi 12 / 163, 71 x 71 x 397 60 / 182, 90 x 90 x 301
+// 77 / 165, 128 x 128 x 1024 463 / 369; interior update 64 x 64 x 1024 135 / 142, 96 x 96 x 600
+// 172 / 167, 128 x 128 x 1024 453 / 370.
+constexpr long kFlatNodes = 5000000;
+
 template <typename R, bool NSFD, int TI, int K, bool SC>
 hipError_t stencil_eb_launch(Domain* d, const int* zr, int pb0, int pb1) {
   const mithra_grid& g = d->g;
@@ -1362,9 +1728,7 @@ hipError_t stencil_eb_launch(Domain* d, const int* zr, int pb0, int pb1) {
   const long nblk = (long)tilesJ * tilesI * chunks;
   const double* a = d->co.a;
   const StencilConst s = {a[0], a[1], a[2], a[3], d->co.alpha, d->co.beta};
-  EvalConst q;
-  q.mdt = -g.dt; q.dx2 = 2.0 * g.dx; q.dy2 = 2.0 * g.dy; q.dz2 = 2.0 * g.dz;
-  q.rmdt = 1.0 / q.mdt; q.rdx2 = 1.0 / q.dx2; q.rdy2 = 1.0 / q.dy2; q.rdz2 = 1.0 / q.dz2;
+  const EvalConst q = eval_const(g);
   hipLaunchKernelGGL((k_stencil_eb<R, NSFD, TI, K, SC>), dim3((unsigned)nblk), dim3(kTileJ * TI), 0, d->stream,
                      d->lvl[d->i_np1], d->lvl[d->i_n], d->lvl[d->i_nm1], d->eb, g.N0, g.N1, g.N2, tilesJ, tilesI, s,
                      q, zr, pb0, pb1);
@@ -1375,7 +1739,10 @@ template <typename R, bool NSFD, bool SC = false>
 hipError_t stencil_eb_variant(Domain* d, const int* zr, int pb0, int pb1) {
   static_assert(kFusedVariants == 4, "variant table and switch disagree");
   switch (d->tile_fused) {
-    case 0: return stencil_eb_launch<R, NSFD, 4, 64, SC>(d, zr, pb0, pb1);
+    // the flat form up to kFlatNodes, where it takes a third of the tiles' time (see there)
+    case 0:
+      if (d->nodes < kFlatNodes) return stencil_eb_flat_launch<R, NSFD, SC>(d, zr, pb0, pb1);
+      return stencil_eb_launch<R, NSFD, 4, 64, SC>(d, zr, pb0, pb1);
     case 1: return stencil_eb_launch<R, NSFD, 8, 64, SC>(d, zr, pb0, pb1);
     // under space charge 16-row tiles need more than the 128 registers a 1024-thread
     // workgroup allows (they spill): that variant runs the 8-row form
@@ -1403,12 +1770,12 @@ hipError_t stencil_eb_impl(Domain* d) {
 }
 
 template <typename R>
-hipError_t interior_impl(Domain* d, bool fuse_yfaces) {
-  const int ymask = fuse_yfaces ? yface_mask(d->tile_interior, d->g.N1) : 0;
+hipError_t interior_impl(Domain* d, bool fuse_faces) {
+  const int ymask = fuse_faces ? faces_mask(d->tile_interior, d->g.N1) : 0;
   const hipError_t e = d->g.solver == MITHRA_SOLVER_NSFD
                            ? field_variant<R, true>(d, 0, d->tile_interior, 0, 0, nullptr, 0, -1, ymask)
                            : field_variant<R, false>(d, 0, d->tile_interior, 0, 0, nullptr, 0, -1, ymask);
-  d->yfaces_pending = e == hipSuccess ? ymask : 0;
+  d->faces_pending = e == hipSuccess ? ymask : 0;
   return e;
 }
 
@@ -1479,11 +1846,11 @@ hipError_t boundaries_impl(Domain* d) {
   }
   for (int t = 0; t < 17; ++t) c.hC[t] = d->co.hC[t];
   FieldSet P = d->lvl[d->i_np1], N = d->lvl[d->i_n], M = d->lvl[d->i_nm1];
-  const int ymask = d->yfaces_pending;  // y faces the interior launch already updated
-  d->yfaces_pending = 0;
-  const long nf = mur_face_count(g.N0, g.N1, g.N2, ymask);
+  const int mask = d->faces_pending;  // faces the interior launch already updated
+  d->faces_pending = 0;
+  const long nf = mur_face_count(g.N0, g.N1, g.N2, mask);
   hipLaunchKernelGGL((k_mur_faces<R>), dim3((unsigned)((nf + 255) / 256), d->ncomp), dim3(256), 0, d->stream, P, N, M,
-                     d->ncomp, g.N0, g.N1, g.N2, c, ymask);
+                     d->ncomp, g.N0, g.N1, g.N2, c, mask);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || g.truncation_order != 2) return e;
   const long ne = 4L * ((g.N2 - 2) + (g.N0 - 2) + (g.N1 - 2));
@@ -1509,9 +1876,27 @@ hipError_t eval_impl(Domain* d, int klo, int khi, const int* zr = nullptr, int p
 extern const int kTileShapes[kTileVariants][2] = {{4, 64}, {2, 64}, {4, 32}, {4, 128}, {8, 32},
                                                   {8, 64}, {16, 32}, {4, 64}, {8, 64}, {16, 64}};
 
-hipError_t launch_interior(Domain* d, bool fuse_yfaces) {
-  return d->precision == MITHRA_PRECISION_FP64 ? interior_impl<double>(d, fuse_yfaces)
-                                               : interior_impl<float>(d, fuse_yfaces);
+// The shapes a domain starts with.  In FP32 the flat interior update is the fastest at every size
+// tried; in FP64 the LDS-staged 4 x 64 tiles from kFlatNodes on (see there).  The E/B evaluation
+// reads more neighbours: its LDS forms win from 8M nodes in FP64 (128 x 128 x 512 139 against
+// 165 us, 128 x 128 x 1024 263 / 323, 211 x 211 x 1531 1273 / 1357) and in FP32 from 16M nodes when
+// the 64-node rows of the tiles waste few lanes (128 x 128 x 1024 186 / 215; but 150 x 150 x 1000
+// 318 flat, 323 tiled).  The 8-row tiles fetch fewer halo rows, the 4-row ones suit ragged meshes.
+int default_tile(const Domain* d, int kernel) {
+  const int N1 = d->g.N1;
+  const bool f64 = d->precision == MITHRA_PRECISION_FP64, aligned = 10 * ((N1 + 63) / 64 * 64) < 11 * N1;
+  if (kernel == 0) return f64 && d->nodes >= kFlatNodes ? 7 : 0;
+  if (kernel == 1) return f64 ? (d->nodes < 8000000 ? 0 : aligned ? 8 : 7) : (d->nodes >= 16000000 && aligned ? 8 : 0);
+  return d->nodes >= kFlatNodes && aligned ? 1 : 0;  // the fused kernel
+}
+
+int flat_tiles(int N0, int N1) { return (int)(((long)N1 * (N0 - 2) + kFlatThreads - 1) / kFlatThreads); }
+
+int flat_planes(long tile_planes) { return flat_planes_for(tile_planes); }
+
+hipError_t launch_interior(Domain* d, bool fuse_faces) {
+  return d->precision == MITHRA_PRECISION_FP64 ? interior_impl<double>(d, fuse_faces)
+                                               : interior_impl<float>(d, fuse_faces);
 }
 
 extern const int kFusedShapes[kFusedVariants][2] = {{4, 64}, {8, 64}, {16, 64}, {8, 128}};
@@ -1577,7 +1962,13 @@ template <typename R>
 hipError_t batch_field_variant(BatchView* V, BatchTiles T, int kernel, int variant, int nsfd, hipStream_t s) {
   if (T.n == 0) return hipSuccess;
   switch (variant) {
-    case 0: return batch_field<R, 4, 64, false>(V, T, kernel, nsfd, s);
+    case 0: {
+      const dim3 g(batch_grid(T.n, 8)), b(kFlatThreads);
+      if (kernel == 1) hipLaunchKernelGGL((kb_eval_flat<R>), g, b, 0, s, V, T);
+      else if (nsfd) hipLaunchKernelGGL((kb_interior_flat<R, true>), g, b, 0, s, V, T);
+      else hipLaunchKernelGGL((kb_interior_flat<R, false>), g, b, 0, s, V, T);
+      return hipGetLastError();
+    }
     case 1: return batch_field<R, 2, 64, false>(V, T, kernel, nsfd, s);
     case 2: return batch_field<R, 4, 32, false>(V, T, kernel, nsfd, s);
     case 3: return batch_field<R, 4, 128, false>(V, T, kernel, nsfd, s);
