@@ -94,7 +94,7 @@ struct mithra_batch {
   // tables
   int2* tiles = nullptr;
   size_t tiles_cap = 0;
-  BatchTiles t_int[2], t_eval, t_faces, t_edges, t_corners, t_part, t_rows, t_inst, t_dep, t_pnodes, t_pred;
+  BatchTiles t_int[2], t_eval, t_faces, t_edges, t_corners, t_part, t_rows, t_inst, t_dep, t_pnodes;
   BatchTiles t_tfsf[3];             // TF/SF lines of the seeded instances, per axis
   size_t dep_lds = 0;
   bool prepared = false;
@@ -166,10 +166,7 @@ int build_tables(mithra_batch* b) {
   table(b->t_inst, [&](int i, const BatchView&) { add(i, 1); });
   table(b->t_dep, [&](int i, const BatchView& v) { add(i, deposit_blocks(v.N2, v.dtilesI, deposit_chunk())); });
   table(b->t_pnodes, [&](int i, const BatchView& v) {
-    if (v.pNz > 0 && v.N0 > 4 && v.N1 > 4) add(i, (long)v.pNz * v.pblocks);
-  });
-  table(b->t_pred, [&](int i, const BatchView& v) {
-    if (v.prows > 0) add(i, ((long)v.pN * v.pNl + 63) / 64);
+    if (v.pNz > 0 && v.pNl > 0 && v.N0 > 4 && v.N1 > 4) add(i, (long)v.pNz * v.pblocks);
   });
   for (int axis = 0; axis < 3; ++axis)
     table(b->t_tfsf[axis], [&](int i, const BatchView& v) {
@@ -190,7 +187,7 @@ int build_tables(mithra_batch* b) {
     BATCH_TRY(hipStreamSynchronize(b->stream));
   }
   BatchTiles* ts[] = {&b->t_int[0], &b->t_int[1], &b->t_eval, &b->t_faces,    &b->t_edges,   &b->t_corners,
-                      &b->t_part,   &b->t_rows,   &b->t_inst, &b->t_dep,      &b->t_pnodes,  &b->t_pred,
+                      &b->t_part,   &b->t_rows,   &b->t_inst, &b->t_dep,      &b->t_pnodes,
                       &b->t_tfsf[0], &b->t_tfsf[1], &b->t_tfsf[2]};
   for (BatchTiles* T : ts) T->t = b->tiles + (size_t)T->t;
   return MITHRA_OK;
@@ -207,7 +204,7 @@ int enqueue_step(mithra_batch* b) {
   BATCH_TRY(launch_batch_eval(V, b->t_eval, b->variant, p, s));
   BATCH_TRY(launch_batch_push(V, b->t_part, s));
   BATCH_TRY(launch_batch_bunching(V, b->t_part, b->t_inst, s));
-  BATCH_TRY(launch_batch_power(V, b->t_pnodes, b->t_pred, s));
+  BATCH_TRY(launch_batch_power(V, b->t_pnodes, s));
   hipLaunchKernelGGL(kb_shift, dim3((b->n + 63) / 64), dim3(64), 0, s, V, b->n);
   BATCH_TRY(hipGetLastError());
   BATCH_TRY(launch_batch_sort(V, b->t_part, b->t_rows, b->t_inst, 0, 0, s));
@@ -469,9 +466,10 @@ int mithra_batch_instance(mithra_batch* b, int i, double time, double time_bunch
   v.dft = d->dft;
   v.pk = d->pk;
   v.pdzr = d->pdzr;
+  v.psums = d->psums;
   v.partial = d->partial;
+  v.pdone = d->pdone;
   v.history = d->history;
-  v.plane_of = d->pk ? d->pk + d->pNz : nullptr;
   v.pNz = d->prows ? d->pNz : 0;
   v.pN = d->pN;
   v.pNl = d->pNl;

@@ -203,9 +203,9 @@ int level_of(const mithra_dev* d, int level) {
 
 void free_power(mithra_dev* d) {
   hipFree(d->pz); hipFree(d->pk); hipFree(d->pdzr); hipFree(d->dft); hipFree(d->ring);
-  hipFree(d->partial); hipFree(d->history);
+  hipFree(d->psums); hipFree(d->partial); hipFree(d->pdone); hipFree(d->history);
   d->pz = nullptr; d->pk = nullptr; d->pdzr = nullptr; d->dft = nullptr; d->ring = nullptr;
-  d->partial = nullptr; d->history = nullptr;
+  d->psums = nullptr; d->partial = nullptr; d->pdone = nullptr; d->history = nullptr;
   delete[] d->plane_of;
   d->plane_of = nullptr;
   d->prows = 0;
@@ -604,9 +604,17 @@ int mithra_dev_power_setup(mithra_dev* d, const mithra_power_params* p, unsigned
       hipMalloc(&d->dft, sizeof(double) * (dft.size() ? dft.size() : 1)) != hipSuccess ||
       hipMalloc(&d->ring, sizeof(double) * ring) != hipSuccess ||
       hipMalloc(&d->partial, sizeof(double) * (size_t)(nz ? nz : 1) * d->pblocks * (p->Nl ? p->Nl : 1)) != hipSuccess ||
+      hipMalloc(&d->pdone, sizeof(unsigned) * (nz ? nz : 1)) != hipSuccess ||
       hipMalloc(&d->history, sizeof(double) * (size_t)rows * (p->N ? p->N : 1) * (p->Nl ? p->Nl : 1)) != hipSuccess) {
     free_power(d);
     return MITHRA_E_NOMEM;
+  }
+  // The DFT's running sums, where they take at most half the ring's memory (16 doubles a node and
+  // frequency against 4 Nf a node) and it can be had; without them the sampler walks the ring.
+  const size_t sums = (size_t)16 * p->Nl * nz * d->N1N0;
+  if (sums && 2 * sums <= ring && hipMalloc(&d->psums, sizeof(double) * sums) != hipSuccess) {
+    (void)hipGetLastError();
+    d->psums = nullptr;
   }
   if (!kz.empty()) MITHRA_TRY(hipMemcpy(d->pk, kz.data(), sizeof(int) * kz.size(), hipMemcpyHostToDevice));
   if (nz) {
@@ -615,6 +623,8 @@ int mithra_dev_power_setup(mithra_dev* d, const mithra_power_params* p, unsigned
   }
   if (!dft.empty()) MITHRA_TRY(hipMemcpy(d->dft, dft.data(), sizeof(double) * dft.size(), hipMemcpyHostToDevice));
   MITHRA_TRY(launch_fill_zero(d, d->ring, sizeof(double) * ring));
+  if (d->psums) MITHRA_TRY(launch_fill_zero(d, d->psums, sizeof(double) * sums));
+  MITHRA_TRY(launch_fill_zero(d, d->pdone, sizeof(unsigned) * (nz ? nz : 1)));
   MITHRA_TRY(launch_fill_zero(d, d->history, sizeof(double) * (size_t)rows * (p->N ? p->N : 1) * (p->Nl ? p->Nl : 1)));
   d->prows = rows;
   return hip_status(hipStreamSynchronize(d->stream));

@@ -240,7 +240,9 @@ struct Domain {
   double* pdzr;             // device: plane fractional position
   double* dft;              // device: [Nl][Nf][4] = cos, sin  (ep = cos + i sin, em = cos - i sin)
   double* ring;             // device: [Nf][4][Nz][N1N0]
+  double* psums;            // device: each node's and frequency's DFT sums (power.hip), or nullptr
   double* partial;          // device: per-block partial sums
+  unsigned* pdone;          // device: per plane, workgroups that have finished (zero between launches)
   double* history;          // device: [rows][N][Nl]
   int pblocks;
   int* plane_of;            // host: for each of N planes, its index among inside planes or -1
@@ -333,12 +335,13 @@ struct BatchView {
   int dTI, dtilesI;         // row-tiled deposit geometry
   // power sampling
   double* ring;
+  double* psums;
   const double* dft;
   const int* pk;
   const double* pdzr;
   double* partial;
+  unsigned* pdone;
   double* history;
-  const int* plane_of;
   unsigned pNz, pN, pNl, pNf, prows;
   int pblocks;
   double pgamma, pbeta, pc0, pc;
@@ -414,7 +417,7 @@ hipError_t launch_batch_sort(BatchView* V, BatchTiles particles, BatchTiles rowb
                              int slot_sel, hipStream_t s);
 hipError_t launch_batch_deposit(BatchView* V, BatchTiles T, int precision, size_t lds, hipStream_t s);
 hipError_t launch_batch_reorder(BatchView* V, BatchTiles particles, hipStream_t s);
-hipError_t launch_batch_power(BatchView* V, BatchTiles nodes, BatchTiles reduce, hipStream_t s);
+hipError_t launch_batch_power(BatchView* V, BatchTiles nodes, hipStream_t s);
 int batch_grid(int ntiles, int per_cu);  // persistent grid size for a table of ntiles entries
 
 int deposit_tile_rows(const Domain* d);      // rows per tile of the row-tiled deposit (0: atomic path)
