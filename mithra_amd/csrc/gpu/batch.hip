@@ -94,7 +94,7 @@ struct mithra_batch {
   // tables
   int2* tiles = nullptr;
   size_t tiles_cap = 0;
-  BatchTiles t_int[2], t_eval, t_faces, t_edges, t_corners, t_part, t_rows, t_inst, t_dep, t_pnodes;
+  BatchTiles t_int[2], t_eval, t_faces, t_rims, t_part, t_rows, t_inst, t_dep, t_pnodes;
   BatchTiles t_tfsf[3];             // TF/SF lines of the seeded instances, per axis
   size_t dep_lds = 0;
   bool prepared = false;
@@ -154,12 +154,8 @@ int build_tables(mithra_batch* b) {
   table(b->t_faces, [&](int i, const BatchView& v) {
     add(i, v.ncomp * ((mur_face_count(v.N0, v.N1, v.N2, v.faces) + 255) / 256));
   });
-  table(b->t_edges, [&](int i, const BatchView& v) {
-    const long ne = 4L * ((v.N2 - 2) + (v.N0 - 2) + (v.N1 - 2));
-    if (v.trunc2) add(i, v.ncomp * ((ne + 255) / 256));
-  });
-  table(b->t_corners, [&](int i, const BatchView& v) {
-    if (v.trunc2) add(i, v.ncomp);
+  table(b->t_rims, [&](int i, const BatchView& v) {
+    if (v.trunc2) add(i, v.ncomp * mur_rim_blocks(v.N0, v.N1, v.N2));
   });
   table(b->t_part, [&](int i, const BatchView& v) { add(i, (v.np + 255) / 256); });
   table(b->t_rows, [&](int i, const BatchView& v) { add(i, ((long)v.rows + 1 + 1023) / 1024); });
@@ -186,7 +182,7 @@ int build_tables(mithra_batch* b) {
     BATCH_TRY(hipMemcpyAsync(b->tiles, all.data(), sizeof(int2) * all.size(), hipMemcpyHostToDevice, b->stream));
     BATCH_TRY(hipStreamSynchronize(b->stream));
   }
-  BatchTiles* ts[] = {&b->t_int[0], &b->t_int[1], &b->t_eval, &b->t_faces,    &b->t_edges,   &b->t_corners,
+  BatchTiles* ts[] = {&b->t_int[0], &b->t_int[1], &b->t_eval, &b->t_faces, &b->t_rims,
                       &b->t_part,   &b->t_rows,   &b->t_inst, &b->t_dep,      &b->t_pnodes,
                       &b->t_tfsf[0], &b->t_tfsf[1], &b->t_tfsf[2]};
   for (BatchTiles* T : ts) T->t = b->tiles + (size_t)T->t;
@@ -200,7 +196,7 @@ int enqueue_step(mithra_batch* b) {
   BATCH_TRY(launch_batch_interior(V, b->t_int[1], b->variant, p, 1, s));
   BATCH_TRY(launch_batch_interior(V, b->t_int[0], b->variant, p, 0, s));
   BATCH_TRY(launch_batch_tfsf(V, b->t_tfsf, p, s));
-  BATCH_TRY(launch_batch_mur(V, b->t_faces, b->t_edges, b->t_corners, p, s));
+  BATCH_TRY(launch_batch_mur(V, b->t_faces, b->t_rims, p, s));
   BATCH_TRY(launch_batch_eval(V, b->t_eval, b->variant, p, s));
   BATCH_TRY(launch_batch_push(V, b->t_part, s));
   BATCH_TRY(launch_batch_bunching(V, b->t_part, b->t_inst, s));
@@ -413,11 +409,7 @@ int mithra_batch_instance(mithra_batch* b, int i, double time, double time_bunch
   for (int t = 0; t < 6; ++t) v.a[t] = d->co.a[t];
   v.alpha = d->co.alpha;
   v.beta = d->co.beta;
-  for (int t = 0; t < 5; ++t) {
-    v.mur.bB[t] = d->co.bB[t]; v.mur.cB[t] = d->co.cB[t]; v.mur.dB[t] = d->co.dB[t];
-    v.mur.eE[t] = d->co.eE[t]; v.mur.fE[t] = d->co.fE[t]; v.mur.gE[t] = d->co.gE[t];
-  }
-  for (int t = 0; t < 17; ++t) v.mur.hC[t] = d->co.hC[t];
+  v.mur = mur_coeffs(d->co);
   v.ev.mdt = -g.dt; v.ev.dx2 = 2.0 * g.dx; v.ev.dy2 = 2.0 * g.dy; v.ev.dz2 = 2.0 * g.dz;
   v.ev.rmdt = 1.0 / v.ev.mdt; v.ev.rdx2 = 1.0 / v.ev.dx2; v.ev.rdy2 = 1.0 / v.ev.dy2; v.ev.rdz2 = 1.0 / v.ev.dz2;
   v.dt = g.dt;
@@ -572,7 +564,7 @@ int mithra_batch_autotune(mithra_batch* b, int reps, int* chosen, float* ms) {
       if (!rc) rc = status(hipEventRecord(e0, b->stream));
       if (!rc) rc = status(launch_batch_interior(b->V, b->t_int[1], v, b->precision, 1, b->stream));
       if (!rc) rc = status(launch_batch_interior(b->V, b->t_int[0], v, b->precision, 0, b->stream));
-      if (!rc) rc = status(launch_batch_mur(b->V, b->t_faces, b->t_edges, b->t_corners, b->precision, b->stream));
+      if (!rc) rc = status(launch_batch_mur(b->V, b->t_faces, b->t_rims, b->precision, b->stream));
       if (!rc) rc = status(launch_batch_eval(b->V, b->t_eval, v, b->precision, b->stream));
       if (!rc) rc = status(hipEventRecord(e1, b->stream));
       if (!rc) rc = status(hipEventSynchronize(e1));

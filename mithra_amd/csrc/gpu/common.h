@@ -69,6 +69,11 @@ __host__ __device__ inline long mur_face_count(int N0, int N1, int N2, int mask)
          2L * (long)(N0 - 2) * (N1 - 2);
 }
 
+// Workgroups of the Mur edges (256 nodes each) and corners (one) of a component.
+__host__ __device__ inline long mur_rim_blocks(int N0, int N1, int N2) {
+  return (4L * ((N2 - 2) + (N0 - 2) + (N1 - 2)) + 255) / 256 + 1;
+}
+
 // Streaming accesses: values read or written once per launch, marked nontemporal so they do
 // not displace reused lines (the stencil's A^n planes) from the caches.
 template <typename T>
@@ -355,6 +360,16 @@ struct BatchView {
 
 inline double* particle_array(Domain* d, int which) { return d->part + (size_t)which * d->cap; }
 
+inline MurCoeffs mur_coeffs(const mithra_coeffs& co) {
+  MurCoeffs c;
+  for (int t = 0; t < 5; ++t) {
+    c.bB[t] = co.bB[t]; c.cB[t] = co.cB[t]; c.dB[t] = co.dB[t];
+    c.eE[t] = co.eE[t]; c.fE[t] = co.fE[t]; c.gE[t] = co.gE[t];
+  }
+  for (int t = 0; t < 17; ++t) c.hC[t] = co.hC[t];
+  return c;
+}
+
 // Launch helpers implemented in field.hip, particles.hip and power.hip.
 // fuse_faces: no TF/SF write follows, so the interior update may take the Mur y faces (faces_mask)
 // with it; launch_boundaries then leaves them alone.
@@ -407,8 +422,7 @@ struct BatchTiles {
   int n;
 };
 hipError_t launch_batch_interior(BatchView* V, BatchTiles T, int variant, int precision, int nsfd, hipStream_t s);
-hipError_t launch_batch_mur(BatchView* V, BatchTiles faces, BatchTiles edges, BatchTiles corners, int precision,
-                            hipStream_t s);
+hipError_t launch_batch_mur(BatchView* V, BatchTiles faces, BatchTiles rims, int precision, hipStream_t s);
 hipError_t launch_batch_tfsf(BatchView* V, const BatchTiles* axes, int precision, hipStream_t s);  // axes[3]
 hipError_t launch_batch_eval(BatchView* V, BatchTiles T, int variant, int precision, hipStream_t s);
 hipError_t launch_batch_push(BatchView* V, BatchTiles T, hipStream_t s);

@@ -700,16 +700,6 @@ __device__ inline double mur_edge(const double* B, TP P, TN N, TN M, long m, lon
          rd(M, m + o3);
 }
 
-template <typename TP, typename TN>
-__device__ inline double mur_corner(const double* h, TP P, TN N, TN M, long m, long sx, long sy,
-                                    long sz) {
-  const long o[7] = {sx, sy, sz, sx + sy, sz + sx, sz + sy, sz + sx + sy};
-  double s = rd(N, m) * h[16] + rd(M, m) * h[8];
-  for (int t = 0; t < 7; ++t) s = s + rd(P, m + o[t]) * h[1 + t] + rd(N, m + o[t]) * h[16] + rd(M, m + o[t]) * h[9 + t];
-  return -s / h[0];
-}
-
-
 // All six faces in one launch: x faces (j, k), y faces (i, k), z faces (i, j), each min/max.
 // The faces in `mask` (faces_mask) were updated by the interior kernel and are skipped.
 template <typename R>
@@ -760,67 +750,85 @@ __global__ void k_mur_faces(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N
   mur_faces_body<R>(P, N, M, ncomp, N0, N1, N2, c, (long)blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, mask);
 }
 
-// The twelve edges (second-order Mur only).
+// The twelve edges and the eight corners (second-order Mur only) in one launch.  A corner reads the new
+// values of three edge nodes, which other threads of the launch store: it computes them again itself,
+// as the buffer holds them, one edge to a lane, so nothing waits for another thread.  A launch of
+// its own for the corners took 4-5 us of every step.  (Edges and corners that compute the faces again
+// too, in the faces' launch, gained 4 us more on 32 x 32 x 128 nodes and lost 4 us at 71 x 71 x 397,
+// where the faces' threads then have the edges' registers and index arithmetic.)
+
+// Value of edge node m along axis 2, 0 or 1 (`set`: 0 z, 1 x, 2 y), on the sides h1, h2 of the two axes
+// across it: x, y of z; y, z of x; z, x of y.
+template <typename R, typename TN, typename TP>
+__device__ inline double mur_edge_value(const MurCoeffs& c, TP P, TN N, TN M, long m, int set, bool h1, bool h2,
+                                        long X, long Z) {
+  double B[5];  // by selects, as in mur_faces_body
+#pragma unroll
+  for (int q = 0; q < 5; ++q) B[q] = set == 0 ? c.eE[q] : set == 1 ? c.fE[q] : c.gE[q];
+  const long s1 = set == 0 ? X : set == 1 ? 1 : Z, s2 = set == 0 ? 1 : set == 1 ? Z : X;
+  const long w = set == 0 ? Z : set == 1 ? X : 1;
+  return (double)(R)mur_edge(B, P, N, M, m, h1 ? -s1 : s1, h2 ? -s2 : s2, w);
+}
+
+// Block b of the pass: edges, 256 nodes each, and in the last one (b = nb - 1) the corners, four lanes
+// each: lanes 0-2 of a corner compute its edges along x, y, z, lane 0 the corner.
 template <typename R>
-__device__ inline void mur_edges_body(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2,
-                                      const MurCoeffs& c, long t, int comp) {
-  const long N1N0 = (long)N1 * N0;
-  const long X = N1, Y = 1, Z = N1N0;
-  const long ez = N2 - 2, ex = N0 - 2, ey = N1 - 2;
+__device__ inline void mur_rims_body(FieldSet Ps, FieldSet Ns, FieldSet Ms, int ncomp, int N0, int N1, int N2,
+                                     const MurCoeffs& c, int b, int nb, int comp) {
+  const long X = N1, Z = (long)N1 * N0;
   if (comp >= ncomp) return;
-  const gptr<const R> pn = G((const R*)component(N, comp));
-  const gptr<const R> pm = G((const R*)component(M, comp));
-  const gptr<R> pp = G((R*)component(P, comp));
-  long m, o1, o2, w;
-  int axis;
+  const gptr<const R> N = G((const R*)component(Ns, comp));
+  const gptr<const R> M = G((const R*)component(Ms, comp));
+  const gptr<R> P = G((R*)component(Ps, comp));
+  if (b == nb - 1) {
+    if (threadIdx.x >= 64) return;  // whole wavefronts: the corners take 32 lanes of the first
+    const int t = (threadIdx.x & 31) >> 2, a = (threadIdx.x & 3) < 3 ? threadIdx.x & 3 : 0;
+    const bool xh = t & 1, yh = t & 2, zh = t & 4;
+    const long m = (xh ? Z - X : 0) + (yh ? N1 - 1 : 0) + (zh ? Z * (N2 - 1) : 0);
+    const long sx = xh ? -X : X, sy = yh ? -1 : 1, sz = zh ? -Z : Z;
+    // edge along x: set 1, sides y, z; along y: set 2, sides z, x; along z: set 0, sides x, y
+    const double v = mur_edge_value<R>(c, P, N, M, m + (a == 0 ? sx : a == 1 ? sy : sz), a == 0 ? 1 : a == 1 ? 2 : 0,
+                                       a == 0 ? yh : a == 1 ? zh : xh, a == 0 ? zh : a == 1 ? xh : yh, X, Z);
+    const int base = __lane_id() & ~3;
+    const long o[7] = {sx, sy, sz, sx + sy, sz + sx, sz + sy, sz + sx + sy};
+    const double p[7] = {__shfl(v, base),  __shfl(v, base + 1), __shfl(v, base + 2), rd(P, m + o[3]),
+                         rd(P, m + o[4]), rd(P, m + o[5]),     rd(P, m + o[6])};
+    const double* h = c.hC;
+    double s = rd(N, m) * h[16] + rd(M, m) * h[8];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) s = s + p[q] * h[1 + q] + rd(N, m + o[q]) * h[16] + rd(M, m + o[q]) * h[9 + q];
+    if (threadIdx.x < 32 && (threadIdx.x & 3) == 0) P[m] = (R)(-s / h[0]);
+    return;
+  }
+  long t = (long)b * 256 + threadIdx.x, m;
+  const long ez = N2 - 2, ex = N0 - 2, ey = N1 - 2;
+  bool h1, h2;
+  int set;
   if (t < 4 * ez) {  // along z at the four (x, y) corners
     const int which = t / ez;
-    const long k = 1 + t % ez;
-    const bool xh = which & 1, yh = which & 2;
-    m = N1N0 * k + (xh ? (long)N1 * (N0 - 1) : 0) + (yh ? N1 - 1 : 0);
-    o1 = xh ? -X : X; o2 = yh ? -Y : Y; w = Z; axis = 0;
+    h1 = which & 1; h2 = which & 2;
+    m = Z * (1 + t % ez) + (h1 ? X * (N0 - 1) : 0) + (h2 ? N1 - 1 : 0);
+    set = 0;
   } else if ((t -= 4 * ez) < 4 * ex) {  // along x at the four (y, z) corners
     const int which = t / ex;
-    const long i = 1 + t % ex;
-    const bool yh = which & 1, zh = which & 2;
-    m = (long)N1 * i + (yh ? N1 - 1 : 0) + (zh ? N1N0 * (N2 - 1) : 0);
-    o1 = yh ? -Y : Y; o2 = zh ? -Z : Z; w = X; axis = 1;
+    h1 = which & 1; h2 = which & 2;
+    m = X * (1 + t % ex) + (h1 ? N1 - 1 : 0) + (h2 ? Z * (N2 - 1) : 0);
+    set = 1;
   } else if ((t -= 4 * ex) < 4 * ey) {  // along y at the four (z, x) corners
     const int which = t / ey;
-    const long j = 1 + t % ey;
-    const bool zh = which & 1, xh = which & 2;
-    m = j + (zh ? N1N0 * (N2 - 1) : 0) + (xh ? N1N0 - N1 : 0);
-    o1 = zh ? -Z : Z; o2 = xh ? -X : X; w = Y; axis = 2;
+    h1 = which & 1; h2 = which & 2;
+    m = 1 + t % ey + (h1 ? Z * (N2 - 1) : 0) + (h2 ? Z - X : 0);
+    set = 2;
   } else {
     return;
   }
-  double B[5];  // by selects, as in mur_faces_body
-#pragma unroll
-  for (int q = 0; q < 5; ++q) B[q] = axis == 0 ? c.eE[q] : axis == 1 ? c.fE[q] : c.gE[q];
-  pp[m] = (R)mur_edge(B, pp, pn, pm, m, o1, o2, w);
+  P[m] = (R)mur_edge_value<R>(c, P, N, M, m, set, h1, h2, X, Z);
 }
 
 template <typename R>
-__global__ void k_mur_edges(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2, MurCoeffs c) {
-  mur_edges_body<R>(P, N, M, ncomp, N0, N1, N2, c, (long)blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y);
-}
-
-template <typename R>
-__device__ inline void mur_corners_body(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2,
-                                        const MurCoeffs& c, int t, int comp) {
-  if (t >= 8 || comp >= ncomp) return;
-  const long N1N0 = (long)N1 * N0;
-  const bool xh = t & 1, yh = t & 2, zh = t & 4;
-  const long m = (xh ? N1N0 - N1 : 0) + (yh ? N1 - 1 : 0) + (zh ? N1N0 * (N2 - 1) : 0);
-  const gptr<const R> pn = G((const R*)component(N, comp));
-  const gptr<const R> pm = G((const R*)component(M, comp));
-  const gptr<R> pp = G((R*)component(P, comp));
-  pp[m] = (R)mur_corner(c.hC, pp, pn, pm, m, xh ? -(long)N1 : N1, yh ? -1L : 1L, zh ? -N1N0 : N1N0);
-}
-
-template <typename R>
-__global__ void k_mur_corners(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1, int N2, MurCoeffs c) {
-  mur_corners_body<R>(P, N, M, ncomp, N0, N1, N2, c, threadIdx.x, blockIdx.y);
+__global__ __launch_bounds__(256) void k_mur_rims(FieldSet P, FieldSet N, FieldSet M, int ncomp, int N0, int N1,
+                                                  int N2, MurCoeffs c) {
+  mur_rims_body<R>(P, N, M, ncomp, N0, N1, N2, c, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
 // E/B on every interior node (FdTd::fieldEvaluate src/fdtd.cpp:818-845, FdTdSC::fieldEvaluate
@@ -1534,8 +1542,8 @@ __global__ __launch_bounds__(256) void kb_tfsf(const BatchView* __restrict__ V, 
   }
 }
 
-// Mur faces / edges / corners: entry .y = comp * blocks_per_comp + block
-template <typename R, int WHICH>
+// Mur faces, or edges and corners: entry .y = comp * blocks_per_comp + block
+template <typename R, bool RIMS>
 __global__ __launch_bounds__(256) void kb_mur(const BatchView* __restrict__ V, BatchTiles T) {
   for (int r = 0;; ++r) {
     const int t = batch_entry(r);
@@ -1544,17 +1552,13 @@ __global__ __launch_bounds__(256) void kb_mur(const BatchView* __restrict__ V, B
     const BatchView& v = V[e.x];
     if (!v.active) continue;
     const FieldSet P = v.lvl[v.i_np1], N = v.lvl[v.i_n], M = v.lvl[v.i_nm1];
-    if (WHICH == 0) {
-      const long nf = mur_face_count(v.N0, v.N1, v.N2, v.faces);
-      const int nb = (int)((nf + 255) / 256);
+    if (RIMS) {
+      const int nb = (int)mur_rim_blocks(v.N0, v.N1, v.N2);
+      mur_rims_body<R>(P, N, M, v.ncomp, v.N0, v.N1, v.N2, v.mur, e.y % nb, nb, e.y / nb);
+    } else {
+      const int nb = (int)((mur_face_count(v.N0, v.N1, v.N2, v.faces) + 255) / 256);
       mur_faces_body<R>(P, N, M, v.ncomp, v.N0, v.N1, v.N2, v.mur, (long)(e.y % nb) * 256 + threadIdx.x, e.y / nb,
                         v.faces);
-    } else if (WHICH == 1) {
-      const long ne = 4L * ((v.N2 - 2) + (v.N0 - 2) + (v.N1 - 2));
-      const int nb = (int)((ne + 255) / 256);
-      mur_edges_body<R>(P, N, M, v.ncomp, v.N0, v.N1, v.N2, v.mur, (long)(e.y % nb) * 256 + threadIdx.x, e.y / nb);
-    } else {
-      mur_corners_body<R>(P, N, M, v.ncomp, v.N0, v.N1, v.N2, v.mur, threadIdx.x, e.y);
     }
   }
 }
@@ -1839,12 +1843,7 @@ hipError_t tfsf_impl(Domain* d, double time, const mithra_seed* seed) {
 template <typename R>
 hipError_t boundaries_impl(Domain* d) {
   const mithra_grid& g = d->g;
-  MurCoeffs c;
-  for (int t = 0; t < 5; ++t) {
-    c.bB[t] = d->co.bB[t]; c.cB[t] = d->co.cB[t]; c.dB[t] = d->co.dB[t];
-    c.eE[t] = d->co.eE[t]; c.fE[t] = d->co.fE[t]; c.gE[t] = d->co.gE[t];
-  }
-  for (int t = 0; t < 17; ++t) c.hC[t] = d->co.hC[t];
+  const MurCoeffs c = mur_coeffs(d->co);
   FieldSet P = d->lvl[d->i_np1], N = d->lvl[d->i_n], M = d->lvl[d->i_nm1];
   const int mask = d->faces_pending;  // faces the interior launch already updated
   d->faces_pending = 0;
@@ -1853,12 +1852,8 @@ hipError_t boundaries_impl(Domain* d) {
                      d->ncomp, g.N0, g.N1, g.N2, c, mask);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || g.truncation_order != 2) return e;
-  const long ne = 4L * ((g.N2 - 2) + (g.N0 - 2) + (g.N1 - 2));
-  hipLaunchKernelGGL((k_mur_edges<R>), dim3((unsigned)((ne + 255) / 256), d->ncomp), dim3(256), 0, d->stream, P, N, M,
-                     d->ncomp, g.N0, g.N1, g.N2, c);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL((k_mur_corners<R>), dim3(1, d->ncomp), dim3(64), 0, d->stream, P, N, M, d->ncomp, g.N0, g.N1,
-                     g.N2, c);
+  hipLaunchKernelGGL((k_mur_rims<R>), dim3((unsigned)mur_rim_blocks(g.N0, g.N1, g.N2), d->ncomp), dim3(256), 0,
+                     d->stream, P, N, M, d->ncomp, g.N0, g.N1, g.N2, c);
   return hipGetLastError();
 }
 
@@ -1887,7 +1882,7 @@ int default_tile(const Domain* d, int kernel) {
   const bool f64 = d->precision == MITHRA_PRECISION_FP64, aligned = 10 * ((N1 + 63) / 64 * 64) < 11 * N1;
   if (kernel == 0) return f64 && d->nodes >= kFlatNodes ? 7 : 0;
   if (kernel == 1) return f64 ? (d->nodes < 8000000 ? 0 : aligned ? 8 : 7) : (d->nodes >= 16000000 && aligned ? 8 : 0);
-  return d->nodes >= kFlatNodes && aligned ? 1 : 0;  // the fused kernel
+  return d->nodes >= 16000000 && aligned ? 1 : 0;  // the fused kernel
 }
 
 int flat_tiles(int N0, int N1) { return (int)(((long)N1 * (N0 - 2) + kFlatThreads - 1) / kFlatThreads); }
@@ -2007,20 +2002,17 @@ hipError_t launch_batch_tfsf(BatchView* V, const BatchTiles* axes, int precision
 }
 
 template <typename R>
-hipError_t batch_mur_impl(BatchView* V, BatchTiles F, BatchTiles E, BatchTiles C, hipStream_t s) {
-  if (F.n) hipLaunchKernelGGL((kb_mur<R, 0>), dim3(batch_grid(F.n, 8)), dim3(256), 0, s, V, F);
-  hipError_t e = hipGetLastError();
+hipError_t batch_mur_impl(BatchView* V, BatchTiles faces, BatchTiles rims, hipStream_t s) {
+  if (faces.n) hipLaunchKernelGGL((kb_mur<R, false>), dim3(batch_grid(faces.n, 8)), dim3(256), 0, s, V, faces);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (E.n) hipLaunchKernelGGL((kb_mur<R, 1>), dim3(batch_grid(E.n, 8)), dim3(256), 0, s, V, E);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (C.n) hipLaunchKernelGGL((kb_mur<R, 2>), dim3(batch_grid(C.n, 8)), dim3(64), 0, s, V, C);
+  if (rims.n) hipLaunchKernelGGL((kb_mur<R, true>), dim3(batch_grid(rims.n, 8)), dim3(256), 0, s, V, rims);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_mur(BatchView* V, BatchTiles faces, BatchTiles edges, BatchTiles corners, int precision,
-                            hipStream_t s) {
-  return precision == MITHRA_PRECISION_FP64 ? batch_mur_impl<double>(V, faces, edges, corners, s)
-                                            : batch_mur_impl<float>(V, faces, edges, corners, s);
+hipError_t launch_batch_mur(BatchView* V, BatchTiles faces, BatchTiles rims, int precision, hipStream_t s) {
+  return precision == MITHRA_PRECISION_FP64 ? batch_mur_impl<double>(V, faces, rims, s)
+                                            : batch_mur_impl<float>(V, faces, rims, s);
 }
 
 }  // namespace mithra
