@@ -160,7 +160,7 @@ int build_tables(mithra_batch* b) {
   table(b->t_part, [&](int i, const BatchView& v) { add(i, (v.np + 255) / 256); });
   table(b->t_rows, [&](int i, const BatchView& v) { add(i, ((long)v.rows + 1 + 1023) / 1024); });
   table(b->t_inst, [&](int i, const BatchView&) { add(i, 1); });
-  table(b->t_dep, [&](int i, const BatchView& v) { add(i, deposit_blocks(v.N2, v.dtilesI, deposit_chunk())); });
+  table(b->t_dep, [&](int i, const BatchView& v) { add(i, deposit_blocks(v.N2, v.dtilesI)); });
   table(b->t_pnodes, [&](int i, const BatchView& v) {
     if (v.pNz > 0 && v.pNl > 0 && v.N0 > 4 && v.N1 > 4) add(i, (long)v.pNz * v.pblocks);
   });

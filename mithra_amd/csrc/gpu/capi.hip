@@ -193,6 +193,7 @@ int run_step(mithra_dev* d, double time, const mithra_seed* seed, const mithra_b
   if (ms) {
     MITHRA_TRY(hipEventSynchronize(d->ev[8]));
     for (int i = 0; i < MITHRA_STEP_PHASES; ++i) MITHRA_TRY(hipEventElapsedTime(&ms[i], d->ev[i], d->ev[i + 1]));
+    if (pipe_in) ms[0] = 0.0f;  // the previous step marched A^{n+1}: only the events' own distance
   }
   return MITHRA_OK;
 }

@@ -435,8 +435,7 @@ hipError_t launch_batch_power(BatchView* V, BatchTiles nodes, hipStream_t s);
 int batch_grid(int ntiles, int per_cu);  // persistent grid size for a table of ntiles entries
 
 int deposit_tile_rows(const Domain* d);      // rows per tile of the row-tiled deposit (0: atomic path)
-long deposit_blocks(int N2, int tilesI, int KC);  // workgroups of the row-tiled deposit (row tiles x z chunks)
-int deposit_chunk();                         // z planes per chunk of the batched deposit
+long deposit_blocks(int N2, int tilesI);     // workgroups of the row-tiled deposit (row tiles x z chunks)
 size_t deposit_lds_bytes(int ncomp, int TI, int N1);  // its LDS per workgroup
 DepositConst make_deposit_const(const Domain* d);
 

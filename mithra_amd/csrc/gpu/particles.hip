@@ -642,9 +642,8 @@ __device__ inline void load_item(HalfItem& it, PT part, long cap, long p) {
   it.q = part[PQ * cap + p];
 }
 
-// Deposits one listed half into the two-plane tile ring of the marching deposit: its lower
-// node plane kc when kc >= kb, its upper one kc+1 when kc+1 < ke (slot = plane & 1, `psz`
-// doubles per slot).
+// Deposits one listed half into the tile of node planes kb .. ke-1 (`psz` doubles each): its lower
+// node plane kc when kc >= kb, its upper one kc+1 when kc+1 < ke.
 template <bool SC>
 __device__ inline void deposit_item(const HalfItem& it, const DepositConst& c, double* tile, int psz, int TI, int kb,
                                     int ke, int i0, int ti, int lo, int hi) {
@@ -674,7 +673,7 @@ __device__ inline void deposit_item(const HalfItem& it, const DepositConst& c, d
   for (int up = 0; up < 2; ++up) {
     const int k = kc + up;
     if (k < kb || k >= ke) continue;
-    double* t = tile + (k & 1) * psz;
+    double* t = tile + (k - kb) * psz;
     if (rho) add_plane<SC>(t, TI, c.N1, up, i0, ti, ic, jc, v);
     else add_plane<false>(t, TI, c.N1, up, i0, ti, ic, jc, v);
   }
@@ -787,25 +786,37 @@ __global__ __launch_bounds__(256) void k_deposit_fixed(FieldSet J, DepositConst 
   }
 }
 
-// Row-tiled current deposition, marching along z (same arithmetic per particle as k_deposit).
-// Workgroup b owns the J (and rho) values of rows i0 .. i0+ti-1, all j, of the node planes
-// kb .. ke-1 of its chunk of KC planes.  It walks the cell planes kc = kb-1 .. ke-1 in turn; the halves
-// listed under plane kc and rows i0-1 .. i0+ti-1 (two contiguous ranges, one per row order,
-// two halves in flight per thread) add their lower nodes to plane kc and their upper nodes to
-// plane kc+1 of a two-plane LDS ring, so each half is weighed once per workgroup.  Once plane
-// kc is complete it is written out and its slot starts plane kc+2.  Every node of the mesh
-// belongs to exactly one workgroup, so no global atomics are needed and the J buffer needs no
-// separate reset (`accumulate` = 0 writes the deposit alone, 1 adds it to what the buffer holds).
-constexpr int kDepositThreads = 512;
-constexpr int kDepositChunk = 4;  // node planes per workgroup (at most)
+// Row-tiled current deposition (same arithmetic per particle as k_deposit).  Workgroup b owns the J
+// (and rho) values of rows i0 .. i0+ti-1, all j, of the node planes kb .. ke-1 of its chunk of KC
+// planes, and holds them in LDS.  The halves listed under the cell planes kb-1 .. ke-1 and rows
+// i0-1 .. i0+ti-1 (a contiguous range per plane and order) are taken in one pass, two in flight per
+// thread; each is weighed once per workgroup and adds to whichever of its nodes the tile holds.  Then
+// the planes are written out.  Every node of the mesh belongs to exactly one workgroup, so no global
+// atomics are needed and the J buffer needs no separate reset (`accumulate` = 0 writes the deposit
+// alone, 1 adds it to what the buffer holds).
+//
+// What bounds it is the chain row starts -> list -> particle -> LDS adds -> barrier -> write, hidden
+// only by the other workgroups of the CU.  A form that marched along z through a two-plane ring, four
+// planes to a workgroup, ran that chain once per cell plane, with half of its threads idle in each
+// (the rows of a tile list some 250 halves a plane); one pass over the whole chunk runs it once, which
+// more than pays for the larger share of halves weighed in two chunks, (KC+1)/KC.  Deposit phase with
+// its order, us, marched -> in one pass: production (256 x 256 x 2048 nodes, 16.8M particles, FP64
+// pipelined) 2077 -> 1870, 128 x 128 x 1024 with rho and 4.2M particles 651 -> 540, 211 x 211 x 1531
+// FP32-bulk 703 -> 625, 128 x 128 x 1024 with 1M particles FP32-bulk 164 -> 131, 45 x 45 x 203 with rho
+// 44 -> 32.  Chunks of three, four and six planes in the same LDS are slower everywhere (more rows
+// weighed twice); so are tiles of 26, 52 and 79 KiB, but for space charge.
+constexpr int kDepositThreads = 512;  // at most
+constexpr int kDepositChunk = 2;      // node planes per workgroup
 
 template <typename R, bool SC, bool SRC = false>
 __device__ inline void deposit_rows_body(const double* __restrict__ part, long cap, FieldSet J, const DepositConst& c,
                                          const unsigned* __restrict__ p_row, const unsigned* __restrict__ p_idx,
                                          const unsigned* __restrict__ m_row, const unsigned* __restrict__ m_idx,
-                                         int TI, int tilesI, int KC, int accumulate, double src_coef,
+                                         int TI, int tilesI, int accumulate, double src_coef,
                                          double src_rho, int skip_empty, int block) {
-  extern __shared__ double tile[];  // [2][ncomp][TI][N1]
+  constexpr int KC = kDepositChunk;
+  extern __shared__ double tile[];  // [KC][ncomp][TI][N1]
+  __shared__ unsigned first[2 * (KC + 1)], upto[2 * (KC + 1)];
   constexpr int ncomp = SC ? 4 : 3;
   const int chunk = block / tilesI;
   const int i0 = (block - chunk * tilesI) * TI;
@@ -815,85 +826,91 @@ __device__ inline void deposit_rows_body(const double* __restrict__ part, long c
   const long N1N0 = (long)N1 * c.N0;
   const int tsz = TI * N1, psz = ncomp * tsz, own = ti * N1;
   const int lo = max(i0 - 1, 0), hi = min(i0 + ti - 1, c.N0 - 2);
-  // slot k & 1 := node plane k (the buffer's values with `accumulate` = 1, else zero)
   const bool add = accumulate == 1;
-  auto start_plane = [&](int k) {
-    double* p = tile + (k & 1) * psz;
+  // list 2 (kc - kb + 1) + h: the halves of cell plane kc = kb-1 .. ke-1, rows lo..hi, of order h (0: rnp,
+  // 1: rnm); upto: the halves in the lists up to and with it
+  const int lists = 2 * (ke - kb + 1);
+  if ((int)threadIdx.x < 64) {
+    const int l = threadIdx.x, kc = kb - 1 + (l >> 1);
+    unsigned n = 0, s = 0;
+    if (l < lists && lo <= hi && kc >= 0 && kc <= c.N2 - 2) {
+      const gptr<const unsigned> row = l & 1 ? G(m_row) : G(p_row);
+      const long r = (long)kc * c.N0;
+      s = row[r + lo];
+      n = row[r + hi + 1] - s;
+    }
+    unsigned sum = n;
+#pragma unroll
+    for (int d = 1; d < 2 * (KC + 1); d <<= 1) {
+      const unsigned up = __shfl_up(sum, d);
+      if (l >= d) sum += up;
+    }
+    if (l < lists) {
+      first[l] = s - (sum - n);  // entry t of the block is list entry first + t (modulo 2^32)
+      upto[l] = sum;
+    }
+  }
+  for (int k = kb; k < ke; ++k) {
+    double* p = tile + (k - kb) * psz;
     const long base = N1N0 * k + (long)N1 * i0;
     for (int o = threadIdx.x; o < own; o += blockDim.x) {
 #pragma unroll
       for (int comp = 0; comp < ncomp; ++comp)
         p[comp * tsz + o] = add ? (double)G((const R*)component(J, comp))[base + o] : 0.0;
     }
-  };
-  start_plane(kb);
-  if (kb + 1 < ke) start_plane(kb + 1);
+  }
   __syncthreads();
-  unsigned prev_total = 0;  // halves listed under the previous cell plane (this tile's rows)
-  for (int kc = kb - 1; kc < ke; ++kc) {
-    // the two ranges of cell plane kc: halves 0 (rnp order) and 1 (rnm order), rows lo..hi
-    unsigned s0 = 0, n0 = 0, s1 = 0, n1 = 0;
-    if (lo <= hi && kc >= 0 && kc <= c.N2 - 2) {
-      const long r = (long)kc * c.N0;
-      s0 = G(p_row)[r + lo];
-      n0 = G(p_row)[r + hi + 1] - s0;
-      s1 = G(m_row)[r + lo];
-      n1 = G(m_row)[r + hi + 1] - s1;
-    }
-    const unsigned total = n0 + n1;
-    auto locate = [&](unsigned t, HalfItem& it) {
-      it.half = t >= n0;
-      it.kk = kc;
-      return (long)(it.half ? G(m_idx)[s1 + (t - n0)] : G(p_idx)[s0 + t]);
-    };
-    for (unsigned t = threadIdx.x; t < total; t += 2 * blockDim.x) {
-      HalfItem a, b;
-      const unsigned tb = t + blockDim.x;
-      const long pa = locate(t, a);
-      b.ok = tb < total;
-      const long pb = b.ok ? locate(tb, b) : pa;
-      load_item(a, G(part), cap, pa);
-      load_item(b, G(part), cap, pb);
-      deposit_item<SC>(a, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
-      if (b.ok) deposit_item<SC>(b, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
-    }
-    __syncthreads();
-    // Node plane kc takes halves of cell planes kc-1 and kc only.  When neither lists any, its J
-    // (and rho) is +0, and in the pipelined form X + a4 J = X bit for bit when a4 (and a5, the
-    // coefficient of rho) carries a minus sign (a4 (+0) = -0, and x + -0 = x for every x, -0
-    // included), so that plane is left untouched.
-    const bool untouched = SRC && skip_empty && prev_total + total == 0;
-    prev_total = total;
-    if (kc >= kb) {  // node plane kc is complete: write it, and its slot becomes plane kc+2
-      double* p = tile + (kc & 1) * psz;
-      const long base = N1N0 * kc + (long)N1 * i0;
-      const bool next = kc + 2 < ke;
-      const bool inner_plane = kc >= 1 && kc <= c.N2 - 2 && !untouched;
-      // one node per thread and pass, its components unrolled: no index division per element
-      for (int o = threadIdx.x; o < own; o += blockDim.x) {
-        bool inner = false;
-        if (SRC) {
-          const int r = o / N1, jj = o - r * N1;
-          inner = inner_plane && i0 + r >= 1 && i0 + r <= c.N0 - 2 && jj >= 1 && jj <= N1 - 2;
-        }
+  const unsigned total = upto[lists - 1];
+  auto locate = [&](unsigned t, HalfItem& it) {
+    int l = 0;
+    while (t >= upto[l]) ++l;
+    it.half = l & 1;
+    it.kk = kb - 1 + (l >> 1);
+    return (long)(it.half ? G(m_idx) : G(p_idx))[first[l] + t];
+  };
+  for (unsigned t = threadIdx.x; t < total; t += 2 * blockDim.x) {
+    HalfItem a, b;
+    const unsigned tb = t + blockDim.x;
+    const long pa = locate(t, a);
+    b.ok = tb < total;
+    const long pb = b.ok ? locate(tb, b) : pa;
+    load_item(a, G(part), cap, pa);
+    load_item(b, G(part), cap, pb);
+    deposit_item<SC>(a, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
+    if (b.ok) deposit_item<SC>(b, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
+  }
+  __syncthreads();
+  for (int k = kb; k < ke; ++k) {
+    const int l = 2 * (k - kb);  // the lists of cell planes k-1 and k: l .. l+3
+    // Node plane k takes halves of cell planes k-1 and k only.  When neither lists any, its J (and rho) is
+    // +0, and in the pipelined form X + a4 J = X bit for bit when a4 (and a5, the coefficient of rho)
+    // carries a minus sign (a4 (+0) = -0, and x + -0 = x for every x, -0 included), so that plane is
+    // left untouched.
+    if (SRC && (k < 1 || k > c.N2 - 2 || (skip_empty && upto[l + 3] == (l ? upto[l - 1] : 0)))) continue;
+    const double* p = tile + (k - kb) * psz;
+    const long base = N1N0 * k + (long)N1 * i0;
+    // one node per thread and pass, its components unrolled: no index division per element
+    for (int o = threadIdx.x; o < own; o += blockDim.x) {
+      bool inner = false;
+      if (SRC) {
+        const int r = o / N1, jj = o - r * N1;
+        inner = i0 + r >= 1 && i0 + r <= c.N0 - 2 && jj >= 1 && jj <= N1 - 2;
+      }
 #pragma unroll
-        for (int comp = 0; comp < ncomp; ++comp) {
-          const gptr<R> out = G((R*)component(J, comp));
-          if (SRC) {
-            // the pipelined step: X + a4 J (and X + a5 rho for phi) at interior nodes, J rounded as
-            // the buffer would hold it
-            if (inner) {
-              const double xo = (double)ld_stream((gptr<const R>)out, base + o);  // read once, written once
-              const double coef = comp < 3 ? src_coef : src_rho;
-              st_stream(out, base + o, (R)(xo + coef * (double)(R)p[comp * tsz + o]));
-            }
-          } else {
-            out[base + o] = (R)p[comp * tsz + o];
+      for (int comp = 0; comp < ncomp; ++comp) {
+        const gptr<R> out = G((R*)component(J, comp));
+        if (SRC) {
+          // the pipelined step: X + a4 J (and X + a5 rho for phi) at interior nodes, J rounded as
+          // the buffer would hold it
+          if (inner) {
+            const double xo = (double)ld_stream((gptr<const R>)out, base + o);  // read once, written once
+            const double coef = comp < 3 ? src_coef : src_rho;
+            st_stream(out, base + o, (R)(xo + coef * (double)(R)p[comp * tsz + o]));
           }
-          if (next) p[comp * tsz + o] = add ? (double)G((const R*)component(J, comp))[base + 2 * N1N0 + o] : 0.0;
+        } else {
+          out[base + o] = (R)p[comp * tsz + o];
         }
       }
-      __syncthreads();
     }
   }
 }
@@ -902,8 +919,8 @@ template <typename R, bool SC, bool SRC = false>
 __global__ __launch_bounds__(kDepositThreads, SC ? 4 : 8) void k_deposit_rows(
     const double* __restrict__ part, long cap, FieldSet J, DepositConst c, const unsigned* __restrict__ p_row,
     const unsigned* __restrict__ p_idx, const unsigned* __restrict__ m_row, const unsigned* __restrict__ m_idx,
-    int TI, int tilesI, int KC, int accumulate, double src_coef, double src_rho, int skip_empty) {
-  deposit_rows_body<R, SC, SRC>(part, cap, J, c, p_row, p_idx, m_row, m_idx, TI, tilesI, KC, accumulate, src_coef,
+    int TI, int tilesI, int accumulate, double src_coef, double src_rho, int skip_empty) {
+  deposit_rows_body<R, SC, SRC>(part, cap, J, c, p_row, p_idx, m_row, m_idx, TI, tilesI, accumulate, src_coef,
                                 src_rho, skip_empty, blockIdx.x);
 }
 
@@ -1173,10 +1190,10 @@ __global__ __launch_bounds__(kDepositThreads) void kb_deposit(const BatchView* _
       const DepositConst c = v.dep;  // a local copy: the LDS atomics cannot alias it
       if (v.ncomp == 4)  // space charge: rho rides as the fourth component
         deposit_rows_body<R, true>(v.part, v.cap, v.lvl[v.i_np1], c, po.row, po.idx, mo.row, mo.idx, v.dTI,
-                                   v.dtilesI, kDepositChunk, 0, 0.0, 0.0, 0, e.y);
+                                   v.dtilesI, 0, 0.0, 0.0, 0, e.y);
       else
         deposit_rows_body<R, false>(v.part, v.cap, v.lvl[v.i_np1], c, po.row, po.idx, mo.row, mo.idx, v.dTI,
-                                    v.dtilesI, kDepositChunk, 0, 0.0, 0.0, 0, e.y);
+                                    v.dtilesI, 0, 0.0, 0.0, 0, e.y);
     }
     __syncthreads();  // the LDS tile is reused by the next entry
   }
@@ -1428,14 +1445,15 @@ hipError_t deposit_fixed_order(Domain* d, int accumulate, unsigned rows) {
   return hipGetLastError();
 }
 
-// Rows per workgroup tile of the row-tiled deposit: its two-plane LDS ring
-// (2 x ncomp x TI x N1 doubles) stays within 40 KiB, so four 512-thread workgroups (eight
-// waves per SIMD, the kernel's register budget) share a CU's 160 KiB; 0 when even one row does
-// not fit.
+// Rows per workgroup tile of the row-tiled deposit: its LDS (kDepositChunk x ncomp x TI x N1 doubles)
+// stays within 40 KiB, so four 512-thread workgroups (eight waves per SIMD, the kernel's register
+// budget) share a CU's 160 KiB, and with rho within 27 KiB for five of 256; 0 when even one row does not
+// fit in 40 KiB.
 int tile_rows(const Domain* d) {
-  const long per_row = 2L * d->ncomp * d->g.N1 * (long)sizeof(double);
-  const long fit = (40L << 10) / per_row;
-  return (int)std::min(fit, 16L);
+  const long per_row = (long)deposit_lds_bytes(d->ncomp, 1, d->g.N1), most = 40L << 10;
+  if (per_row > most) return 0;
+  const long budget = d->ncomp == 4 ? 27L << 10 : most - 128;  // 128: the lists' bounds beside the tile
+  return (int)std::max(1L, std::min(budget / per_row, 16L));
 }
 
 
@@ -1459,11 +1477,9 @@ hipError_t deposit_atomic(Domain* d) {
 
 int deposit_tile_rows(const Domain* d) { return tile_rows(d); }
 
-long deposit_blocks(int N2, int tilesI, int KC) { return (long)tilesI * ((N2 + KC - 1) / KC); }
+long deposit_blocks(int N2, int tilesI) { return (long)tilesI * ((N2 + kDepositChunk - 1) / kDepositChunk); }
 
-int deposit_chunk() { return kDepositChunk; }
-
-size_t deposit_lds_bytes(int ncomp, int TI, int N1) { return sizeof(double) * 2 * ncomp * TI * N1; }
+size_t deposit_lds_bytes(int ncomp, int TI, int N1) { return sizeof(double) * kDepositChunk * ncomp * TI * N1; }
 
 DepositConst make_deposit_const(const Domain* d) { return deposit_const(d); }
 
@@ -1506,26 +1522,28 @@ hipError_t launch_deposit(Domain* d, int accumulate) {
   if ((e = ensure_orders(d, rows)) != hipSuccess) return e;
   if (!d->rm_order_valid && (e = build_order(d, d->ord[1], 1, rows, nullptr)) != hipSuccess) return e;
   if ((e = build_order(d, d->ord[0], 0, rows, d->ord[1].idx)) != hipSuccess) return e;
-  // A single domain must fill the GPU by itself: shorter chunks, then fewer rows per tile,
-  // until there are some 2048 workgroups (each costs a little redundant work at its edges).
-  int TI = tile_rows(d), KC = kDepositChunk;
-  while (deposit_blocks(g.N2, (g.N0 + TI - 1) / TI, KC) < 2048) {
-    if (KC > 2) KC /= 2;
-    else if (TI > 1) TI = (TI + 1) / 2;
-    else break;
-  }
+  // A single domain must fill the GPU by itself: fewer rows per tile until there are some 2048
+  // workgroups (each costs a little redundant work at its edges).
+  int TI = tile_rows(d);
+  while (TI > 1 && deposit_blocks(g.N2, (g.N0 + TI - 1) / TI) < 2048) TI = (TI + 1) / 2;
   const int tilesI = (g.N0 + TI - 1) / TI;
   const DepositConst c = deposit_const(d);
   const FieldSet J = d->lvl[d->i_np1];
   const size_t lds = deposit_lds_bytes(d->ncomp, TI, g.N1);
-  const dim3 grid((unsigned)deposit_blocks(g.N2, tilesI, KC));
+  const long blocks = deposit_blocks(g.N2, tilesI);
+  const dim3 grid((unsigned)blocks);
+  // 256 threads where a workgroup has under 200 halves to weigh (more of them then share a CU: 32 x 32
+  // x 128 29.6 -> 25.2 us, 71 x 71 x 397 45.5 -> 40.7; with 265 halves at 90 x 90 x 301 60.6 -> 63.1),
+  // and with rho, whose registers leave five waves to a SIMD (4.2M particles 586 -> 524).
+  const double halves = 2.0 * d->np * (1.0 + 1.0 / kDepositChunk) * (1.0 + 1.0 / TI) / blocks;
+  const unsigned threads = c.sc || halves < 200.0 ? kDepositThreads / 2 : kDepositThreads;
   const unsigned *pr = d->ord[0].row, *pi = d->ord[0].idx, *mr = d->ord[1].row, *mi = d->ord[1].idx;
   const bool f64 = d->precision == MITHRA_PRECISION_FP64;
   // see deposit_rows_body: exact only when every source coefficient carries a minus sign
   const int skip = std::signbit(src_coef) && (!c.sc || std::signbit(src_rho)) ? 1 : 0;
 #define MITHRA_DEPOSIT(R_, SC_, SRC_)                                                                          \
-  hipLaunchKernelGGL((k_deposit_rows<R_, SC_, SRC_>), grid, dim3(kDepositThreads), lds, d->stream, d->part, d->cap, J, \
-                     c, pr, pi, mr, mi, TI, tilesI, KC, accumulate, src_coef, src_rho, skip)
+  hipLaunchKernelGGL((k_deposit_rows<R_, SC_, SRC_>), grid, dim3(threads), lds, d->stream, d->part, d->cap, J, \
+                     c, pr, pi, mr, mi, TI, tilesI, accumulate, src_coef, src_rho, skip)
   const bool src = accumulate == kDepositSource;
   if (f64) {
     if (c.sc) {
