@@ -260,8 +260,7 @@ int mithra_dev_create(const mithra_grid* grid, const mithra_coeffs* coeffs, int 
   if (hipMalloc(&d->pot_block, stride * 3 * d->ncomp) != hipSuccess ||
       hipMalloc(&d->eb, sizeof(float) * 2 * kEBPairs * (size_t)d->nodes) != hipSuccess ||
       hipMalloc(&d->counters, 2 * sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&d->zrange, 2 * sizeof(int)) != hipSuccess ||
-      hipMalloc(&d->zpart, 1024 * 2 * sizeof(int)) != hipSuccess) {
+      hipMalloc(&d->zrange, 2 * sizeof(int)) != hipSuccess) {
     mithra_dev_destroy(d);
     return MITHRA_E_NOMEM;
   }
@@ -427,9 +426,12 @@ int prepare_particles(mithra_dev* d, long n) {
   if (n > d->cap) {
     hipFree(d->part);
     hipFree(d->pid);
+    hipFree(d->zpart);
     free_sort(d);
     d->part = nullptr;
     d->pid = nullptr;
+    d->zpart = nullptr;
+    d->zpart_blocks = 0;
     d->cap = 0;
     // until the new arrays exist the domain holds no particles: a failed allocation below
     // must leave no launch reading the freed ones
@@ -439,8 +441,10 @@ int prepare_particles(mithra_dev* d, long n) {
     d->zrange_valid = 0;
     const long cap = (n + 63) / 64 * 64;
     if (hipMalloc(&d->part, sizeof(double) * PCOUNT * (size_t)cap) != hipSuccess ||
-        hipMalloc(&d->pid, sizeof(unsigned) * (size_t)cap) != hipSuccess) {
+        hipMalloc(&d->pid, sizeof(unsigned) * (size_t)cap) != hipSuccess ||
+        hipMalloc(&d->zpart, 2 * sizeof(int) * (size_t)((cap + 255) / 256)) != hipSuccess) {
       hipFree(d->part);
+      hipFree(d->pid);
       d->part = nullptr;
       d->pid = nullptr;
       return MITHRA_E_NOMEM;
@@ -452,6 +456,7 @@ int prepare_particles(mithra_dev* d, long n) {
   d->rm_order_valid = 0;  // no cell order describes the new particles yet
   d->order1_is_rnp = 0;
   d->zrange_valid = 0;    // nor a bunch extent
+  d->zpart_blocks = 0;
   return n ? hip_status(launch_particle_ids(d)) : MITHRA_OK;
 }
 

@@ -228,7 +228,8 @@ struct Domain {
   // sampler (planes pk_lo .. pk_hi + 1) read
   int lazy_fields;
   int* zrange;              // device: bunch z-cell extent after the last push
-  void* zpart;              // device: per-workgroup partial extents
+  void* zpart;              // device: the last push's extents per workgroup of 256 particles
+  int zpart_blocks;         // partial extents not yet reduced into zrange (0: none)
   int zrange_valid;         // zrange describes the current particle positions
   int pk_lo, pk_hi;         // power planes' cells (pk_lo > pk_hi: none)
   int zero_pending;         // the A^{n+1} buffer is logically zero (current_reset), not yet written
@@ -391,7 +392,7 @@ hipError_t launch_eval_eb_step(Domain* d);  // all planes, or the lazy subset wh
 hipError_t launch_stencil_eb(Domain* d);
 constexpr int kFusedVariants = 4;
 extern const int kFusedShapes[kFusedVariants][2];
-hipError_t launch_zrange(Domain* d);
+hipError_t launch_zrange(Domain* d);  // reduces what the last push left into zrange, unless a deposit has
 // Tile shapes {rows, planes} of the marched field kernels, selected by Domain::tile_*.
 constexpr int kTileVariants = 10;  // 7..9: LDS-staged interior update
 extern const int kTileShapes[kTileVariants][2];

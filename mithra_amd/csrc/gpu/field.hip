@@ -1763,6 +1763,7 @@ hipError_t stencil_eb_impl(Domain* d) {
   const int* zr = nullptr;
   int pb0 = 0, pb1 = -1;
   if (d->lazy_fields && d->zrange_valid) {
+    if (const hipError_t e = launch_zrange(d); e != hipSuccess) return e;
     zr = d->zrange;
     lazy_planes(d, &pb0, &pb1);
   }
@@ -1914,6 +1915,7 @@ hipError_t launch_eval_eb(Domain* d) { return launch_eval_eb_range(d, 1, d->g.N2
 
 hipError_t launch_eval_eb_step(Domain* d) {
   if (!d->lazy_fields || !d->zrange_valid) return launch_eval_eb(d);
+  if (const hipError_t e = launch_zrange(d); e != hipSuccess) return e;
   int pb0, pb1;
   lazy_planes(d, &pb0, &pb1);
   return d->precision == MITHRA_PRECISION_FP64 ? eval_impl<double>(d, 1, d->g.N2 - 2, d->zrange, pb0, pb1)

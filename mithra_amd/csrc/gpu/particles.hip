@@ -226,11 +226,11 @@ __device__ void undulator_field(const PushConst& c, UT und, const BeamDev* beams
 // E/B grid does not change between sub-steps, so a particle is read from HBM once per field
 // step and advanced n_sub times in registers; the time of each sub-step is accumulated exactly
 // as Solver::solve() accumulates timeBunch_ (src/solver.cpp:1316-1321).
+// Returns the particle's new z.
 template <bool BEAMS>
-__device__ inline void push_body(double* __restrict__ part, long cap, long n, const float* __restrict__ eb,
+__device__ inline double push_body(double* __restrict__ part, long cap, const float* __restrict__ eb,
                                  const UndDev* __restrict__ und, const BeamDev* __restrict__ beams, int n_opt,
                                  int n_ext, const PushConst& c, unsigned long long* __restrict__ counters, long p) {
-  if (p >= n) return;
   const gptr<double> X = G(part);
   const gptr<const f2> ebg = G(reinterpret_cast<const f2*>(eb));
   const gptr<const UndDev> undg = G(und);
@@ -341,65 +341,58 @@ __device__ inline void push_body(double* __restrict__ part, long cap, long n, co
   X[PE * cap + p] = e;
   if (nt) atomicAdd(&counters[0], (unsigned long long)nt);
   if (ncross) atomicAdd(&counters[1], (unsigned long long)ncross);
+  return z;
+}
+
+// z extent of the bunch in cells (clamped to the mesh), for the lazy E/B evaluation: the push leaves each
+// workgroup's min / max of its particles' new cells, and workgroup 0 of the pass that reads those
+// particles next, the deposit's keys, reduces them into zr[0..1] (without a deposit in between,
+// k_zcells_final does).  As two launches of their own the passes took 9 us of every step, and at 16.8M
+// particles read the positions again.
+__device__ inline void zcells_reduce(int lo, int hi, int2* out) {  // one workgroup of 256 threads
+  __shared__ int s_lo[4], s_hi[4];
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) {
+    lo = min(lo, __shfl_xor(lo, h));
+    hi = max(hi, __shfl_xor(hi, h));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_lo[threadIdx.x >> 6] = lo;
+    s_hi[threadIdx.x >> 6] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *out = make_int2(min(min(s_lo[0], s_lo[1]), min(s_lo[2], s_lo[3])), max(max(s_hi[0], s_hi[1]), max(s_hi[2], s_hi[3])));
+}
+
+__device__ inline void zcells_final(const int2* __restrict__ partial, int nb, int2* zr) {
+  int lo = 0x7fffffff, hi = -1;
+  for (int b = threadIdx.x; b < nb; b += 256) {
+    const int2 v = partial[b];
+    lo = min(lo, v.x);
+    hi = max(hi, v.y);
+  }
+  zcells_reduce(lo, hi, zr);
+}
+
+__global__ __launch_bounds__(256) void k_zcells_final(const int2* __restrict__ partial, int nb, int2* __restrict__ zr) {
+  zcells_final(partial, nb, zr);
 }
 
 template <bool BEAMS>
 __global__ __launch_bounds__(256) void k_push(double* __restrict__ part, long cap, long n,
                                               const float* __restrict__ eb, const UndDev* __restrict__ und,
                                               const BeamDev* __restrict__ beams, int n_opt, int n_ext, PushConst c,
-                                              unsigned long long* __restrict__ counters) {
-  push_body<BEAMS>(part, cap, n, eb, und, beams, n_opt, n_ext, c, counters,
-                   (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// z extent of the bunch in cells (clamped to the mesh), for the lazy E/B evaluation: per
-// workgroup min / max, then one workgroup reduces the partials into zr[0..1].
-constexpr int kZBlocks = 1024;
-
-__global__ __launch_bounds__(256) void k_zcells(const double* __restrict__ part, long cap, long n, double zmin,
-                                                double dz, double iz, int kmax_cell, int2* __restrict__ partial) {
-  __shared__ int s_lo[256], s_hi[256];
+                                              unsigned long long* __restrict__ counters, int2* __restrict__ zpart) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   int lo = 0x7fffffff, hi = -1;
-  for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (long)gridDim.x * blockDim.x) {
-    const double zz = floor(div_rn(part[PZ * cap + p] - zmin, dz, iz));
-    const int k = zz >= 0.0 ? (zz <= (double)kmax_cell ? (int)zz : kmax_cell) : 0;
-    lo = min(lo, k);
-    hi = max(hi, k);
+  if (p < n) {
+    const double z = push_body<BEAMS>(part, cap, eb, und, beams, n_opt, n_ext, c, counters, p);
+    const double zz = floor(div_rn(z - c.zmin, c.dz, c.iz));
+    const int most = c.N2 - 2;
+    lo = hi = zz >= 0.0 ? (zz <= (double)most ? (int)zz : most) : 0;
   }
-  s_lo[threadIdx.x] = lo;
-  s_hi[threadIdx.x] = hi;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      s_lo[threadIdx.x] = min(s_lo[threadIdx.x], s_lo[threadIdx.x + h]);
-      s_hi[threadIdx.x] = max(s_hi[threadIdx.x], s_hi[threadIdx.x + h]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = make_int2(s_lo[0], s_hi[0]);
-}
-
-__global__ __launch_bounds__(256) void k_zcells_final(const int2* __restrict__ partial, int nb, int* __restrict__ zr) {
-  __shared__ int s_lo[256], s_hi[256];
-  int lo = 0x7fffffff, hi = -1;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    lo = min(lo, partial[b].x);
-    hi = max(hi, partial[b].y);
-  }
-  s_lo[threadIdx.x] = lo;
-  s_hi[threadIdx.x] = hi;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      s_lo[threadIdx.x] = min(s_lo[threadIdx.x], s_lo[threadIdx.x + h]);
-      s_hi[threadIdx.x] = max(s_hi[threadIdx.x], s_hi[threadIdx.x + h]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    zr[0] = s_lo[0];
-    zr[1] = s_hi[0];
-  }
+  zcells_reduce(lo, hi, zpart + blockIdx.x);
 }
 
 __global__ void k_bunch_begin(double* __restrict__ part, long cap, long n) {
@@ -567,7 +560,9 @@ __global__ __launch_bounds__(256) void k_deposit(const double* __restrict__ part
 // With span = N1 - 1 the key is the cell, (k N0 + i) span + j, and the sentinel rows span.
 __global__ __launch_bounds__(256) void k_row_keys(const double* __restrict__ part, long cap, long n, DepositConst c,
                                                   int use_rm, unsigned rows, unsigned span, unsigned* __restrict__ key,
-                                                  unsigned* __restrict__ val) {
+                                                  unsigned* __restrict__ val, const int2* __restrict__ zpart,
+                                                  int zblocks, int2* __restrict__ zr) {
+  if (blockIdx.x == 0 && zblocks) zcells_final(zpart, zblocks, zr);
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int o = use_rm ? PXM : PX;
@@ -962,7 +957,8 @@ __global__ __launch_bounds__(256) void kb_push(BatchView* __restrict__ V, BatchT
     if (!v.active) continue;
     PushConst c = v.push;
     c.tb0 = v.time_bunch;
-    push_body<false>(v.part, v.cap, v.np, v.eb, v.und, nullptr, 0, 0, c, v.counters, (long)e.y * 256 + threadIdx.x);
+    const long p = (long)e.y * 256 + threadIdx.x;
+    if (p < v.np) push_body<false>(v.part, v.cap, v.eb, v.und, nullptr, 0, 0, c, v.counters, p);
   }
 }
 
@@ -1135,7 +1131,10 @@ __global__ __launch_bounds__(256) void kb_sort_scatter(BatchView* __restrict__ V
 // 1: the key of each listed particle (rnp, or rnm with use_rm) and the row counts.
 __global__ __launch_bounds__(256) void k_guided_keys(const double* __restrict__ part, long cap, long n, DepositConst c,
                                                      int use_rm, unsigned rows, const unsigned* __restrict__ guide,
-                                                     unsigned* __restrict__ key, unsigned* __restrict__ cnt) {
+                                                     unsigned* __restrict__ key, unsigned* __restrict__ cnt,
+                                                     const int2* __restrict__ zpart, int zblocks,
+                                                     int2* __restrict__ zr) {
+  if (blockIdx.x == 0 && zblocks) zcells_final(zpart, zblocks, zr);
   const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
   unsigned k = kNoKey;
   if (s < n) {
@@ -1287,18 +1286,11 @@ hipError_t launch_bunching(Domain* d, double k, double* partial, int blocks) {
 }
 
 hipError_t launch_zrange(Domain* d) {
-  d->zrange_valid = 0;
-  if (d->np == 0) return hipSuccess;
-  const mithra_grid& g = d->g;
-  const long want = (d->np + 255) / 256;
-  const int nb = (int)(want < kZBlocks ? want : kZBlocks);
-  hipLaunchKernelGGL(k_zcells, dim3(nb), dim3(256), 0, d->stream, d->part, d->cap, d->np, g.zmin, g.dz, 1.0 / g.dz,
-                     g.N2 - 2, (int2*)d->zpart);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_zcells_final, dim3(1), dim3(256), 0, d->stream, (const int2*)d->zpart, nb, d->zrange);
-  if ((e = hipGetLastError()) == hipSuccess) d->zrange_valid = 1;
-  return e;
+  if (!d->zpart_blocks) return hipSuccess;
+  hipLaunchKernelGGL(k_zcells_final, dim3(1), dim3(256), 0, d->stream, (const int2*)d->zpart, d->zpart_blocks,
+                     (int2*)d->zrange);
+  d->zpart_blocks = 0;
+  return hipGetLastError();
 }
 
 hipError_t launch_bunch_begin(Domain* d) {
@@ -1325,15 +1317,20 @@ hipError_t launch_push(Domain* d, const mithra_bunch_params* p, const UndDev* un
   c.tb0 = time_bunch; c.dtb_time = bunch_time_step;
   c.n_sub = n_sub; c.n_und = n_und; c.save_rnm = save_rnm;
   c.dist0 = n_und > 0 ? d->und_dist0 : 0.0;  // kept at upload: `und` is device memory
+  const unsigned blocks = (unsigned)((d->np + 255) / 256);
+  d->zrange_valid = 0;
   if (d->n_opt + d->n_ext > 0)
-    hipLaunchKernelGGL(k_push<true>, dim3((unsigned)((d->np + 255) / 256)), dim3(256), 0, d->stream, d->part, d->cap,
-                       d->np, d->eb, und, d->beams, d->n_opt, d->n_ext, c, d->counters);
+    hipLaunchKernelGGL(k_push<true>, dim3(blocks), dim3(256), 0, d->stream, d->part, d->cap, d->np, d->eb, und,
+                       d->beams, d->n_opt, d->n_ext, c, d->counters, (int2*)d->zpart);
   else
-    hipLaunchKernelGGL(k_push<false>, dim3((unsigned)((d->np + 255) / 256)), dim3(256), 0, d->stream, d->part,
-                       d->cap, d->np, d->eb, und, nullptr, 0, 0, c, d->counters);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return launch_zrange(d);
+    hipLaunchKernelGGL(k_push<false>, dim3(blocks), dim3(256), 0, d->stream, d->part, d->cap, d->np, d->eb, und,
+                       nullptr, 0, 0, c, d->counters, (int2*)d->zpart);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) {
+    d->zrange_valid = 1;
+    d->zpart_blocks = (int)blocks;
+  }
+  return e;
 }
 
 // Cells of the fixed-order deposit's keys: (N2 - 1) N0 rows of N1 - 1 cells (0 when they do
@@ -1365,13 +1362,15 @@ hipError_t build_order(Domain* d, CellOrder& o, int use_rm, unsigned rows, const
   if (d->deterministic) {
     const unsigned span = (unsigned)(c.N1 - 1);  // cells
     hipLaunchKernelGGL(k_row_keys, dim3(grid), dim3(256), 0, d->stream, d->part, d->cap, d->np, c, use_rm, rows,
-                       span, o.key, o.idx);
+                       span, o.key, o.idx, (const int2*)d->zpart, d->zpart_blocks, (int2*)d->zrange);
     if ((e = hipGetLastError()) != hipSuccess) return e;
+    d->zpart_blocks = 0;
     return sort_order(d, o, d->np, rows, span);
   }
   hipLaunchKernelGGL(k_guided_keys, dim3(grid), dim3(256), 0, d->stream, d->part, d->cap, d->np, c, use_rm, rows,
-                     guide, d->key_alt, d->row_cnt);
+                     guide, d->key_alt, d->row_cnt, (const int2*)d->zpart, d->zpart_blocks, (int2*)d->zrange);
   if ((e = hipGetLastError()) != hipSuccess) return e;
+  d->zpart_blocks = 0;
   if ((e = scan_row_counts(d, d->row_cnt, o.row, rows)) != hipSuccess) {
     (void)launch_fill_zero(d, d->row_cnt, sizeof(unsigned) * ((size_t)rows + 1));  // counts zero again
     return e;

@@ -76,6 +76,51 @@ __global__ __launch_bounds__(256) void k_cell_start(const unsigned* __restrict__
   cell_start[c] = (unsigned)lo;
 }
 
+// Exclusive scan of the row counts (n entries) in one launch: a workgroup scans its kScanChunk entries
+// and adds up all the entries before them itself, so no workgroup waits for another and nothing has to
+// be initialised.  rocPRIM's look-back scan is two launches, 4.5-5 us each on small meshes; the sums'
+// reads grow with the square of n, to 16 KB a thread-row at kScanMost, where the two are even (LARGE).
+constexpr int kScanThreads = 1024, kScanChunk = 4 * kScanThreads;
+constexpr unsigned kScanMost = 1u << 17;
+
+__global__ __launch_bounds__(kScanThreads) void k_scan_counts(const unsigned* __restrict__ cnt, unsigned n,
+                                                              unsigned* __restrict__ out) {
+  __shared__ unsigned wave_sum[kScanThreads / 64], before[kScanThreads / 64];
+  const unsigned first = blockIdx.x * kScanChunk, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  unsigned sum = 0;
+  // whole chunks only lie before this one; the arrays are 256-byte aligned
+#pragma unroll 8
+  for (unsigned i = 4 * threadIdx.x; i < first; i += kScanChunk) {
+    const uint4 v = *reinterpret_cast<const uint4*>(cnt + i);
+    sum += (v.x + v.y) + (v.z + v.w);
+  }
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) sum += __shfl_xor(sum, h);
+  if (lane == 0) before[w] = sum;
+  unsigned c[4], own = 0;
+  const unsigned at = first + 4 * threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    c[q] = at + q < n ? cnt[at + q] : 0u;
+    own += c[q];
+  }
+  unsigned run = own;  // inclusive scan over the wavefront
+#pragma unroll
+  for (int h = 1; h < 64; h <<= 1) {
+    const unsigned up = __shfl_up(run, h);
+    if (lane >= (unsigned)h) run += up;
+  }
+  if (lane == 63) wave_sum[w] = run;
+  __syncthreads();
+  unsigned start = run - own;
+  for (unsigned q = 0; q < kScanThreads / 64; ++q) start += before[q] + (q < w ? wave_sum[q] : 0u);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (at + q < n) out[at + q] = start;
+    start += c[q];
+  }
+}
+
 }  // namespace
 
 hipError_t launch_particle_ids(Domain* d) {
@@ -164,6 +209,11 @@ hipError_t sort_order(Domain* d, CellOrder& o, long n, unsigned rows, unsigned s
 // row[r] = cnt[0] + ... + cnt[r-1] for r in [0, rows]: the start of every row of a counting
 // order (cnt has rows + 1 entries, the last one the bucket of halves that deposit nothing).
 hipError_t scan_row_counts(Domain* d, const unsigned* cnt, unsigned* row, unsigned rows) {
+  if (rows < kScanMost) {
+    hipLaunchKernelGGL(k_scan_counts, dim3((rows + kScanChunk) / kScanChunk), dim3(kScanThreads), 0, d->stream, cnt,
+                       rows + 1, row);
+    return hipGetLastError();
+  }
   size_t bytes = 0;
   hipError_t e = rocprim::exclusive_scan(nullptr, bytes, cnt, row, 0u, (size_t)rows + 1, rocprim::plus<unsigned>(),
                                          d->stream);
