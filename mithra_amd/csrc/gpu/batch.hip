@@ -95,7 +95,7 @@ struct mithra_batch {
   int2* tiles = nullptr;
   size_t tiles_cap = 0;
   BatchTiles t_int[2], t_eval, t_faces, t_rims, t_part, t_rows, t_inst, t_dep, t_pnodes;
-  BatchTiles t_tfsf[3];             // TF/SF lines of the seeded instances, per axis
+  BatchTiles t_tfsf;                // TF/SF nodes of the seeded instances
   size_t dep_lds = 0;
   bool prepared = false;
   std::vector<long> step;           // host mirror of each instance's step
@@ -164,13 +164,9 @@ int build_tables(mithra_batch* b) {
   table(b->t_pnodes, [&](int i, const BatchView& v) {
     if (v.pNz > 0 && v.pNl > 0 && v.N0 > 4 && v.N1 > 4) add(i, (long)v.pNz * v.pblocks);
   });
-  for (int axis = 0; axis < 3; ++axis)
-    table(b->t_tfsf[axis], [&](int i, const BatchView& v) {
-      if (!v.seeded) return;
-      const long lines = axis == 0 ? (long)(v.N1 - 4) * (v.N2 - 4)
-                                   : axis == 1 ? (long)(v.N0 - 4) * (v.N2 - 4) : (long)(v.N0 - 4) * (v.N1 - 4);
-      add(i, (lines + 63) / 64);  // 256 work items (four injections of 64 lines) per entry
-    });
+  table(b->t_tfsf, [&](int i, const BatchView& v) {
+    if (v.seeded) add(i, (tfsf_nodes(v.N0, v.N1, v.N2) + 255) / 256);
+  });
   if (all.size() > b->tiles_cap) {
     (void)hipFree(b->tiles);
     b->tiles = nullptr;
@@ -184,7 +180,7 @@ int build_tables(mithra_batch* b) {
   }
   BatchTiles* ts[] = {&b->t_int[0], &b->t_int[1], &b->t_eval, &b->t_faces, &b->t_rims,
                       &b->t_part,   &b->t_rows,   &b->t_inst, &b->t_dep,      &b->t_pnodes,
-                      &b->t_tfsf[0], &b->t_tfsf[1], &b->t_tfsf[2]};
+                      &b->t_tfsf};
   for (BatchTiles* T : ts) T->t = b->tiles + (size_t)T->t;
   return MITHRA_OK;
 }

@@ -125,6 +125,9 @@ struct BeamDev {
   double sigma_invg[2];
 };
 
+// The square, correctly rounded; pow(x, 2) is a general power of some hundred instructions on the device.
+__device__ inline double sq(double x) { return x * x; }
+
 // Signal::self (src/classes.cpp:534-575) of a seed or a beam: the carrier at phase `phase` times
 // the pulse envelope of the signal type.
 template <typename S>
@@ -137,18 +140,18 @@ __device__ double signal(const S& s, double t, double phase) {
       return -cos(2 * kPI * f0 * (t - t0) + cep + phase) * 2.7724 * (t - t0) / (ss * ss) *
              exp(-1.3863 * (t - t0) * (t - t0) / (ss * ss));
     case MITHRA_SIGNAL_GAUSSIAN:
-      return c * exp(-1.3863 * pow((t - t0) / ss, 2));
+      return c * exp(-1.3863 * sq((t - t0) / ss));
     case MITHRA_SIGNAL_SECANT:
       return c / cosh((t - t0) / ss);
     case MITHRA_SIGNAL_FLATTOP:
-      if (t - t0 <= -ss / 2.0) return c * exp(-pow((t - t0 + ss / 2.0) * f0 / s.nR, 2));
+      if (t - t0 <= -ss / 2.0) return c * exp(-sq((t - t0 + ss / 2.0) * f0 / s.nR));
       if (t - t0 <= ss / 2.0) return c;
-      return c * exp(-pow((t - t0 - ss / 2.0) * f0 / s.nR, 2));
+      return c * exp(-sq((t - t0 - ss / 2.0) * f0 / s.nR));
     case MITHRA_SIGNAL_INVGAUSSIAN: {
-      double env = pow((1.0 + pow((t - t0) / s.sigma_invg[0], 2)) * (1.0 + pow((t - t0) / s.sigma_invg[1], 2)), 0.25);
-      if (t - t0 <= -ss / 2.0) return c * env * exp(-pow((t - t0 + ss / 2.0) * f0 / s.nR, 2));
+      double env = pow((1.0 + sq((t - t0) / s.sigma_invg[0])) * (1.0 + sq((t - t0) / s.sigma_invg[1])), 0.25);
+      if (t - t0 <= -ss / 2.0) return c * env * exp(-sq((t - t0 + ss / 2.0) * f0 / s.nR));
       if (t - t0 <= ss / 2.0) return c * env;
-      return c * env * exp(-pow((t - t0 - ss / 2.0) * f0 / s.nR, 2));
+      return c * env * exp(-sq((t - t0 - ss / 2.0) * f0 / s.nR));
     }
   }
   return 0.0;
@@ -424,7 +427,8 @@ struct BatchTiles {
 };
 hipError_t launch_batch_interior(BatchView* V, BatchTiles T, int variant, int precision, int nsfd, hipStream_t s);
 hipError_t launch_batch_mur(BatchView* V, BatchTiles faces, BatchTiles rims, int precision, hipStream_t s);
-hipError_t launch_batch_tfsf(BatchView* V, const BatchTiles* axes, int precision, hipStream_t s);  // axes[3]
+hipError_t launch_batch_tfsf(BatchView* V, BatchTiles T, int precision, hipStream_t s);
+long tfsf_nodes(int N0, int N1, int N2);  // work items of the TF/SF injection, 256 to a batch entry
 hipError_t launch_batch_eval(BatchView* V, BatchTiles T, int variant, int precision, hipStream_t s);
 hipError_t launch_batch_push(BatchView* V, BatchTiles T, hipStream_t s);
 hipError_t launch_batch_bunching(BatchView* V, BatchTiles particles, BatchTiles inst, hipStream_t s);

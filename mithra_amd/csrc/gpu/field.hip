@@ -431,9 +431,9 @@ __device__ void seed_fields(const mithra_seed& s, double r0, double r1, double r
       const double zRs = kPI * s.radius[1] * s.radius[1] / l;
       const double wrs = sqrt(1.0 + z * z / (zRs * zRs));
       const double p = 0.5 * (atan(z / zRp) + atan(z / zRs) - kPI) -
-                       kPI * z / l * (pow(x / (zRp * wrp), 2) + pow(y / (zRs * wrs), 2));
+                       kPI * z / l * (sq(x / (zRp * wrp)) + sq(y / (zRs * wrs)));
       ts = signal(s, tl, p);
-      const double t = exp(-pow(x / (s.radius[0] * wrp), 2) - pow(y / (s.radius[1] * wrs), 2)) / sqrt(wrs * wrp) *
+      const double t = exp(-sq(x / (s.radius[0] * wrp)) - sq(y / (s.radius[1] * wrs))) / sqrt(wrs * wrp) *
                        s.amplitude;
       amp = t * ts;
     }
@@ -448,74 +448,105 @@ __device__ void seed_fields(const mithra_seed& s, double r0, double r1, double r
   a[2] *= s.gamma;
 }
 
+// TF/SF injection (src/fdtd.cpp:307-373).  Axis 0 injects into planes i = 1, 2, N0-2, N0-3 at the j, k
+// two nodes or more from the mesh's faces, axes 1 and 2 likewise: plane 1 takes minus the seed at
+// plane 2, plane 2 plus the seed at plane 1, and so at the other end.  The reference runs the axes, and
+// the four planes of an axis, one after the other, and a node where planes cross takes one injection
+// of each.  Here a thread owns a node and applies all of its injections in the reference's order, so
+// one launch serves the three axes: tfsf_count nodes, those with one injection first, in the plane's
+// order, then the rest, so that hardly any wavefront evaluates more than one seed.  On an axis
+// of fewer than six nodes planes coincide, and every node of the mesh is asked.
+//
+// Bound by the latency of one seed evaluation.  Three launches, with the squares by pow(x, 2), took 12 us
+// each on 32 x 32 x 128 nodes and 34 us on 128 x 128 x 1024; NOTETFSF.
+__host__ __device__ inline long tfsf_count(int N0, int N1, int N2) {
+  if (N0 < 6 || N1 < 6 || N2 < 6) return (long)N0 * N1 * N2;
+  const long a = N0 - 4, b = N1 - 4, c = N2 - 4;
+  return 2 * (b * c + a * c + a * b) + 2 * ((b - 2) * (c - 2) + (a - 2) * (c - 2) + (a - 2) * (b - 2)) +
+         4 * (c + (b - 2) + (a - 2));
+}
+
+// Node t of the list.
+__device__ inline void tfsf_node(long t, int N0, int N1, int N2, int ijk[3]) {
+  if (N0 < 6 || N1 < 6 || N2 < 6) {
+    ijk[1] = (int)(t % N1);
+    ijk[0] = (int)(t / N1 % N0);
+    ijk[2] = (int)(t / N1 / N0);
+    return;
+  }
+  const int a = N0 - 4, b = N1 - 4, c = N2 - 4;
+  // a plane of u x v nodes from node lo on, at both ends (first, last) of an axis
+  auto planes = [&](int u, int v, int lo, int first, int last, int& pu, int& pv, int& pw) {
+    const long n = (long)u * v;
+    if (t < 2 * n) {
+      const bool hi = t >= n;
+      const int q = (int)(t - (hi ? n : 0));
+      pu = lo + q % u;
+      pv = lo + q / u;
+      pw = hi ? last : first;
+      return true;
+    }
+    t -= 2 * n;
+    return false;
+  };
+  int &i = ijk[0], &j = ijk[1], &k = ijk[2];
+  if (planes(b, c, 2, 1, N0 - 2, j, k, i) || planes(a, c, 2, 1, N1 - 2, i, k, j) ||
+      planes(b, a, 2, 1, N2 - 2, j, i, k) || planes(b - 2, c - 2, 3, 2, N0 - 3, j, k, i) ||
+      planes(a - 2, c - 2, 3, 2, N1 - 3, i, k, j) || planes(b - 2, a - 2, 3, 2, N2 - 3, j, i, k))
+    return;
+  // the inner planes' crossings: along z with their ends, along y, along x
+  auto lines = [&](int n, int lo, int& along, int& p, int& q, int lastp, int lastq) {
+    if (t < 4L * n) {
+      const int which = (int)(t / n);
+      along = lo + (int)(t % n);
+      p = which & 1 ? lastp : 2;
+      q = which & 2 ? lastq : 2;
+      return true;
+    }
+    t -= 4L * n;
+    return false;
+  };
+  if (lines(c, 2, k, i, j, N0 - 3, N1 - 3) || lines(b - 2, 3, j, i, k, N0 - 3, N2 - 3)) return;
+  lines(a - 2, 3, i, j, k, N1 - 3, N2 - 3);
+}
+
 template <typename R>
-__device__ inline void tfsf_apply(FieldSet A, long m, double px, double py, double pz, double time,
-                                  const mithra_seed& s, double coef, bool minus) {
-  double a[3];
-  seed_fields(s, px, py, pz, time, a);
-  for (int c = 0; c < 3; ++c) {
-    R* p = (R*)A.c[c];
-    double v = (double)p[m];
-    p[m] = (R)(minus ? v - coef * a[c] : v + coef * a[c]);
+__device__ inline void tfsf_body(FieldSet A, int N0, int N1, int N2, const mithra_grid& g, const mithra_seed& s,
+                                 double time, double a1, double a2, double a3, long t) {
+  if (t >= tfsf_count(N0, N1, N2)) return;
+  int ijk[3];
+  tfsf_node(t, N0, N1, N2, ijk);
+  const int i = ijk[0], j = ijk[1], k = ijk[2];
+  const bool in0 = i >= 2 && i < N0 - 2, in1 = j >= 2 && j < N1 - 2, in2 = k >= 2 && k < N2 - 2;
+  const long m = (long)N1 * N0 * k + (long)N1 * i + j;
+  R* const p[3] = {(R*)A.c[0], (R*)A.c[1], (R*)A.c[2]};
+#pragma unroll 1
+  for (int axis = 0; axis < 3; ++axis) {
+    const int n = axis == 0 ? N0 : axis == 1 ? N1 : N2, at = axis == 0 ? i : axis == 1 ? j : k;
+    if (!(axis == 0 ? in1 && in2 : axis == 1 ? in0 && in2 : in0 && in1)) continue;
+    // the axis's four injections: into plane 1 from 2, 2 from 1, n-2 from n-3, n-3 from n-2
+    unsigned hits = (at == 1 ? 1u : 0u) | (at == 2 ? 2u : 0u) | (at == n - 2 ? 4u : 0u) | (at == n - 3 ? 8u : 0u);
+    for (; hits; hits &= hits - 1) {
+      const int q = __builtin_ctz(hits);
+      const int from = q == 0 ? 2 : q == 1 ? 1 : q == 2 ? n - 3 : n - 2;
+      const double x = g.xmin + (axis == 0 ? from : i) * g.dx, y = g.ymin + (axis == 1 ? from : j) * g.dy,
+                   z = g.zmin + (axis == 2 ? from : k) * g.dz;
+      const double coef = axis == 0 ? a1 : axis == 1 ? a2 : a3;
+      double a[3];
+      seed_fields(s, x, y, z, time, a);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double v = (double)p[c][m];
+        p[c][m] = (R)(q & 1 ? v + coef * a[c] : v - coef * a[c]);
+      }
+    }
   }
 }
 
-// TF/SF injection (src/fdtd.cpp:307-373).  axis 0: planes i = 1, 2, N0-2, N0-3 over (j, k);
-// axis 1: planes j = 1, 2, N1-2, N1-3 over (i, k); axis 2: planes k = 1, 2, np-2, np-3 over (i, j).
-// The three axes run as three launches in the reference's loop order.  Launches carry four work
-// items per line.  Where the axis has 6 nodes or more its four planes are distinct, and work item
-// t = 64 (4 g + q) + l applies injection q of line 64 g + l alone (q is uniform over a
-// wavefront, so each wavefront follows one branch).  On a shorter axis two planes coincide, and
-// work item t < lines applies all four injections of line t in the reference's order, so the node
-// touched twice receives its contributions in the same sequence.
 template <typename R>
-__device__ inline void tfsf_body(FieldSet A, int axis, int N0, int N1, int N2, const mithra_grid& g,
-                                 const mithra_seed& s, double time, double coef, long t) {
-  const long N1N0 = (long)N1 * N0;
-  const bool split = (axis == 0 ? N0 : axis == 1 ? N1 : N2) >= 6;
-  int q = 0;
-  if (split) {
-    q = (int)((t >> 6) & 3);
-    t = ((t >> 8) << 6) + (t & 63);
-  }
-  const bool q0 = !split || q == 0, q1 = !split || q == 1, q2 = !split || q == 2, q3 = !split || q == 3;
-  if (axis == 0) {
-    const long nj = N1 - 4, nk = N2 - 4;
-    if (t >= nj * nk) return;
-    const long j = 2 + t % nj, k = 2 + t / nj;
-    const double y = g.ymin + j * g.dy, z = g.zmin + k * g.dz;
-    const long base = N1N0 * k + j;
-    if (q0) tfsf_apply<R>(A, base + N1 * 1, g.xmin + 2 * g.dx, y, z, time, s, coef, true);
-    if (q1) tfsf_apply<R>(A, base + N1 * 2, g.xmin + 1 * g.dx, y, z, time, s, coef, false);
-    if (q2) tfsf_apply<R>(A, base + (long)N1 * (N0 - 2), g.xmin + (N0 - 3) * g.dx, y, z, time, s, coef, true);
-    if (q3) tfsf_apply<R>(A, base + (long)N1 * (N0 - 3), g.xmin + (N0 - 2) * g.dx, y, z, time, s, coef, false);
-  } else if (axis == 1) {
-    const long ni = N0 - 4, nk = N2 - 4;
-    if (t >= ni * nk) return;
-    const long i = 2 + t % ni, k = 2 + t / ni;
-    const double x = g.xmin + i * g.dx, z = g.zmin + k * g.dz;
-    const long base = N1N0 * k + (long)N1 * i;
-    if (q0) tfsf_apply<R>(A, base + 1, x, g.ymin + 2 * g.dy, z, time, s, coef, true);
-    if (q1) tfsf_apply<R>(A, base + 2, x, g.ymin + 1 * g.dy, z, time, s, coef, false);
-    if (q2) tfsf_apply<R>(A, base + N1 - 2, x, g.ymin + (N1 - 3) * g.dy, z, time, s, coef, true);
-    if (q3) tfsf_apply<R>(A, base + N1 - 3, x, g.ymin + (N1 - 2) * g.dy, z, time, s, coef, false);
-  } else {
-    const long ni = N0 - 4, nj = N1 - 4;
-    if (t >= ni * nj) return;
-    const long j = 2 + t % nj, i = 2 + t / nj;
-    const double x = g.xmin + i * g.dx, y = g.ymin + j * g.dy;
-    const long base = (long)N1 * i + j;
-    if (q0) tfsf_apply<R>(A, base + N1N0 * 1, x, y, g.zmin + 2 * g.dz, time, s, coef, true);
-    if (q1) tfsf_apply<R>(A, base + N1N0 * 2, x, y, g.zmin + 1 * g.dz, time, s, coef, false);
-    if (q2) tfsf_apply<R>(A, base + N1N0 * (N2 - 2), x, y, g.zmin + (N2 - 3) * g.dz, time, s, coef, true);
-    if (q3) tfsf_apply<R>(A, base + N1N0 * (N2 - 3), x, y, g.zmin + (N2 - 2) * g.dz, time, s, coef, false);
-  }
-}
-
-template <typename R>
-__global__ void k_tfsf(FieldSet A, int axis, int N0, int N1, int N2, mithra_grid g, mithra_seed s, double time,
-                       double coef) {
-  tfsf_body<R>(A, axis, N0, N1, N2, g, s, time, coef, (long)blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(256) void k_tfsf(FieldSet A, int N0, int N1, int N2, mithra_grid g, mithra_seed s,
+                                              double time, double a1, double a2, double a3) {
+  tfsf_body<R>(A, N0, N1, N2, g, s, time, a1, a2, a3, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // ---- the super-gaussian seed's TF/SF injection ------------------------------------------------
@@ -595,9 +626,9 @@ __device__ bool sg_term(const mithra_seed& s, double r0, double r1, double r2, d
   const double zRs = kPI * s.radius[1] * s.radius[1] / l;
   const double wrs = sqrt(1.0 + z * z / (zRs * zRs));
   const double p = 0.5 * (atan(z / zRp) + atan(z / zRs) - kPI) -
-                   kPI * z / l * (pow(x / (zRp * wrp), 2) + pow(y / (zRs * wrs), 2));
+                   kPI * z / l * (sq(x / (zRp * wrp)) + sq(y / (zRs * wrs)));
   ts = signal(s, tl, p);
-  const double t = exp(-pow(x / (s.radius[0] * wrp), 2) - pow(y / (s.radius[1] * wrs), 2)) / sqrt(wrs * wrp) *
+  const double t = exp(-sq(x / (s.radius[0] * wrp)) - sq(y / (s.radius[1] * wrs))) / sqrt(wrs * wrp) *
                    s.amplitude;
   *term = t * ts;
   return false;
@@ -1526,18 +1557,16 @@ __global__ __launch_bounds__(kFlatThreads) void kb_eval_flat(const BatchView* __
   }
 }
 
-// TF/SF injection of the seeded instances, one axis per launch (the reference's order);
-// entry .y = block of 256 lines of the axis.
+// TF/SF injection of the seeded instances: entry .y = block of 256 nodes of the list.
 template <typename R>
-__global__ __launch_bounds__(256) void kb_tfsf(const BatchView* __restrict__ V, BatchTiles T, int axis) {
+__global__ __launch_bounds__(256) void kb_tfsf(const BatchView* __restrict__ V, BatchTiles T) {
   for (int r = 0;; ++r) {
     const int t = batch_entry(r);
     if (t >= T.n) break;
     const int2 e = T.t[t];
     const BatchView& v = V[e.x];
     if (!v.active || !v.seeded) continue;
-    const double coef = axis == 0 ? v.a[1] : axis == 1 ? v.a[2] : v.a[3];
-    tfsf_body<R>(v.lvl[v.i_np1], axis, v.N0, v.N1, v.N2, v.grid, v.seed, v.time, coef,
+    tfsf_body<R>(v.lvl[v.i_np1], v.N0, v.N1, v.N2, v.grid, v.seed, v.time, v.a[1], v.a[2], v.a[3],
                  (long)e.y * 256 + threadIdx.x);
   }
 }
@@ -1829,16 +1858,10 @@ hipError_t tfsf_impl(Domain* d, double time, const mithra_seed* seed) {
   // update starts from (src/classes.cpp:758-851, src/fdtd.cpp:239), so nothing is injected
   if (seed->seed_type >= MITHRA_SEED_STANDING_PLANEWAVE) return hipSuccess;
   if (seed->seed_type == MITHRA_SEED_SUPERGAUSSIANBEAM) return tfsf_sg_impl<R>(d, time, seed);
-  const long n[3] = {(long)(g.N1 - 4) * (g.N2 - 4), (long)(g.N0 - 4) * (g.N2 - 4), (long)(g.N0 - 4) * (g.N1 - 4)};
-  const double coef[3] = {d->co.a[1], d->co.a[2], d->co.a[3]};
-  for (int axis = 0; axis < 3; ++axis) {
-    if (n[axis] <= 0) continue;
-    hipLaunchKernelGGL((k_tfsf<R>), dim3((unsigned)((n[axis] + 63) / 64)), dim3(256), 0, d->stream,
-                       d->lvl[d->i_np1], axis, g.N0, g.N1, g.N2, g, *seed, time, coef[axis]);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  hipLaunchKernelGGL((k_tfsf<R>), dim3((unsigned)((tfsf_count(g.N0, g.N1, g.N2) + 255) / 256)), dim3(256), 0,
+                     d->stream, d->lvl[d->i_np1], g.N0, g.N1, g.N2, g, *seed, time, d->co.a[1], d->co.a[2],
+                     d->co.a[3]);
+  return hipGetLastError();
 }
 
 template <typename R>
@@ -1989,19 +2012,16 @@ hipError_t launch_batch_eval(BatchView* V, BatchTiles T, int variant, int precis
                                             : batch_field_variant<float>(V, T, 1, variant, 0, s);
 }
 
-hipError_t launch_batch_tfsf(BatchView* V, const BatchTiles* axes, int precision, hipStream_t s) {
-  for (int axis = 0; axis < 3; ++axis) {
-    const BatchTiles& T = axes[axis];
-    if (!T.n) continue;
-    if (precision == MITHRA_PRECISION_FP64)
-      hipLaunchKernelGGL((kb_tfsf<double>), dim3(batch_grid(T.n, 8)), dim3(256), 0, s, V, T, axis);
-    else
-      hipLaunchKernelGGL((kb_tfsf<float>), dim3(batch_grid(T.n, 8)), dim3(256), 0, s, V, T, axis);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+hipError_t launch_batch_tfsf(BatchView* V, BatchTiles T, int precision, hipStream_t s) {
+  if (!T.n) return hipSuccess;
+  if (precision == MITHRA_PRECISION_FP64)
+    hipLaunchKernelGGL((kb_tfsf<double>), dim3(batch_grid(T.n, 8)), dim3(256), 0, s, V, T);
+  else
+    hipLaunchKernelGGL((kb_tfsf<float>), dim3(batch_grid(T.n, 8)), dim3(256), 0, s, V, T);
+  return hipGetLastError();
 }
+
+long tfsf_nodes(int N0, int N1, int N2) { return tfsf_count(N0, N1, N2); }
 
 template <typename R>
 hipError_t batch_mur_impl(BatchView* V, BatchTiles faces, BatchTiles rims, hipStream_t s) {

@@ -50,7 +50,7 @@ __device__ void beam_fields(const BeamDev& s, const double rl[3], double t0, dou
       if (truncated) {  // the truncation test comes first for the standing wave (src/beam.cc:312-322)
         const double x = rv[0] * s.polarization[0] + rv[1] * s.polarization[1] + rv[2] * s.polarization[2];
         const double y = rv[0] * s.yv[0] + rv[1] * s.yv[1] + rv[2] * s.yv[2];
-        if (pow(x / s.radius[0], 2) + pow(y / s.radius[1], 2) > 1.0) return;
+        if (sq(x / s.radius[0]) + sq(y / s.radius[1]) > 1.0) return;
       }
       const double ts = signal(s, tl, p0), tsm = signal(s, tlm, p0);
       te = ts - tsm;
@@ -62,7 +62,7 @@ __device__ void beam_fields(const BeamDev& s, const double rl[3], double t0, dou
       if (truncated) {
         const double x = rv[0] * s.polarization[0] + rv[1] * s.polarization[1] + rv[2] * s.polarization[2];
         const double y = rv[0] * s.yv[0] + rv[1] * s.yv[1] + rv[2] * s.yv[2];
-        if (pow(x / s.radius[0], 2) + pow(y / s.radius[1], 2) > 1.0) return;
+        if (sq(x / s.radius[0]) + sq(y / s.radius[1]) > 1.0) return;
       }
       te = tb = ts;
     }
@@ -97,8 +97,8 @@ __device__ void beam_fields(const BeamDev& s, const double rl[3], double t0, dou
   double ex[3] = {0.0, 0.0, 0.0}, by[3] = {0.0, 0.0, 0.0}, ez[3] = {0.0, 0.0, 0.0}, bz[3] = {0.0, 0.0, 0.0};
   if (!super) {
     const double x0 = x / wrp, y0 = y / wrs;
-    const double q0 = 0.5 * (atanP + atanS) - kPI * z / s.l * (pow(x0 / s.zR[0], 2) + pow(y0 / s.zR[1], 2));
-    double t = exp(-pow(x0 / s.radius[0], 2) - pow(y0 / s.radius[1], 2)) / sqrt(wrs * wrp);
+    const double q0 = 0.5 * (atanP + atanS) - kPI * z / s.l * (sq(x0 / s.zR[0]) + sq(y0 / s.zR[1]));
+    double t = exp(-sq(x0 / s.radius[0]) - sq(y0 / s.radius[1])) / sqrt(wrs * wrp);
     t *= s.amplitude;
     if (!standing) {  // Solver::gaussianBeam (src/beam.cc:142-197)
       double ts = signal(s, tl, q0 - kPI / 2.0);
@@ -128,8 +128,8 @@ __device__ void beam_fields(const BeamDev& s, const double rl[3], double t0, dou
         const double x0 = (x - i * s.radius[0]) / wrp;
         const double y0 = (y - j * s.radius[1]) / wrs;
         if (fabs(x0) > 4.0 * s.radius[0] || fabs(y0) > 4.0 * s.radius[1]) continue;
-        const double q0 = 0.5 * (atanP + atanS) - kPI * z / s.l * (pow(x0 / s.zR[0], 2) + pow(y / s.zR[1], 2));
-        const double t = af * exp(-pow(x0 / s.radius[0], 2) - pow(y0 / s.radius[1], 2));
+        const double q0 = 0.5 * (atanP + atanS) - kPI * z / s.l * (sq(x0 / s.zR[0]) + sq(y / s.zR[1]));
+        const double t = af * exp(-sq(x0 / s.radius[0]) - sq(y0 / s.radius[1]));
         if (!standing) {
           double ts = signal(s, tl, q0 - kPI / 2.0);
           add3(ex, t * ts, s.polarization);
@@ -195,7 +195,7 @@ __device__ void undulator_field(const PushConst& c, UT und, const BeamDev* beams
       bz = b0 * sinh(ku * ly) * cos(ku * lz);
     } else {
       const double s = (lz < 0.0) ? lz : lz - L;     // distance into the fringe
-      double sz = exp(-pow(ku * s, 2) / 2.0);
+      double sz = exp(-sq(ku * s) / 2.0);
       if (lz < 0.0 && u != 0) {
         const UndDev V = *(const UndDev*)(und + (u - 1));
         const double r0 = V.rb + V.L - U.rb;

@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) void k_cell_start(const unsigned* __restrict__
 
 // Exclusive scan of the row counts (n entries) in one launch: a workgroup scans its kScanChunk entries
 // and adds up all the entries before them itself, so no workgroup waits for another and nothing has to
-// be initialised.  rocPRIM's look-back scan is two launches, 4.5-5 us each on small meshes; the sums'
-// reads grow with the square of n, to 16 KB a thread-row at kScanMost, where the two are even (LARGE).
+// be initialised.  rocPRIM's look-back scan is two launches, 4.5-5 us each on small meshes, against 3.9 us
+// at 4k rows and 5.4 at 27k; the reads before a workgroup grow with n, to 512 KB at kScanMost.
 constexpr int kScanThreads = 1024, kScanChunk = 4 * kScanThreads;
 constexpr unsigned kScanMost = 1u << 17;
 
