@@ -22,6 +22,52 @@ constexpr int kDefaultSortInterval = 16;
 
 inline int hip_status(hipError_t e) { return e == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)e; }
 
+// A chunk of nodes of one level in the caller's layout: xyz[3 t + c] of node m0 + t, or scalar[t].
+template <typename R>
+__global__ __launch_bounds__(256) void k_pack_potentials(FieldSet f, long m0, long n, double* __restrict__ xyz,
+                                                         double* __restrict__ scalar) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (xyz && t < 3 * n) xyz[t] = (double)((const R*)component(f, (int)(t % 3)))[m0 + t / 3];
+  if (scalar && t < n) scalar[t] = (double)((const R*)component(f, 3))[m0 + t];
+}
+
+// A chunk of nodes of E/B (six floats a node on the device) as e[3 t + c], b[3 t + c].
+__global__ __launch_bounds__(256) void k_pack_fields(const float* __restrict__ eb, long m0, long n,
+                                                     float* __restrict__ e, float* __restrict__ b) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= 3 * n) return;
+  const float* src = eb + 6 * (m0 + t / 3) + t % 3;
+  if (e) e[t] = src[0];
+  if (b) b[t] = src[3];
+}
+
+// The records (q, rnp[3], rnm[3], gb[3], e) of the particles whose load number lies in [lo, hi), in
+// load order.  A wavefront lists those among its 64 particles and writes them together, so that a record
+// leaves as 88 neighbouring bytes.
+__global__ __launch_bounds__(256) void k_pack_particles(const double* __restrict__ part, long cap,
+                                                        const unsigned* __restrict__ id, long n, long lo, long hi,
+                                                        double* __restrict__ out) {
+  __shared__ unsigned sp[4][64], sid[4][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long p = (long)blockIdx.x * 256 + threadIdx.x;
+  const unsigned num = p < n ? id[p] : 0u;
+  const bool in = p < n && (long)num >= lo && (long)num < hi;
+  const unsigned long long m = __ballot(in);
+  if (m == 0) return;
+  if (in) {
+    const int at = __popcll(m & ((1ull << lane) - 1));
+    sp[w][at] = (unsigned)p;
+    sid[w][at] = (unsigned)(num - lo);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  for (int t = lane; t < 11 * __popcll(m); t += 64) {
+    const int r = t / 11, c = t % 11;
+    const int a = c == 0 ? (int)PQ : c == 10 ? (int)PE : c - 1;
+    out[11l * sid[w][r] + c] = part[a * cap + sp[w][r]];
+  }
+}
+
 #define MITHRA_TRY(expr)                      \
   do {                                        \
     hipError_t _e = (expr);                   \
@@ -292,6 +338,7 @@ int mithra_dev_destroy(mithra_dev* d) {
   hipFree(d->det_block);
   free_power(d);
   hipFree(d->diag);
+  stage_free(&d->stage);
   hipFree(d->sg_buf);
   hipFree(d->vring);
   hipFree(d->vdft);
@@ -380,39 +427,43 @@ int mithra_dev_get_potentials(mithra_dev* d, int level, double* a, double* phi) 
   if (int rc = settle(d)) return rc;
   const int li = level_of(d, level);
   if (li < 0) return MITHRA_E_ARG;
-  MITHRA_TRY(hipStreamSynchronize(d->stream));
-  const size_t n = (size_t)d->nodes;
-  std::vector<double> dbl(n);
-  std::vector<float> flt;
-  auto get = [&](int c, double* dst, size_t stride) -> hipError_t {
-    hipError_t e;
-    if (d->precision == MITHRA_PRECISION_FP64) {
-      e = hipMemcpy(dbl.data(), d->lvl[li].c[c], n * sizeof(double), hipMemcpyDeviceToHost);
-    } else {
-      flt.resize(n);
-      e = hipMemcpy(flt.data(), d->lvl[li].c[c], n * sizeof(float), hipMemcpyDeviceToHost);
-      for (size_t m = 0; m < n; ++m) dbl[m] = flt[m];
-    }
-    if (e == hipSuccess)
-      for (size_t m = 0; m < n; ++m) dst[stride * m] = dbl[m];
-    return e;
+  const FieldSet f = d->lvl[li];
+  if (d->ncomp != 4) phi = nullptr;
+  if (!a && !phi) return hip_status(hipStreamSynchronize(d->stream));
+  auto put = [&](long m0, long n, char* slot) {
+    double* pa = a ? (double*)slot : nullptr;
+    double* pp = phi ? (double*)slot + (a ? 3 * n : 0) : nullptr;
+    const dim3 grid((unsigned)(((a ? 3 * n : n) + 255) / 256));
+    if (d->precision == MITHRA_PRECISION_FP64)
+      hipLaunchKernelGGL(k_pack_potentials<double>, grid, dim3(256), 0, d->stream, f, m0, n, pa, pp);
+    else
+      hipLaunchKernelGGL(k_pack_potentials<float>, grid, dim3(256), 0, d->stream, f, m0, n, pa, pp);
+    return hipGetLastError();
   };
-  if (a)
-    for (int c = 0; c < 3; ++c) MITHRA_TRY(get(c, a + c, 3));
-  if (phi && d->ncomp == 4) MITHRA_TRY(get(3, phi, 1));
-  return MITHRA_OK;
+  auto take = [&](long m0, long n, const char* slot) {
+    const double* v = (const double*)slot;
+    if (a) std::memcpy(a + 3 * m0, v, sizeof(double) * 3 * n);
+    if (phi) std::memcpy(phi + m0, v + (a ? 3 * n : 0), sizeof(double) * n);
+  };
+  return stage_chunks(&d->stage, d->stream, d->nodes, sizeof(double) * ((a ? 3 : 0) + (phi ? 1 : 0)), put, take);
 }
 
 int mithra_dev_get_fields(mithra_dev* d, float* e, float* b) {
   if (!d) return MITHRA_E_ARG;
-  MITHRA_TRY(hipStreamSynchronize(d->stream));
-  std::vector<float> h(2 * kEBPairs * (size_t)d->nodes);  // per node: Ex Ey Ez Bx By Bz
-  MITHRA_TRY(hipMemcpy(h.data(), d->eb, sizeof(float) * h.size(), hipMemcpyDeviceToHost));
-  for (size_t m = 0; m < (size_t)d->nodes; ++m) {
-    if (e) { e[3 * m] = h[6 * m]; e[3 * m + 1] = h[6 * m + 1]; e[3 * m + 2] = h[6 * m + 2]; }
-    if (b) { b[3 * m] = h[6 * m + 3]; b[3 * m + 1] = h[6 * m + 4]; b[3 * m + 2] = h[6 * m + 5]; }
-  }
-  return MITHRA_OK;
+  if (!e && !b) return hip_status(hipStreamSynchronize(d->stream));
+  auto put = [&](long m0, long n, char* slot) {
+    float* pe = e ? (float*)slot : nullptr;
+    float* pb = b ? (float*)slot + (e ? 3 * n : 0) : nullptr;
+    hipLaunchKernelGGL(k_pack_fields, dim3((unsigned)((3 * n + 255) / 256)), dim3(256), 0, d->stream, d->eb, m0, n,
+                       pe, pb);
+    return hipGetLastError();
+  };
+  auto take = [&](long m0, long n, const char* slot) {
+    const float* v = (const float*)slot;
+    if (e) std::memcpy(e + 3 * m0, v, sizeof(float) * 3 * n);
+    if (b) std::memcpy(b + 3 * m0, v + (e ? 3 * n : 0), sizeof(float) * 3 * n);
+  };
+  return stage_chunks(&d->stage, d->stream, d->nodes, sizeof(float) * 3 * ((e ? 1 : 0) + (b ? 1 : 0)), put, take);
 }
 
 }  // extern "C"
@@ -493,17 +544,13 @@ int mithra_dev_take_bunch(mithra_dev* d, const mithra_bunch* b) {
 
 int mithra_dev_get_particles(mithra_dev* d, double* q, long n) {
   if (!d || n != d->np || (n > 0 && !q)) return MITHRA_E_ARG;
-  MITHRA_TRY(hipStreamSynchronize(d->stream));
-  static const int from[PCOUNT] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 0, 10};
-  if (n == 0) return MITHRA_OK;
-  std::vector<unsigned> id(n);
-  MITHRA_TRY(hipMemcpy(id.data(), d->pid, sizeof(unsigned) * n, hipMemcpyDeviceToHost));
-  std::vector<double> col(n);
-  for (int a = 0; a < PCOUNT; ++a) {
-    MITHRA_TRY(hipMemcpy(col.data(), particle_array(d, a), sizeof(double) * n, hipMemcpyDeviceToHost));
-    for (long p = 0; p < n; ++p) q[11 * (long)id[p] + from[a]] = col[p];  // back to load order
-  }
-  return MITHRA_OK;
+  auto put = [&](long lo, long m, char* slot) {
+    hipLaunchKernelGGL(k_pack_particles, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, d->stream, d->part, d->cap,
+                       d->pid, n, lo, lo + m, (double*)slot);
+    return hipGetLastError();
+  };
+  auto take = [&](long lo, long m, const char* slot) { std::memcpy(q + 11 * lo, slot, sizeof(double) * 11 * m); };
+  return stage_chunks(&d->stage, d->stream, n, sizeof(double) * 11, put, take);
 }
 
 long mithra_dev_particle_count(const mithra_dev* d) { return d ? d->np : -1; }

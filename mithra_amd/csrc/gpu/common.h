@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../../include/mithra_gpu.h"
+#include "stage.h"
 
 namespace mithra {
 
@@ -265,6 +266,7 @@ struct Domain {
   // staging of the diagnostics gathers (diagnostics.hip), grown on demand
   void* diag;
   size_t diag_bytes;
+  HostStage stage;          // pinned slots of transfers to the host
   // power map of one plane (power visualization, diagnostics.hip): ring [Nf][4][N1N0] of the
   // lab-frame fields, DFT phases [Nf] (cos, sin), the map; vk < 0: none
   double* vring;

