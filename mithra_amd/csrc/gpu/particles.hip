@@ -175,6 +175,37 @@ __device__ inline void add_beam(const PushConst& c, const BeamDev& b, double x, 
   et[2] += eT[2];
 }
 
+// sinh and cosh of one argument.  Within one radian (k_u y of a bunch near its axis) their Taylor series
+// to x^19, whose remainder is below 1e-18 and whose terms have one sign, so that Horner's form stays within an
+// ulp; beyond it the library's.
+__device__ inline void sinhcosh(double x, double* sh, double* ch) {
+  if (fabs(x) <= 1.0) {
+    const double t = x * x;
+    double s = 1.0 / 121645100408832000.0, c = 1.0 / 6402373705728000.0;  // 19!, 18!
+    s = fma(s, t, 1.0 / 355687428096000.0);
+    c = fma(c, t, 1.0 / 20922789888000.0);
+    s = fma(s, t, 1.0 / 1307674368000.0);
+    c = fma(c, t, 1.0 / 87178291200.0);
+    s = fma(s, t, 1.0 / 6227020800.0);
+    c = fma(c, t, 1.0 / 479001600.0);
+    s = fma(s, t, 1.0 / 39916800.0);
+    c = fma(c, t, 1.0 / 3628800.0);
+    s = fma(s, t, 1.0 / 362880.0);
+    c = fma(c, t, 1.0 / 40320.0);
+    s = fma(s, t, 1.0 / 5040.0);
+    c = fma(c, t, 1.0 / 720.0);
+    s = fma(s, t, 1.0 / 120.0);
+    c = fma(c, t, 1.0 / 24.0);
+    s = fma(s, t, 1.0 / 6.0);
+    c = fma(c, t, 0.5);
+    *sh = fma(s * t, x, x);
+    *ch = fma(c, t, 1.0);
+  } else {
+    *sh = sinh(x);
+    *ch = cosh(x);
+  }
+}
+
 // Solver::undulatorField (src/solver.cpp:1798-1877) with Solver::staticUndulator (src/beam.cc:14-76):
 // adds every undulator's boosted-frame fields at r in table order; BEAMS: some are optical.
 template <bool BEAMS, typename UT>
@@ -189,10 +220,13 @@ __device__ void undulator_field(const PushConst& c, UT und, const BeamDev* beams
     const double b0 = U.b0, ku = U.ku, ct = U.ct, st = U.st, L = U.L;
     const double lz = c.gamma * (z + c.beta * c.c0 * (tb + c.dt_shift)) - U.rb;
     const double ly = x * ct + y * st;
-    double d1, bz;
+    double d1, bz, sh, ch;
+    sinhcosh(ku * ly, &sh, &ch);
     if (lz >= 0.0 && lz <= L) {
-      d1 = b0 * cosh(ku * ly) * sin(ku * lz) * c.gamma;
-      bz = b0 * sinh(ku * ly) * cos(ku * lz);
+      double sv, cv;
+      sincos(ku * lz, &sv, &cv);
+      d1 = b0 * ch * sv * c.gamma;
+      bz = b0 * sh * cv;
     } else {
       const double s = (lz < 0.0) ? lz : lz - L;     // distance into the fringe
       double sz = exp(-sq(ku * s) / 2.0);
@@ -209,8 +243,8 @@ __device__ void undulator_field(const PushConst& c, UT und, const BeamDev* beams
         else sz *= 0.35875 + 0.48829 * cos(kPI * s / r0) + 0.14128 * cos(2.0 * kPI * s / r0) +
                    0.01168 * cos(3.0 * kPI * s / r0);
       }
-      d1 = b0 * cosh(ku * ly) * sz * ku * s * c.gamma;
-      bz = b0 * sinh(ku * ly) * sz;
+      d1 = b0 * ch * sz * ku * s * c.gamma;
+      bz = b0 * sh * sz;
     }
     bt[0] += d1 * ct;
     bt[1] += d1 * st;
@@ -227,16 +261,24 @@ __device__ void undulator_field(const PushConst& c, UT und, const BeamDev* beams
 // step and advanced n_sub times in registers; the time of each sub-step is accumulated exactly
 // as Solver::solve() accumulates timeBunch_ (src/solver.cpp:1316-1321).
 // Returns the particle's new z.
+//
+// Its 1100 instructions a wavefront, two thirds of them the undulator's sin, cos, sinh and cosh, cost as much as
+// its 136 bytes a particle.  One argument reduction for sin and cos, series for sinh and cosh, the E/B of a y
+// pair in three 16-byte loads and the emission flag written only when it changes, at four wavefronts to a
+// SIMD: 16.8M particles 898 -> 786 us, 4.2M 200 -> 163, 1M 66 -> 57.
 template <bool BEAMS>
 __device__ inline double push_body(double* __restrict__ part, long cap, const float* __restrict__ eb,
                                  const UndDev* __restrict__ und, const BeamDev* __restrict__ beams, int n_opt,
                                  int n_ext, const PushConst& c, unsigned long long* __restrict__ counters, long p) {
   const gptr<double> X = G(part);
-  const gptr<const f2> ebg = G(reinterpret_cast<const f2*>(eb));
+  // the two nodes of a y pair lie side by side, 48 bytes from an 8-byte boundary
+  typedef float f4_8 __attribute__((ext_vector_type(4), aligned(8)));
+  const gptr<const float> ebg = G(eb);
   const gptr<const UndDev> undg = G(und);
   double x = X[PX * cap + p], y = X[PY * cap + p], z = X[PZ * cap + p];
   double gx = X[PGX * cap + p], gy = X[PGY * cap + p], gz = X[PGZ * cap + p];
-  double e = X[PE * cap + p];
+  const double e_before = X[PE * cap + p];
+  double e = e_before;
   if (c.save_rnm) {  // rnm = rnp (src/solver.cpp:1311-1312)
     X[PXM * cap + p] = x;
     X[PYM * cap + p] = y;
@@ -273,23 +315,24 @@ __device__ inline double push_body(double* __restrict__ part, long cap, const fl
         // E/B is held in registers at a time.
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          f2 q0[4], q1[4], q2[4];
+          f4_8 q[2][3];  // at x offsets 0 and 1: E, B of the nodes j and j + 1
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const long o = m + (h ? N1N0 : 0) + ((u & 1) ? N1 : 0) + (u >> 1);
-            q0[u] = ebg[kEBPairs * o];
-            q1[u] = ebg[kEBPairs * o + 1];
-            q2[u] = ebg[kEBPairs * o + 2];
+          for (int u = 0; u < 2; ++u) {
+            const gptr<const f4_8> at = (gptr<const f4_8>)(ebg + 2 * kEBPairs * (m + (h ? N1N0 : 0) + (u ? N1 : 0)));
+            q[u][0] = at[0];
+            q[u][1] = at[1];
+            q[u][2] = at[2];
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
+            const f4_8* v = q[u & 1];
             const double w = ((u & 1) ? dxr : 1.0 - dxr) * ((u >> 1) ? dyr : 1.0 - dyr) * (h ? dzr : 1.0 - dzr);
-            et[0] += w * (double)q0[u].x;
-            et[1] += w * (double)q0[u].y;
-            et[2] += w * (double)q1[u].x;
-            bt[0] += w * (double)q1[u].y;
-            bt[1] += w * (double)q2[u].x;
-            bt[2] += w * (double)q2[u].y;
+            et[0] += w * (double)(u >> 1 ? v[1].z : v[0].x);
+            et[1] += w * (double)(u >> 1 ? v[1].w : v[0].y);
+            et[2] += w * (double)(u >> 1 ? v[2].x : v[0].z);
+            bt[0] += w * (double)(u >> 1 ? v[2].y : v[0].w);
+            bt[1] += w * (double)(u >> 1 ? v[2].z : v[1].x);
+            bt[2] += w * (double)(u >> 1 ? v[2].w : v[1].y);
           }
         }
       } else if (!b1x && !b1y && b1z) {
@@ -338,7 +381,7 @@ __device__ inline double push_body(double* __restrict__ part, long cap, const fl
   X[PGX * cap + p] = gx;
   X[PGY * cap + p] = gy;
   X[PGZ * cap + p] = gz;
-  X[PE * cap + p] = e;
+  if (e != e_before) X[PE * cap + p] = e;  // emitted on this step
   if (nt) atomicAdd(&counters[0], (unsigned long long)nt);
   if (ncross) atomicAdd(&counters[1], (unsigned long long)ncross);
   return z;
