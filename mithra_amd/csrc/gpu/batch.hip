@@ -194,9 +194,8 @@ int enqueue_step(mithra_batch* b) {
   BATCH_TRY(launch_batch_tfsf(V, b->t_tfsf, p, s));
   BATCH_TRY(launch_batch_mur(V, b->t_faces, b->t_rims, p, s));
   BATCH_TRY(launch_batch_eval(V, b->t_eval, b->variant, p, s));
-  BATCH_TRY(launch_batch_push(V, b->t_part, s));
+  BATCH_TRY(launch_batch_push_power(V, b->t_part, b->t_pnodes, s));
   BATCH_TRY(launch_batch_bunching(V, b->t_part, b->t_inst, s));
-  BATCH_TRY(launch_batch_power(V, b->t_pnodes, s));
   hipLaunchKernelGGL(kb_shift, dim3((b->n + 63) / 64), dim3(64), 0, s, V, b->n);
   BATCH_TRY(hipGetLastError());
   BATCH_TRY(launch_batch_sort(V, b->t_part, b->t_rows, b->t_inst, 0, 0, s));

@@ -221,9 +221,14 @@ int run_step(mithra_dev* d, double time, const mithra_seed* seed, const mithra_b
   MITHRA_TRY(mark(3));
   MITHRA_TRY(pipe_out ? launch_stencil_eb(d) : launch_eval_eb_step(d));
   MITHRA_TRY(mark(4));
-  MITHRA_TRY(launch_push(d, p, d->und_dev, n_und, time_bunch, bunch_time_step, n_sub, 1));
-  MITHRA_TRY(mark(5));
-  if (power_row >= 0) MITHRA_TRY(launch_power(d, n_time, (unsigned)power_row));
+  if (power_row >= 0 && !ms) {
+    MITHRA_TRY(launch_push_power(d, p, d->und_dev, n_und, time_bunch, bunch_time_step, n_sub, n_time,
+                                 (unsigned)power_row));
+  } else {  // timed: each phase by itself
+    MITHRA_TRY(launch_push(d, p, d->und_dev, n_und, time_bunch, bunch_time_step, n_sub, 1));
+    MITHRA_TRY(mark(5));
+    if (power_row >= 0) MITHRA_TRY(launch_power(d, n_time, (unsigned)power_row));
+  }
   MITHRA_TRY(mark(6));
   const int t = d->i_nm1;  // field shift; the free level then holds X when pipelined
   d->i_nm1 = d->i_n;
