@@ -97,6 +97,7 @@ struct mithra_batch {
   BatchTiles t_int[2], t_eval, t_faces, t_rims, t_part, t_rows, t_inst, t_dep, t_pnodes;
   BatchTiles t_tfsf;                // TF/SF nodes of the seeded instances
   size_t dep_lds = 0;
+  unsigned most_rows = 0;           // of any instance: rows of the deposit's orders
   bool prepared = false;
   std::vector<long> step;           // host mirror of each instance's step
   hipGraphExec_t exec = nullptr;
@@ -198,7 +199,7 @@ int enqueue_step(mithra_batch* b) {
   BATCH_TRY(launch_batch_bunching(V, b->t_part, b->t_inst, s));
   hipLaunchKernelGGL(kb_shift, dim3((b->n + 63) / 64), dim3(64), 0, s, V, b->n);
   BATCH_TRY(hipGetLastError());
-  BATCH_TRY(launch_batch_sort(V, b->t_part, b->t_rows, b->t_inst, 0, 0, s));
+  BATCH_TRY(launch_batch_sort(V, b->t_part, b->t_rows, b->t_inst, b->most_rows, 0, 0, s));
   BATCH_TRY(launch_batch_deposit(V, b->t_dep, p, b->dep_lds, s));
   BATCH_TRY(launch_batch_reorder(V, b->t_part, s));
   hipLaunchKernelGGL(kb_advance, dim3((b->n + 63) / 64), dim3(64), 0, s, V, b->n);
@@ -261,18 +262,20 @@ void set_tile_geometry(mithra_batch* b, int variant) {
 
 int prepare(mithra_batch* b) {
   b->dep_lds = 0;
+  b->most_rows = 0;
   for (int i = 0; i < b->n; ++i)
     if (!b->ready[i]) return MITHRA_E_STATE;
   set_tile_geometry(b, b->variant);
   for (int i = 0; i < b->n; ++i) {
     const BatchView& v = b->hv[i];
     b->dep_lds = std::max(b->dep_lds, deposit_lds_bytes(v.ncomp, v.dTI, v.N1));
+    b->most_rows = std::max(b->most_rows, v.rows);
   }
   if (int rc = upload_views(b)) return rc;
   if (int rc = build_tables(b)) return rc;
   // The rnm halves of the first deposit: the first push sets rnm to the present rnp, so the
   // present rnp is sorted once, into the slot the first step reads as its rnm order.
-  BATCH_TRY(launch_batch_sort(b->V, b->t_part, b->t_rows, b->t_inst, 0, 1, b->stream));
+  BATCH_TRY(launch_batch_sort(b->V, b->t_part, b->t_rows, b->t_inst, b->most_rows, 0, 1, b->stream));
   if (int rc = capture(b)) return rc;
   b->prepared = true;
   return MITHRA_OK;

@@ -414,6 +414,9 @@ unsigned long long fixed_order_cells(const Domain* d);  // cells of the fixed-or
 bool deposit_tiled(const Domain* d);
 hipError_t launch_bunching(Domain* d, double k, double* partial, int blocks);
 hipError_t launch_power(Domain* d, unsigned n_time, unsigned row);
+// Row counts up to here are scanned in one launch, each workgroup adding up those before its own (512 KB
+// of reads for the last one).
+constexpr unsigned kScanMost = 1u << 17;
 // The push and the power sample of one step, in one launch where both have work
 hipError_t launch_push_power(Domain* d, const mithra_bunch_params* p, const UndDev* und, int n_und, double time_bunch,
                              double bunch_time_step, int n_sub, unsigned n_time, unsigned row);
@@ -437,8 +440,8 @@ long tfsf_nodes(int N0, int N1, int N2);  // work items of the TF/SF injection, 
 hipError_t launch_batch_eval(BatchView* V, BatchTiles T, int variant, int precision, hipStream_t s);
 hipError_t launch_batch_push_power(BatchView* V, BatchTiles particles, BatchTiles nodes, hipStream_t s);
 hipError_t launch_batch_bunching(BatchView* V, BatchTiles particles, BatchTiles inst, hipStream_t s);
-hipError_t launch_batch_sort(BatchView* V, BatchTiles particles, BatchTiles rowblocks, BatchTiles inst, int use_rm,
-                             int slot_sel, hipStream_t s);
+hipError_t launch_batch_sort(BatchView* V, BatchTiles particles, BatchTiles rowblocks, BatchTiles inst,
+                             unsigned most_rows, int use_rm, int slot_sel, hipStream_t s);
 hipError_t launch_batch_deposit(BatchView* V, BatchTiles T, int precision, size_t lds, hipStream_t s);
 hipError_t launch_batch_reorder(BatchView* V, BatchTiles particles, hipStream_t s);
 int batch_grid(int ntiles, int per_cu);  // persistent grid size for a table of ntiles entries

@@ -81,7 +81,6 @@ __global__ __launch_bounds__(256) void k_cell_start(const unsigned* __restrict__
 // be initialised.  rocPRIM's look-back scan is two launches, 4.5-5 us each on small meshes, against 3.9 us
 // at 4k rows and 5.4 at 27k; the reads before a workgroup grow with n, to 512 KB at kScanMost.
 constexpr int kScanThreads = 1024, kScanChunk = 4 * kScanThreads;
-constexpr unsigned kScanMost = 1u << 17;
 
 __global__ __launch_bounds__(kScanThreads) void k_scan_counts(const unsigned* __restrict__ cnt, unsigned n,
                                                               unsigned* __restrict__ out) {
