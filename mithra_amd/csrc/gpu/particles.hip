@@ -873,7 +873,11 @@ __global__ __launch_bounds__(256) void k_deposit_fixed(FieldSet J, DepositConst 
 // its order, us, marched -> in one pass: production (256 x 256 x 2048 nodes, 16.8M particles, FP64
 // pipelined) 2077 -> 1870, 128 x 128 x 1024 with rho and 4.2M particles 651 -> 540, 211 x 211 x 1531
 // FP32-bulk 703 -> 625, 128 x 128 x 1024 with 1M particles FP32-bulk 164 -> 131, 45 x 45 x 203 with rho
-// 44 -> 32.  Chunks of three, four and six planes in the same LDS are slower everywhere (more rows
+// 44 -> 32.  A block that lists nothing leaves before it clears a tile, the next pair of entries is looked up
+// while the tile is cleared or the pair before it weighed, and the pipelined form leaves X alone where J is
+// +0: the deposit alone 1808 -> 1613 at the production size, 462 -> 416 with rho, 569 -> 546 at 211 x 211 x 1531.
+// Mapping neighbouring tiles to one XCD is slower (1808 -> 2102): the bunch's planes then load the XCDs unevenly.
+// Chunks of three, four and six planes in the same LDS are slower everywhere (more rows
 // weighed twice); so are tiles of 26, 52 and 79 KiB, but for space charge.
 constexpr int kDepositThreads = 512;  // at most
 constexpr int kDepositChunk = 2;      // node planes per workgroup
@@ -920,6 +924,34 @@ __device__ inline void deposit_rows_body(const double* __restrict__ part, long c
       upto[l] = sum;
     }
   }
+  __syncthreads();
+  const unsigned total = upto[lists - 1];
+  if (total == 0) {  // nothing listed: no tile is needed
+    if (SRC ? skip_empty != 0 : add) return;  // see below; x + (+0) read and written back is x
+    if (!SRC) {
+      for (int k = kb; k < ke; ++k) {
+        const long base = N1N0 * k + (long)N1 * i0;
+        for (int o = threadIdx.x; o < own; o += blockDim.x)
+#pragma unroll
+          for (int comp = 0; comp < ncomp; ++comp) G((R*)component(J, comp))[base + o] = (R)0.0;
+      }
+      return;
+    }
+  }
+  // the entry t of the block: its list, and its particle
+  auto locate = [&](unsigned t, int& l) {
+    l = 0;
+    while (t >= upto[l]) ++l;
+    return (l & 1 ? G(m_idx) : G(p_idx))[first[l] + t];
+  };
+  // a thread's next pair of entries is looked up while the tile is cleared, or the pair before it weighed
+  int la = 0, lb = 0;
+  unsigned pa = 0, pb = 0;
+  auto next_pair = [&](unsigned t) {
+    if (t < total) pa = locate(t, la);
+    if (t + blockDim.x < total) pb = locate(t + blockDim.x, lb);
+  };
+  next_pair(threadIdx.x);
   for (int k = kb; k < ke; ++k) {
     double* p = tile + (k - kb) * psz;
     const long base = N1N0 * k + (long)N1 * i0;
@@ -930,22 +962,16 @@ __device__ inline void deposit_rows_body(const double* __restrict__ part, long c
     }
   }
   __syncthreads();
-  const unsigned total = upto[lists - 1];
-  auto locate = [&](unsigned t, HalfItem& it) {
-    int l = 0;
-    while (t >= upto[l]) ++l;
-    it.half = l & 1;
-    it.kk = kb - 1 + (l >> 1);
-    return (long)(it.half ? G(m_idx) : G(p_idx))[first[l] + t];
-  };
   for (unsigned t = threadIdx.x; t < total; t += 2 * blockDim.x) {
     HalfItem a, b;
-    const unsigned tb = t + blockDim.x;
-    const long pa = locate(t, a);
-    b.ok = tb < total;
-    const long pb = b.ok ? locate(tb, b) : pa;
+    b.ok = t + blockDim.x < total;
+    a.half = la & 1;
+    a.kk = kb - 1 + (la >> 1);
+    b.half = lb & 1;
+    b.kk = kb - 1 + (lb >> 1);
     load_item(a, G(part), cap, pa);
-    load_item(b, G(part), cap, pb);
+    load_item(b, G(part), cap, b.ok ? pb : pa);
+    next_pair(t + 2 * blockDim.x);
     deposit_item<SC>(a, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
     if (b.ok) deposit_item<SC>(b, c, tile, psz, TI, kb, ke, i0, ti, lo, hi);
   }
@@ -971,11 +997,12 @@ __device__ inline void deposit_rows_body(const double* __restrict__ part, long c
         const gptr<R> out = G((R*)component(J, comp));
         if (SRC) {
           // the pipelined step: X + a4 J (and X + a5 rho for phi) at interior nodes, J rounded as
-          // the buffer would hold it
-          if (inner) {
+          // the buffer would hold it; X stays as it is where J is +0, as in an untouched plane
+          const double jv = p[comp * tsz + o];
+          if (inner && !(skip_empty && jv == 0.0)) {
             const double xo = (double)ld_stream((gptr<const R>)out, base + o);  // read once, written once
             const double coef = comp < 3 ? src_coef : src_rho;
-            st_stream(out, base + o, (R)(xo + coef * (double)(R)p[comp * tsz + o]));
+            st_stream(out, base + o, (R)(xo + coef * (double)(R)jv));
           }
         } else {
           out[base + o] = (R)p[comp * tsz + o];
