@@ -302,6 +302,7 @@ int write_back(mithra_batch* b) {
     d->rm_order_valid = 0;
     d->zero_pending = 0;
     d->zrange_valid = 0;
+    d->pslot = d->pNf;  // the next sample's sums start afresh
   }
   return MITHRA_OK;
 }

@@ -637,6 +637,7 @@ int mithra_dev_power_setup(mithra_dev* d, const mithra_power_params* p, unsigned
     }
   }
   d->pNz = nz;
+  d->pslot = -1;
   d->pk_lo = 1;
   d->pk_hi = 0;
   for (int c : hk) {

@@ -254,6 +254,7 @@ struct Domain {
   double* partial;          // device: per-block partial sums
   unsigned* pdone;          // device: per plane, workgroups that have finished (zero between launches)
   double* history;          // device: [rows][N][Nl]
+  long pslot;               // ring slot of the last sample (-1: none yet)
   int pblocks;
   int* plane_of;            // host: for each of N planes, its index among inside planes or -1
   // laser beams of the push (mithra_dev_set_beams): n_opt optical-undulator beams, then n_ext

@@ -455,6 +455,7 @@ struct PowerWork {
   PowerBufs bufs;
   double* row;
   unsigned slot;
+  bool fresh;
   int per_plane;     // workgroups per plane
   unsigned blocks;
 };
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(256, 4) void k_push_power(double* __restrict__ part
                                                     PushConst c, unsigned long long* __restrict__ counters,
                                                     int2* __restrict__ zpart, PowerWork w) {
   if (blockIdx.x < w.blocks)
-    power_body(eb, w.bufs, w.row, c.N0, c.N1, w.slot, (int)blockIdx.x % w.per_plane, w.per_plane,
+    power_body(eb, w.bufs, w.row, c.N0, c.N1, w.slot, w.fresh, (int)blockIdx.x % w.per_plane, w.per_plane,
                blockIdx.x / w.per_plane);
   else
     push_block<false>(part, cap, n, eb, und, nullptr, 0, 0, c, counters, zpart, blockIdx.x - w.blocks);
@@ -1060,7 +1061,7 @@ __global__ __launch_bounds__(256, 4) void kb_push_power(BatchView* __restrict__ 
       if (!v.active || v.step >= (long)v.prows) continue;  // uniform over the workgroup
       const PowerBufs B = power_bufs(v);
       power_body(v.eb, B, v.history + (size_t)v.step * v.pN * v.pNl, v.N0, v.N1, (unsigned)(v.step % v.pNf),
-                 e.y % v.pblocks, v.pblocks, e.y / v.pblocks);
+                 v.step % v.pNf == 0, e.y % v.pblocks, v.pblocks, e.y / v.pblocks);
       __syncthreads();  // the LDS of the reduction is reused by the next entry
     }
     return;
@@ -1534,7 +1535,9 @@ hipError_t launch_push_power(Domain* d, const mithra_bunch_params* p, const UndD
     return e == hipSuccess ? launch_power(d, n_time, row) : e;
   }
   static_assert(kPowerBlock == 256, "the push's workgroups");
-  const PowerWork w = {power_bufs(*d), d->history + (size_t)row * d->pN * d->pNl, n_time % d->pNf, d->pblocks,
+  bool fresh;
+  const unsigned slot = sampler_slot(d, n_time, &fresh);
+  const PowerWork w = {power_bufs(*d), d->history + (size_t)row * d->pN * d->pNl, slot, fresh, d->pblocks,
                        (unsigned)d->pblocks * d->pNz};
   return push(d, p, und, n_und, time_bunch, bunch_time_step, n_sub, 1, &w);
 }

@@ -10,9 +10,10 @@
 // frequency keeps its eight sums per node and exchanges the slot's old products for the new ones.
 // The products are exact (Dekker's two-product by FMA) and the sums are pairs of doubles (Knuth's
 // two-sum), so what is taken out is what was put in and the sums carry some 100 bits, more than the
-// plain sum over the ring has.  They are summed afresh whenever slot 0 comes round, which bounds
-// what their rounding can collect to one pass over the ring, and a node whose sums are not finite
-// sums its ring plainly.  Walking the ring of 139-152 slots at every step, with one workgroup per
+// plain sum over the ring has.  They are summed afresh at slot 0 and whenever a slot does not lie behind the
+// one sampled before it (sampler_slot), so that no more than one pass over the ring collects rounding or
+// keeps what is left of a value far larger than those after it, however the samples are spaced.  A node whose
+// sums are not finite is summed afresh too, and plainly while its ring holds an infinity or a NaN.  Walking the ring of 139-152 slots at every step, with one workgroup per
 // 256 nodes, was bound by the latency of those reads on small planes and by the bytes (32 a slot
 // and node) on large ones: 32 x 32 nodes 24 -> 12 us a step between events, 71 x 71 27 -> 12.5,
 // 128 x 128 33 -> 15, 256 x 256 70 -> 20.
@@ -94,9 +95,10 @@ __device__ inline double power_of(const double* f) {
   return (f[0] * f[6] - f[1] * -f[7]) - (f[2] * f[4] - f[3] * -f[5]);
 }
 
-// Workgroup bx of nbx of inside plane pz; row receives the plane's N x Nl powers.
+// Workgroup bx of nbx of inside plane pz; row receives the plane's N x Nl powers.  fresh: the sums are
+// taken from the whole ring.
 __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs& B, double* __restrict__ row, int N0,
-                                  int N1, unsigned slot, int bx, int nbx, unsigned pz) {
+                                  int N1, unsigned slot, bool fresh, int bx, int nbx, unsigned pz) {
   const long ni_count = (long)(N0 - 4) * (N1 - 4);
   const long t = (long)bx * blockDim.x + threadIdx.x;
   const long N1N0 = (long)N1 * N0;
@@ -107,7 +109,7 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
   const long i = own ? 2 + t / (N1 - 4) : 0, j = own ? 2 + t % (N1 - 4) : 0;
   const long node = (long)N1 * i + j;
   const gptr<double> ring = G(B.ring) + (size_t)pz * N1N0 + node;  // of this node: slot m, field f at m ring_slot + f field
-  double fresh[4], old[4] = {0.0, 0.0, 0.0, 0.0};
+  double put[4], old[4] = {0.0, 0.0, 0.0, 0.0};
   if (own) {
     const gptr<const f2> ebg = G(reinterpret_cast<const f2*>(eb));
     const long mi = (long)G(B.plane_k)[pz] * N1N0 + node;
@@ -119,15 +121,15 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
     const double et1 = (1.0 - dzr) * (double)a0.y + dzr * (double)b0.y;
     const double bt0 = (1.0 - dzr) * (double)a1.y + dzr * (double)b1.y;
     const double bt1 = (1.0 - dzr) * (double)a2.x + dzr * (double)b2.x;
-    fresh[0] = B.gamma * (et0 + B.c0 * B.beta * bt1);
-    fresh[1] = B.gamma * (et1 - B.c0 * B.beta * bt0);
-    fresh[2] = B.gamma * (bt0 - B.beta / B.c0 * et1);
-    fresh[3] = B.gamma * (bt1 + B.beta / B.c0 * et0);
+    put[0] = B.gamma * (et0 + B.c0 * B.beta * bt1);
+    put[1] = B.gamma * (et1 - B.c0 * B.beta * bt0);
+    put[2] = B.gamma * (bt0 - B.beta / B.c0 * et1);
+    put[3] = B.gamma * (bt1 + B.beta / B.c0 * et0);
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const gptr<double> r = ring + slot * ring_slot + f * field;
-      if (B.sums && slot) old[f] = *r;
-      *r = fresh[f];
+      if (B.sums && !fresh) old[f] = *r;
+      *r = put[f];
     }
   }
   for (unsigned l = 0; l < B.Nl; ++l) {
@@ -139,15 +141,23 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
       bool finite = false;
       if (B.sums) {
         Sum2 q[8];
-        if (slot) {
+        auto settled = [&]() {
+          bool ok = true;
+#pragma unroll
+          for (int k = 0; k < 8; ++k) ok = ok && isfinite(q[k].hi) && isfinite(q[k].lo);
+          return ok;
+        };
+        if (!fresh) {
           const double cs = w[2 * slot], sn = w[2 * slot + 1];
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
             q[k] = {S[2 * k * N1N0], S[(2 * k + 1) * N1N0]};
-            q[k] = add_product(q[k], fresh[k >> 1], k & 1 ? sn : cs);
+            q[k] = add_product(q[k], put[k >> 1], k & 1 ? sn : cs);
             q[k] = add_product(q[k], -old[k >> 1], k & 1 ? sn : cs);
           }
-        } else {
+          finite = settled();
+        }
+        if (!finite) {
 #pragma unroll
           for (int k = 0; k < 8; ++k) q[k] = {0.0, 0.0};
           walk_ring<2>(ring, field, w, B.Nf, [&](const double* x, double cs, double sn) {
@@ -157,12 +167,11 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
               q[2 * f + 1] = add_product(q[2 * f + 1], x[f], sn);
             }
           });
+          finite = settled();
         }
-        finite = true;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
           sum[k] = q[k].hi;
-          finite = finite && isfinite(q[k].hi) && isfinite(q[k].lo);
           S[2 * k * N1N0] = q[k].hi;
           S[(2 * k + 1) * N1N0] = q[k].lo;
         }
@@ -177,12 +186,6 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
             sum[2 * f + 1] += x[f] * sn;
           }
         });
-        if (B.sums)
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            S[2 * k * N1N0] = sum[k];
-            S[(2 * k + 1) * N1N0] = 0.0;
-          }
       }
       v = B.pc * power_of(sum);
     }
@@ -213,6 +216,14 @@ __device__ inline void power_body(const float* __restrict__ eb, const PowerBufs&
       if (plane_of[k] == (int)pz) row[k * B.Nl + l] = s;
   }
   if (threadIdx.x == 0) B.done[pz] = 0;  // for the next launch
+}
+
+// The slot a domain samples at n_time, and whether its sums start afresh there.
+inline unsigned sampler_slot(Domain* d, unsigned n_time, bool* fresh) {
+  const unsigned slot = n_time % d->pNf;
+  *fresh = slot == 0 || (long)slot <= d->pslot;
+  d->pslot = slot;
+  return slot;
 }
 
 // Of a Domain or a BatchView (their members are named alike)
