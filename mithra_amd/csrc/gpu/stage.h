@@ -26,7 +26,7 @@ struct HostStage {
 
 // Chunks of a transfer of `total` bytes: four of them for overlap, but not so small that their launches
 // show nor so large that the pinned memory does.
-constexpr size_t kSlotLow = 256 << 10, kSlotHigh = 2 << 20;
+constexpr size_t kSlotLow = 512 << 10, kSlotHigh = 2 << 20;
 
 inline void stage_free(HostStage* h) {
   if (h->base) (void)hipHostFree(h->base);

@@ -396,6 +396,12 @@ __global__ void k_next_epoch(int* epoch) {
   if (threadIdx.x == 0) *epoch += 1;
 }
 
+// A chunk of the outputs into pinned memory.
+__global__ __launch_bounds__(256) void k_copy_out(const float* __restrict__ y, float* __restrict__ out, long n) {
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (t < n) out[t] = y[t];
+}
+
 __global__ void k_fill(float* __restrict__ p, long n, float v) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) p[t] = v;
@@ -766,7 +772,8 @@ int mithra_mlp_forward(mithra_mlp* p, const float* x, long n, float* y) {
   if (int rc = forward(p, 0, p->members, n, false)) return rc;
   const float* out = p->Z[p->layers - 1];
   auto put = [&](long i, long m, char* slot) {
-    return hipMemcpyAsync(slot, out + i, sizeof(float) * m, hipMemcpyDeviceToHost, p->stream);
+    hipLaunchKernelGGL(k_copy_out, dim3(blocks(m)), dim3(256), 0, p->stream, out + i, (float*)slot, m);
+    return hipGetLastError();
   };
   auto take = [&](long i, long m, const char* slot) { std::memcpy(y + i, slot, sizeof(float) * m); };
   return mithra::stage_chunks(&p->stage, p->stream, (long)p->members * n * dL, sizeof(float), put, take);
