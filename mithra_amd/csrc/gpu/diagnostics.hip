@@ -48,8 +48,8 @@ int diag_room(mithra_dev* d, size_t bytes) {
 }
 
 // E, B (e, b[3 q + c]), A^n (a[3 q + c]) and phi^n (phi[q]; 0 without space charge) of nodes[q], in the
-// caller's layout: list and results lie in pinned host memory.  A thread takes one component, and the
-// indices were checked against the mesh on the host.
+// caller's layout: list and results lie in one slot, in pinned host memory where it can be had.  A thread
+// takes one component, and the indices were checked against the mesh on the host.
 template <typename R>
 __global__ __launch_bounds__(256) void k_sample_nodes(const long* __restrict__ nodes, long n,
                                                       const float* __restrict__ eb, FieldSet an, int ncomp,
@@ -233,12 +233,12 @@ int mithra_dev_sample_nodes(mithra_dev* d, const long* nodes, long n, float* e, 
     *pe = (float*)(*pp + m);
     *pb = *pe + 3 * m;
   };
-  auto put = [&](long q0, long m, char* slot) {
+  auto list = [&](long q0, long m, char* slot) { std::memcpy(slot, nodes + q0, sizeof(long) * m); };
+  auto put = [&](long, long m, char* slot) {
     long* pn;
     double *pa, *pp;
     float *pe, *pb;
     parts(slot, m, &pn, &pa, &pp, &pe, &pb);
-    std::memcpy(pn, nodes + q0, sizeof(long) * m);
     const dim3 grid((unsigned)((3 * m + 255) / 256));
     if (d->precision == MITHRA_PRECISION_FP64)
       hipLaunchKernelGGL(k_sample_nodes<double>, grid, dim3(256), 0, d->stream, pn, m, d->eb, an, d->ncomp, pe, pb,
@@ -258,7 +258,8 @@ int mithra_dev_sample_nodes(mithra_dev* d, const long* nodes, long n, float* e, 
     if (a) std::memcpy(a + 3 * q0, pa, sizeof(double) * 3 * m);
     if (phi) std::memcpy(phi + q0, pp, sizeof(double) * m);
   };
-  return stage_chunks(&d->stage, d->stream, n, sizeof(long) + 4 * sizeof(double) + 6 * sizeof(float), put, take);
+  return stage_listed(&d->stage, d->stream, n, sizeof(long) + 4 * sizeof(double) + 6 * sizeof(float), sizeof(long),
+                      list, put, take);
 }
 
 int mithra_dev_bunch_sums(mithra_dev* d, double* out) {

@@ -4,7 +4,8 @@
 // here, and a host pass more wherever the caller's layout is not the device's.  Instead two slots
 // of pinned memory alternate: a kernel writes a chunk, already in the caller's layout, over the bus
 // into one slot while the host copies the other slot out, so that the host copy (32 GB/s into fresh pages)
-// bounds it, no device memory is needed, and no host pass is spent on the layout.  Measured:
+// bounds it, no device memory is needed, and no host pass is spent on the layout.  Where pinned memory is
+// refused, the chunks go through a slot on the device and the runtime's pageable copy.  Measured:
 // 262144 particles' records (23 MB) 6.8 -> 1.05 ms, the potentials of two levels of 131072 nodes (6.3 MB)
 // 1.17 -> 0.39 ms, 524k of a mesh's nodes by index 4.1 -> 1.4 ms.
 #pragma once
@@ -13,6 +14,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <new>
 
 #include "../../../include/mithra_gpu.h"
 
@@ -35,7 +37,8 @@ inline void stage_free(HostStage* h) {
   *h = HostStage{};
 }
 
-// Nothing may be in flight on the stage's slots (stage_chunks leaves none).
+// Room for two slots of `slot` bytes; E_NOMEM where the pinned memory is refused (the stage then has none).
+// Nothing may be in flight on the stage's slots (the transfers leave none).
 inline int stage_room(HostStage* h, size_t slot) {
   for (auto& e : h->ev)
     if (!e) {
@@ -47,16 +50,53 @@ inline int stage_room(HostStage* h, size_t slot) {
   h->base = nullptr;
   h->slot = 0;
   void* p = nullptr;
-  if (hipHostMalloc(&p, 2 * slot, hipHostMallocDefault) != hipSuccess) return MITHRA_E_NOMEM;
+  if (hipHostMalloc(&p, 2 * slot, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // answered here: no later launch is to report it
+    return MITHRA_E_NOMEM;
+  }
   h->base = (char*)p;
   h->slot = slot;
   return MITHRA_OK;
 }
 
-// n items of `unit` bytes to the host: put(first, count, slot) enqueues on `s` what writes a chunk into the
-// slot, take(first, count, slot) copies it out on the host.  The stream is idle on return.
-template <class Put, class Take>
-int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take take) {
+// The transfer where no pinned memory is to be had: chunk by chunk through a slot on the device, given back
+// at the end, and a pageable one.
+template <class List, class Put, class Take>
+int stage_pageable(hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
+  void* dev = nullptr;
+  size_t slot = std::max(kSlotLow, unit);
+  while (hipMalloc(&dev, slot) != hipSuccess) {
+    (void)hipGetLastError();
+    dev = nullptr;
+    if (slot / 2 < std::max<size_t>(4096, unit)) return MITHRA_E_NOMEM;
+    slot /= 2;
+  }
+  const long per = (long)(slot / unit);
+  char* host = new (std::nothrow) char[std::min(slot, (size_t)n * unit)];
+  hipError_t e = host ? hipSuccess : hipErrorOutOfMemory;
+  for (long first = 0; first < n && e == hipSuccess; first += per) {
+    const long m = std::min(per, n - first);
+    if (listed) {
+      list(first, m, host);
+      e = hipMemcpyAsync(dev, host, listed * m, hipMemcpyHostToDevice, s);
+    }
+    if (e == hipSuccess) e = put(first, m, (char*)dev);
+    if (e == hipSuccess) e = hipMemcpyAsync(host, dev, unit * m, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess) take(first, m, (const char*)host);
+  }
+  const hipError_t done = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = done;
+  (void)hipFree(dev);
+  delete[] host;
+  return e == hipSuccess ? MITHRA_OK : e == hipErrorOutOfMemory ? MITHRA_E_NOMEM : MITHRA_E_HIP - (int)e;
+}
+
+// n items of `unit` bytes to the host: list(first, count, slot) fills the `listed` bytes an item at the
+// slot's beginning that the kernel reads, put(first, count, slot) enqueues on `s` what writes a chunk into the slot,
+// take(first, count, slot) copies it out on the host.  The stream is idle on return.
+template <class List, class Put, class Take>
+int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
   if (n <= 0) {
     const hipError_t idle = hipStreamSynchronize(s);
     return idle == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)idle;
@@ -64,13 +104,16 @@ int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take
   const size_t want = std::min(std::max((size_t)n * unit / 4, kSlotLow), kSlotHigh);
   const long per = std::min<long>(n, std::max<long>(1, (long)(want / unit)));
   const size_t bytes = ((size_t)per * unit + 255) / 256 * 256;
-  if (int rc = stage_room(h, bytes)) return rc;
+  if (const int rc = stage_room(h, bytes))
+    return rc == MITHRA_E_NOMEM ? stage_pageable(s, n, unit, listed, list, put, take) : rc;
   const long chunks = (n + per - 1) / per;
   hipError_t e = hipSuccess;
   for (long c = 0; c <= chunks && e == hipSuccess; ++c) {
     if (c < chunks) {
-      const long first = c * per;
-      e = put(first, std::min(per, n - first), h->base + (c & 1) * h->slot);
+      const long first = c * per, m = std::min(per, n - first);
+      char* slot = h->base + (c & 1) * h->slot;
+      if (listed) list(first, m, slot);
+      e = put(first, m, slot);
       if (e == hipSuccess) e = hipEventRecord(h->ev[c & 1], s);
     }
     if (c > 0 && e == hipSuccess) {
@@ -82,6 +125,12 @@ int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take
   const hipError_t done = hipStreamSynchronize(s);
   if (e == hipSuccess) e = done;
   return e == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)e;
+}
+
+// The same without a list.
+template <class Put, class Take>
+int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take take) {
+  return stage_listed(h, s, n, unit, 0, [](long, long, char*) {}, put, take);
 }
 
 }  // namespace mithra

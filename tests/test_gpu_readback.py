@@ -61,7 +61,7 @@ def test_fields_come_back(shape, space_charge, precision):
         assert np.array_equal(sphi, phi0[at] if space_charge else np.zeros(count))
 
 
-@pytest.mark.parametrize("n", [1, 63, 2978, 2979, 40001])  # 2978 records: the last that fit one slot
+@pytest.mark.parametrize("n", [1, 63, 2978, 2979, 5957, 5958, 40001])  # 5957 records: the last that fit one slot
 def test_particles_come_back_in_load_order(n):
     rng = np.random.default_rng(n)
     dom = _domain((32, 32, 64), abi.PRECISION_FP64, 0)
