@@ -24,17 +24,33 @@ struct HostStage {
   char* base;       // two slots, pinned; kept by the owner for its next transfer
   size_t slot;      // bytes of one
   hipEvent_t ev[2];
+  void* dev;        // a slot on the device, for transfers without pinned memory
+  size_t dev_slot;
+  bool used;        // a transfer has been made
 };
 
 // Chunks of a transfer of `total` bytes: four of them for overlap, but not so small that their launches
 // show nor so large that the pinned memory does.
 constexpr size_t kSlotLow = 512 << 10, kSlotHigh = 2 << 20;
 
+// An owner's first transfer goes without pinned memory up to this many bytes: allocating and freeing that takes
+// more than a pageable copy of as much, and many owners are read once.  A fresh domain's first ten nodes by
+// index, us: 50 through pinned slots, 41 so; a small network's first prediction (3 x 512 rows of 5): 74, 60.
+constexpr size_t kOnce = 64 << 10;
+
 inline void stage_free(HostStage* h) {
   if (h->base) (void)hipHostFree(h->base);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
+  if (h->dev) (void)hipFree(h->dev);
   *h = HostStage{};
+}
+
+// Whether this is the owner's first transfer, and one of `most` bytes or less.
+inline bool stage_first(HostStage* h, size_t bytes, size_t most) {
+  const bool first = !h->used;
+  h->used = true;
+  return first && bytes <= most;
 }
 
 // Room for two slots of `slot` bytes; E_NOMEM where the pinned memory is refused (the stage then has none).
@@ -59,18 +75,28 @@ inline int stage_room(HostStage* h, size_t slot) {
   return MITHRA_OK;
 }
 
-// The transfer where no pinned memory is to be had: chunk by chunk through a slot on the device, given back
-// at the end, and a pageable one.
+// The transfer without pinned memory: chunk by chunk through a slot on the device, which the owner keeps, and a
+// pageable one.
 template <class List, class Put, class Take>
-int stage_pageable(hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
-  void* dev = nullptr;
-  size_t slot = std::max(kSlotLow, unit);
-  while (hipMalloc(&dev, slot) != hipSuccess) {
-    (void)hipGetLastError();
-    dev = nullptr;
-    if (slot / 2 < std::max<size_t>(4096, unit)) return MITHRA_E_NOMEM;
-    slot /= 2;
+int stage_pageable(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
+  const size_t want = std::max(std::min(kSlotLow, (size_t)n * unit), unit);
+  if (h->dev_slot < want) {
+    void* p = nullptr;
+    size_t slot = want;
+    while (slot > h->dev_slot && hipMalloc(&p, slot) != hipSuccess) {  // down to what it has, or a page
+      (void)hipGetLastError();
+      p = nullptr;
+      slot = slot / 2 < std::max<size_t>(4096, unit) ? 0 : slot / 2;
+    }
+    if (p) {
+      if (h->dev) (void)hipFree(h->dev);
+      h->dev = p;
+      h->dev_slot = slot;
+    }
   }
+  if (h->dev_slot < unit) return MITHRA_E_NOMEM;
+  void* const dev = h->dev;
+  const size_t slot = h->dev_slot;
   const long per = (long)(slot / unit);
   char* host = new (std::nothrow) char[std::min(slot, (size_t)n * unit)];
   hipError_t e = host ? hipSuccess : hipErrorOutOfMemory;
@@ -87,7 +113,6 @@ int stage_pageable(hipStream_t s, long n, size_t unit, size_t listed, List list,
   }
   const hipError_t done = hipStreamSynchronize(s);
   if (e == hipSuccess) e = done;
-  (void)hipFree(dev);
   delete[] host;
   return e == hipSuccess ? MITHRA_OK : e == hipErrorOutOfMemory ? MITHRA_E_NOMEM : MITHRA_E_HIP - (int)e;
 }
@@ -101,11 +126,12 @@ int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed
     const hipError_t idle = hipStreamSynchronize(s);
     return idle == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)idle;
   }
+  if (stage_first(h, (size_t)n * unit, kOnce)) return stage_pageable(h, s, n, unit, listed, list, put, take);
   const size_t want = std::min(std::max((size_t)n * unit / 4, kSlotLow), kSlotHigh);
   const long per = std::min<long>(n, std::max<long>(1, (long)(want / unit)));
   const size_t bytes = ((size_t)per * unit + 255) / 256 * 256;
   if (const int rc = stage_room(h, bytes))
-    return rc == MITHRA_E_NOMEM ? stage_pageable(s, n, unit, listed, list, put, take) : rc;
+    return rc == MITHRA_E_NOMEM ? stage_pageable(h, s, n, unit, listed, list, put, take) : rc;
   const long chunks = (n + per - 1) / per;
   hipError_t e = hipSuccess;
   for (long c = 0; c <= chunks && e == hipSuccess; ++c) {

@@ -771,12 +771,19 @@ int mithra_mlp_forward(mithra_mlp* p, const float* x, long n, float* y) {
   const int dL = p->dims[p->layers];
   if (int rc = forward(p, 0, p->members, n, false)) return rc;
   const float* out = p->Z[p->layers - 1];
+  const long values = (long)p->members * n * dL;
+  // the layout is the caller's: a network's only prediction, when small, is a plain copy (see kOnce)
+  if (mithra::stage_first(&p->stage, sizeof(float) * values, 3 << 19)) {
+    SG_TRY(hipMemcpyAsync(y, out, sizeof(float) * values, hipMemcpyDeviceToHost, p->stream));
+    SG_TRY(hipStreamSynchronize(p->stream));
+    return MITHRA_OK;
+  }
   auto put = [&](long i, long m, char* slot) {
     hipLaunchKernelGGL(k_copy_out, dim3(blocks(m)), dim3(256), 0, p->stream, out + i, (float*)slot, m);
     return hipGetLastError();
   };
   auto take = [&](long i, long m, const char* slot) { std::memcpy(y + i, slot, sizeof(float) * m); };
-  return mithra::stage_chunks(&p->stage, p->stream, (long)p->members * n * dL, sizeof(float), put, take);
+  return mithra::stage_chunks(&p->stage, p->stream, values, sizeof(float), put, take);
 }
 
 // Loss (mean squared error over the n x d_out targets) and its gradient for one member, in the

@@ -1,6 +1,6 @@
 // Staged transfers (mithra_amd/csrc/gpu/stage.h) on a runtime of the host's own that refuses memory on demand
 // and, as HIP does, keeps a refusal as the last error until it is asked for.  Each line printed: what ran, status,
-// whether the items came through, calls of `put`, bytes still pinned or allocated.
+// whether the items came through, calls of `put`, bytes held pinned, bytes held on the device.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -11,23 +11,28 @@
 
 size_t pinned_most = ~(size_t)0, device_most = ~(size_t)0;  // refused above
 hipError_t last = hipSuccess;
-std::map<void*, size_t> held;
-
-static hipError_t grant(void** p, size_t n, size_t most) {
-  if (n > most) return last = hipErrorOutOfMemory;
-  *p = std::malloc(n);
-  held[*p] = n;
-  return hipSuccess;
-}
-static hipError_t give_back(void* p) {
-  held.erase(p);
-  std::free(p);
-  return hipSuccess;
-}
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return grant(p, n, pinned_most); }
-hipError_t hipHostFree(void* p) { return give_back(p); }
-hipError_t hipMalloc(void** p, size_t n) { return grant(p, n, device_most); }
-hipError_t hipFree(void* p) { return give_back(p); }
+struct Memory {
+  std::map<void*, size_t> held;
+  hipError_t grant(void** p, size_t n, size_t most) {
+    if (n > most) return last = hipErrorOutOfMemory;
+    held[*p = std::malloc(n)] = n;
+    return hipSuccess;
+  }
+  hipError_t give_back(void* p) {
+    held.erase(p);
+    std::free(p);
+    return hipSuccess;
+  }
+  size_t bytes() const {
+    size_t sum = 0;
+    for (auto& a : held) sum += a.second;
+    return sum;
+  }
+} pinned, device;
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return pinned.grant(p, n, pinned_most); }
+hipError_t hipHostFree(void* p) { return pinned.give_back(p); }
+hipError_t hipMalloc(void** p, size_t n) { return device.grant(p, n, device_most); }
+hipError_t hipFree(void* p) { return device.give_back(p); }
 hipError_t hipGetLastError() {
   const hipError_t e = last;
   last = hipSuccess;
@@ -62,27 +67,31 @@ static void transfer(const char* name, mithra::HostStage* h, long n, size_t fail
   const int rc = mithra::stage_chunks(h, 0, n, sizeof(Item), put, take);
   bool good = true;
   for (long i = 0; i < n; ++i) good = good && got[i].in == i && got[i].out[9] == 3.0 * (double)i;
-  size_t bytes = 0;
-  for (auto& a : held) bytes += a.second;
-  std::printf("%s %ld %d %d %zu %zu\n", name, n, rc, (int)good, puts, bytes);
+  std::printf("%s %ld %d %d %zu %zu %zu\n", name, n, rc, (int)good, puts, pinned.bytes(), device.bytes());
 }
 
 int main() {
-  for (long n : {0L, 1L, 5957L, 5958L, 100001L}) {
+  for (long n : {0L, 1L, 744L, 745L, 5957L, 5958L, 100001L}) {
     mithra::HostStage h = {};
+    transfer("first", &h, n);
     transfer("pinned", &h, n);
-    transfer("again", &h, n);
+    transfer("failing", &h, n, 0);
     mithra::stage_free(&h);
     pinned_most = 0;
     transfer("refused", &h, n);
-    device_most = 100000;
+    transfer("refused", &h, n);
+    pinned_most = ~(size_t)0;
+    transfer("granted", &h, n);
+    mithra::stage_free(&h);
+    pinned_most = 0;
+    device_most = 50000;
     transfer("little", &h, n);
+    transfer("little", &h, n);
+    mithra::stage_free(&h);
     device_most = 0;
     transfer("none", &h, n);
-    device_most = pinned_most = ~(size_t)0;
-    transfer("granted", &h, n);
-    transfer("failing", &h, n, 0);
     mithra::stage_free(&h);
-    std::printf("left %ld %zu 0 0 0\n", n, held.size());
+    device_most = pinned_most = ~(size_t)0;
+    std::printf("left %ld 0 0 0 %zu %zu\n", n, pinned.bytes(), device.bytes());
   }
 }

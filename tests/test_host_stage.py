@@ -27,27 +27,38 @@ def of(lines, name):
     return [line[1:] for line in lines if line[0] == name]
 
 
-@pytest.mark.parametrize("name", ["pinned", "again", "refused", "little", "granted"])
+SIZES = [0, 1, 744, 745, 5957, 5958, 100001]
+
+
+@pytest.mark.parametrize("name", ["first", "pinned", "refused", "little", "granted"])
 def test_transfer_comes_through(lines, name):
-    """With pinned memory, without any, with a device that grants 100 kB at most, and with pinned memory granted
+    """With pinned memory, without any, with a device that grants 50 kB at most, and with pinned memory granted
     again after a refusal, whose error no later launch may report."""
-    assert len(of(lines, name)) == 5
-    for n, status, good, _, _ in of(lines, name):
+    assert sorted({line[0] for line in of(lines, name)}) == SIZES
+    for n, status, good, *_ in of(lines, name):
         assert (status, good) == (OK, 1), (name, n)
 
 
 def test_nothing_granted(lines):
-    for n, status, good, puts, held in of(lines, "none"):
-        assert (status, puts, held) == ((OK if n == 0 else NOMEM), 0, 0)
+    for n, status, good, puts, *held in of(lines, "none"):
+        assert (status, puts, held) == (OK if n == 0 else NOMEM, 0, [0, 0])
 
 
 def test_failing_chunk_ends_the_transfer(lines):
-    for n, status, good, puts, _ in of(lines, "failing"):
+    for n, status, good, puts, *_ in of(lines, "failing"):
         assert (status != OK, puts) == ((n > 0), min(n, 1))
 
 
-def test_memory_is_given_back(lines):
-    for _, held, *_ in of(lines, "left"):
-        assert held == 0
-    for name in ("refused", "little"):
-        assert all(held == 0 for *_, held in of(lines, name))
+def test_memory_is_bounded_and_given_back(lines):
+    for _, _, _, _, *held in of(lines, "left"):
+        assert held == [0, 0]
+    for name, most in (("refused", 512 << 10), ("little", 50000)):
+        for *_, pinned, device in of(lines, name):
+            assert pinned == 0 and device <= most
+    assert max(line[4] for line in of(lines, "pinned")) <= 4 << 20
+
+
+def test_a_first_small_transfer_pins_nothing(lines):
+    """744 records are 64 kB: as many as an owner's first transfer takes without pinned memory."""
+    assert [line[4] > 0 for line in of(lines, "first")] == [n > 744 for n in SIZES]
+    assert [line[4] > 0 for line in of(lines, "pinned")] == [n > 0 for n in SIZES]
