@@ -258,8 +258,8 @@ int mithra_dev_sample_nodes(mithra_dev* d, const long* nodes, long n, float* e, 
     if (a) std::memcpy(a + 3 * q0, pa, sizeof(double) * 3 * m);
     if (phi) std::memcpy(phi + q0, pp, sizeof(double) * m);
   };
-  return stage_listed(&d->stage, d->stream, n, sizeof(long) + 4 * sizeof(double) + 6 * sizeof(float), sizeof(long),
-                      list, put, take);
+  return stage_listed(&d->stage, d->stream, n, sizeof(long) + 4 * sizeof(double) + 6 * sizeof(float), kAnyChunks,
+                      sizeof(long), list, put, take);
 }
 
 int mithra_dev_bunch_sums(mithra_dev* d, double* out) {

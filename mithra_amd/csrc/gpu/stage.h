@@ -33,6 +33,8 @@ struct HostStage {
 // show nor so large that the pinned memory does.
 constexpr size_t kSlotLow = 512 << 10, kSlotHigh = 2 << 20;
 
+constexpr long kAnyChunks = 1l << 62;
+
 // An owner's first transfer goes without pinned memory up to this many bytes: allocating and freeing that takes
 // more than a pageable copy of as much, and many owners are read once.  A fresh domain's first ten nodes by
 // index, us: 50 through pinned slots, 41 so; a small network's first prediction (3 x 512 rows of 5): 74, 60.
@@ -78,8 +80,9 @@ inline int stage_room(HostStage* h, size_t slot) {
 // The transfer without pinned memory: chunk by chunk through a slot on the device, which the owner keeps, and a
 // pageable one.
 template <class List, class Put, class Take>
-int stage_pageable(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
-  const size_t want = std::max(std::min(kSlotLow, (size_t)n * unit), unit);
+int stage_pageable(HostStage* h, hipStream_t s, long n, size_t unit, long chunks, size_t listed, List list, Put put,
+                   Take take) {
+  const size_t want = std::max(std::min(kSlotLow, (size_t)n * unit), (size_t)((n + chunks - 1) / chunks) * unit);
   if (h->dev_slot < want) {
     void* p = nullptr;
     size_t slot = want;
@@ -119,19 +122,21 @@ int stage_pageable(HostStage* h, hipStream_t s, long n, size_t unit, size_t list
 
 // n items of `unit` bytes to the host: list(first, count, slot) fills the `listed` bytes an item at the
 // slot's beginning that the kernel reads, put(first, count, slot) enqueues on `s` what writes a chunk into the slot,
-// take(first, count, slot) copies it out on the host.  The stream is idle on return.
+// take(first, count, slot) copies it out on the host.  No more than `most` chunks, where the memory for
+// larger ones can be had.  The stream is idle on return.
 template <class List, class Put, class Take>
-int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed, List list, Put put, Take take) {
+int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, long most, size_t listed, List list, Put put,
+                 Take take) {
   if (n <= 0) {
     const hipError_t idle = hipStreamSynchronize(s);
     return idle == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)idle;
   }
-  if (stage_first(h, (size_t)n * unit, kOnce)) return stage_pageable(h, s, n, unit, listed, list, put, take);
+  if (stage_first(h, (size_t)n * unit, kOnce)) return stage_pageable(h, s, n, unit, most, listed, list, put, take);
   const size_t want = std::min(std::max((size_t)n * unit / 4, kSlotLow), kSlotHigh);
-  const long per = std::min<long>(n, std::max<long>(1, (long)(want / unit)));
+  const long per = std::min<long>(n, std::max<long>((n + most - 1) / most, (long)(want / unit)));
   const size_t bytes = ((size_t)per * unit + 255) / 256 * 256;
   if (const int rc = stage_room(h, bytes))
-    return rc == MITHRA_E_NOMEM ? stage_pageable(h, s, n, unit, listed, list, put, take) : rc;
+    return rc == MITHRA_E_NOMEM ? stage_pageable(h, s, n, unit, most, listed, list, put, take) : rc;
   const long chunks = (n + per - 1) / per;
   hipError_t e = hipSuccess;
   for (long c = 0; c <= chunks && e == hipSuccess; ++c) {
@@ -155,8 +160,8 @@ int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, size_t listed
 
 // The same without a list.
 template <class Put, class Take>
-int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take take) {
-  return stage_listed(h, s, n, unit, 0, [](long, long, char*) {}, put, take);
+int stage_chunks(HostStage* h, hipStream_t s, long n, size_t unit, Put put, Take take, long most = kAnyChunks) {
+  return stage_listed(h, s, n, unit, most, 0, [](long, long, char*) {}, put, take);
 }
 
 }  // namespace mithra

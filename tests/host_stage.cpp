@@ -50,7 +50,8 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 
 #include "stage.h"
 
-static void transfer(const char* name, mithra::HostStage* h, long n, size_t fail_at = ~(size_t)0) {
+static void transfer(const char* name, mithra::HostStage* h, long n, size_t fail_at = ~(size_t)0,
+                     long most = 1l << 62) {
   struct Item { long in; double out[10]; };  // 88 bytes, as a particle's record
   std::vector<Item> got(n);
   size_t puts = 0;
@@ -64,7 +65,7 @@ static void transfer(const char* name, mithra::HostStage* h, long n, size_t fail
     return hipGetLastError();  // as after a launch
   };
   auto take = [&](long first, long m, const char* slot) { std::memcpy(got.data() + first, slot, sizeof(Item) * m); };
-  const int rc = mithra::stage_chunks(h, 0, n, sizeof(Item), put, take);
+  const int rc = mithra::stage_chunks(h, 0, n, sizeof(Item), put, take, most);
   bool good = true;
   for (long i = 0; i < n; ++i) good = good && got[i].in == i && got[i].out[9] == 3.0 * (double)i;
   std::printf("%s %ld %d %d %zu %zu %zu\n", name, n, rc, (int)good, puts, pinned.bytes(), device.bytes());
@@ -77,7 +78,11 @@ int main() {
     transfer("pinned", &h, n);
     transfer("failing", &h, n, 0);
     mithra::stage_free(&h);
+    transfer("three", &h, n, ~(size_t)0, 3);
+    mithra::stage_free(&h);
     pinned_most = 0;
+    transfer("three", &h, n, ~(size_t)0, 3);
+    mithra::stage_free(&h);
     transfer("refused", &h, n);
     transfer("refused", &h, n);
     pinned_most = ~(size_t)0;

@@ -62,3 +62,8 @@ def test_a_first_small_transfer_pins_nothing(lines):
     """744 records are 64 kB: as many as an owner's first transfer takes without pinned memory."""
     assert [line[4] > 0 for line in of(lines, "first")] == [n > 744 for n in SIZES]
     assert [line[4] > 0 for line in of(lines, "pinned")] == [n > 0 for n in SIZES]
+
+
+def test_no_more_chunks_than_asked(lines):
+    for n, status, good, puts, *_ in of(lines, "three"):
+        assert (status, good) == (OK, 1) and puts <= 3
