@@ -123,7 +123,7 @@ __device__ inline float silu_grad(float z) {
 //   kHidden z = acc + bias; Z = z (when kept for the backward pass), act = bf16(silu(z))
 //   kOutput z = acc + bias; Z = z
 //   kLoss   y = acc + bias against the targets: dZ = bf16(2 (y - t) scale), the tile's column sums of
-//           2 (y - t) scale (FP32) and its sum of (y - t)^2
+//           2 (y - t) scale (FP32) and its sum of (y - t)^2 (FP64: a tile has up to 16384 terms)
 //   kBack   g = acc silu'(Z): dZ = bf16(g), the tile's column sums of g (FP32)
 // so that biases, activations, losses and bias gradients cost no launches and no passes of their own.
 // A training step of 256 rows (five members, 264-512-512-512-256) is a chain of short launches: 30 of
@@ -143,7 +143,7 @@ struct Epi {
   float scale;
   float* colsum;       // kLoss, kBack: [row tile][N] column sums
   long scol;
-  float* loss;         // kLoss: [tile] sums of squares
+  double* loss;        // kLoss: [tile] sums of squares
   long sloss;
 };
 
@@ -212,9 +212,10 @@ __device__ inline void gemm_tile(const GemmArgs& g, const Epi& q, char* lds, int
     buf ^= 1;
   }
   // the epilogue reuses the staging memory: every wavefront is past its last read of it
-  float* const sums = reinterpret_cast<float*>(lds);  // [2][BN] column sums, [4] losses
+  float* const sums = reinterpret_cast<float*>(lds);  // [2][BN] column sums
+  double* const losses = reinterpret_cast<double*>(sums + 2 * BN);  // [4]
   constexpr bool kSums = EPI == kLoss || EPI == kBack;
-  float sq = 0.0f;
+  double sq = 0.0;
 #pragma unroll
   for (int j = 0; j < WN; ++j) {
     const int c = n0 + wn + 32 * j + (lane & 31);
@@ -242,7 +243,7 @@ __device__ inline void gemm_tile(const GemmArgs& g, const Epi& q, char* lds, int
           const float gr = 2.0f * d * q.scale;
           q.act[e * q.sact + at] = (__bf16)gr;
           col += gr;
-          sq += d * d;
+          sq += (double)d * (double)d;
         } else {
           const float gr = x * silu_grad(q.Z[e * q.sz + at]);
           q.act[e * q.sact + at] = (__bf16)gr;
@@ -257,15 +258,14 @@ __device__ inline void gemm_tile(const GemmArgs& g, const Epi& q, char* lds, int
   if (EPI == kLoss) {
 #pragma unroll
     for (int h = 32; h > 0; h >>= 1) sq += __shfl_xor(sq, h);
-    if (lane == 0) sums[2 * BN + w] = sq;
+    if (lane == 0) losses[w] = sq;
   }
   if (kSums) {
     __syncthreads();
     if ((int)threadIdx.x < BN && n0 + (int)threadIdx.x < g.N)
       q.colsum[e * q.scol + (long)by * g.N + n0 + threadIdx.x] = sums[threadIdx.x] + sums[BN + threadIdx.x];
     if (EPI == kLoss && threadIdx.x == 0)
-      q.loss[e * q.sloss + (long)by * nbx + bx] =
-          (sums[2 * BN] + sums[2 * BN + 1]) + (sums[2 * BN + 2] + sums[2 * BN + 3]);
+      q.loss[e * q.sloss + (long)by * nbx + bx] = (losses[0] + losses[1]) + (losses[2] + losses[3]);
   }
 }
 
@@ -308,15 +308,15 @@ struct BiasLayers {
 };
 
 __global__ __launch_bounds__(64) void k_bias_grad(BiasLayers t, float* __restrict__ g, long pm,
-                                                  const float* __restrict__ loss, int nb,
+                                                  const double* __restrict__ loss, int nb,
                                                   const int* __restrict__ epoch, float* __restrict__ out, int members,
                                                   float scale) {
   if (out && blockIdx.x == gridDim.x - 1) {  // one more column of workgroups than the biases take
     const int e = threadIdx.x;
     if (blockIdx.y == 0 && blockIdx.z == 0 && e < members) {
-      float s = 0.0f;
+      double s = 0.0;
       for (int i = 0; i < nb; ++i) s += loss[(long)e * nb + i];
-      out[(long)*epoch * members + e] += s * scale;
+      out[(long)*epoch * members + e] += (float)(s * (double)scale);
     }
     return;
   }
@@ -433,7 +433,7 @@ struct mithra_mlp {
   mithra::HostStage stage = {};     // pinned slots of transfers to the host
   float* xin = nullptr;             // FP32 staging of the inputs, n x d_0
   float* tgt = nullptr;             // targets, n x d_L (shared)
-  float* partial = nullptr;         // the loss's sums per tile, members x tiles
+  double* partial = nullptr;        // the loss's sums per tile, members x tiles
   int maxw = 0;
   // resident training data
   long n_data = 0;
@@ -453,7 +453,8 @@ void free_acts(mithra_mlp* p) {
   (void)hipFree(p->dZ[0]); (void)hipFree(p->dZ[1]);
   (void)hipFree(p->xin); (void)hipFree(p->tgt); (void)hipFree(p->partial);
   p->dZ[0] = p->dZ[1] = nullptr;
-  p->xin = p->tgt = p->partial = nullptr;
+  p->xin = p->tgt = nullptr;
+  p->partial = nullptr;
   p->cap = 0;
 }
 
@@ -476,7 +477,7 @@ int ensure_acts(mithra_mlp* p, long n) {
        hipMalloc(&p->dZ[1], sizeof(__bf16) * E * n * p->maxw) == hipSuccess &&
        hipMalloc(&p->xin, sizeof(float) * n * p->dims[0]) == hipSuccess &&
        hipMalloc(&p->tgt, sizeof(float) * n * p->dims[L]) == hipSuccess &&
-       hipMalloc(&p->partial, sizeof(float) * E * tiles64(n) * tiles64(p->dims[L])) == hipSuccess;
+       hipMalloc(&p->partial, sizeof(double) * E * tiles64(n) * tiles64(p->dims[L])) == hipSuccess;
   if (!ok) {
     free_acts(p);
     return MITHRA_E_NOMEM;
@@ -616,8 +617,8 @@ int backward(mithra_mlp* p, int e0, int ne, long n, float* loss, const int* epoc
     SG_TRY(hipGetLastError());
   }
   if (loss) {
-    std::vector<float> part((size_t)ne * nb);
-    SG_TRY(hipMemcpyAsync(part.data(), p->partial, sizeof(float) * part.size(), hipMemcpyDeviceToHost, s));
+    std::vector<double> part((size_t)ne * nb);
+    SG_TRY(hipMemcpyAsync(part.data(), p->partial, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
     SG_TRY(hipStreamSynchronize(s));
     for (int e = 0; e < ne; ++e) {
       double sum = 0.0;
