@@ -298,6 +298,11 @@ class March:
         self.n += 1
 
 
+def shape_name(shape):
+    rows, planes = shape
+    return f"{rows}x{planes}" if rows else f"flat, {planes} planes at most,"
+
+
 def run_gpu(job, steps, warmup, precision, reorder=16, pipelined=True, deterministic=False):
     """Warm-up, then `steps` timed steps, then a few steps with per-phase HIP events.  Pipelined:
     each group of steps is one complete pipelined run (mithra_dev_step_pipelined, more = 1 on all
@@ -310,7 +315,7 @@ def run_gpu(job, steps, warmup, precision, reorder=16, pipelined=True, determini
         dom.set_deterministic(True)
     (ci, ce), tune_ms = dom.autotune(reps=2)
     log("autotune (ms per launch, tile shapes rows x planes): " + "; ".join(
-        f"{abi.tile_shape(v)[0]}x{abi.tile_shape(v)[1]} interior {tune_ms[0, v]:.3f} eval {tune_ms[1, v]:.3f}"
+        f"{shape_name(abi.tile_shape(v))} interior {tune_ms[0, v]:.3f} eval {tune_ms[1, v]:.3f}"
         for v in range(abi.TILE_VARIANTS)))
     tiles = {"interior": list(abi.tile_shape(ci)), "eval": list(abi.tile_shape(ce))}
     if pipelined:

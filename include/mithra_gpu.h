@@ -343,15 +343,17 @@ int mithra_dev_set_reorder_interval(mithra_dev* dev, int interval);
 int mithra_dev_set_deterministic(mithra_dev* dev, int on);
 
 /* Tile shapes of the two marched field kernels (interior update, E/B evaluation): variant v
- * has `rows` x-rows of 64 y-nodes per workgroup and marches `planes` z-planes; variant 0 lays
- * its rows end to end over the plane and marches fewer planes (at most eight, fewer on small
- * meshes); variants 7-9 stage the interior update's A^n planes in LDS.  A domain starts with the
- * shapes that suit its mesh and precision.  When no TF/SF seed is injected, the interior
+ * has `rows` x-rows of 64 y-nodes per workgroup and marches `planes` z-planes; variant 0, the flat
+ * form, lays 256 lanes end to end over the plane (rows = 0) and marches at most `planes`, fewer on
+ * small meshes; variants 7-9 stage the interior update's A^n planes in LDS.  A domain starts with
+ * the shapes that suit its mesh and precision; mithra_dev_tiles reads the present ones (each
+ * pointer may be NULL; `fused` is a variant of mithra_fused_tile_shape).  When no TF/SF seed is injected, the interior
  * update of every shape also updates the Mur y faces, which the boundary pass then skips.
  * Every shape computes identical values; only the speed differs. */
 #define MITHRA_TILE_VARIANTS 10
 int mithra_tile_shape(int variant, int* rows, int* planes);
 int mithra_dev_set_tiles(mithra_dev* dev, int interior, int eval);
+int mithra_dev_tiles(const mithra_dev* dev, int* interior, int* eval, int* fused);
 /* Autotuner: times `reps` launches of every tile shape of both kernels (the interior update
  * together with the Mur boundaries, the E/B evaluation alone) on this domain's mesh and keeps
  * the fastest of each.  The domain's state is left as it was (the interior update
@@ -518,7 +520,9 @@ int mithra_dev_bunching_noalloc(mithra_dev* dev, double k, double* b_out);
 /* mithra_dev_step with HIP events recorded on the handle's stream between its phases; ms[i]
  * receives the duration of phase i: 0 interior update, 1 TF/SF, 2 Mur boundaries, 3 E/B
  * evaluation, 4 bunch sub-steps, 5 power sample, 6 current reset, 7 current deposition.
- * Waits for the step to finish.  No counterpart in the reference: the measurement hook. */
+ * Waits for the step to finish.  The phases are launched one by one, also the bunch sub-steps and the
+ * power sample, which mithra_dev_step launches together where both have work.  No counterpart
+ * in the reference: the measurement hook. */
 #define MITHRA_STEP_PHASES 8
 int mithra_dev_step_timed(mithra_dev* dev, double time, const mithra_seed* seed, const mithra_bunch_params* p,
                           const mithra_undulator* und, int n_und, double time_bunch, double bunch_time_step,
@@ -549,8 +553,8 @@ int mithra_dev_step_pipelined(mithra_dev* dev, double time, const mithra_seed* s
 /* 1 while a pipelined run is pending (the last step had more = 1 and was pipelined), else 0. */
 int mithra_dev_pipeline_pending(const mithra_dev* dev);
 /* Tile shapes of the pipelined step's fused kernel: `rows` x-rows of 64 y-nodes, `planes`
- * z-planes per workgroup (variant 0 on meshes under 5 million nodes: as variant 0 above); every
- * shape computes identical values.  autotune_fused times each
+ * z-planes per workgroup (variant 0 on meshes under 5 million nodes runs the flat form, as variant 0
+ * above, whatever its shape here); every shape computes identical values.  autotune_fused times each
  * (reps launches after one warm-up, ms[v] the mean) on the handle's current levels, keeps the
  * fastest and restores the level and the E/B array it writes.  No counterpart in the reference. */
 #define MITHRA_FUSED_TILE_VARIANTS 4

@@ -94,7 +94,7 @@ FUSED_TILE_VARIANTS = 4   # shapes of the pipelined step's fused kernel (MITHRA_
 
 
 def tile_shape(variant):
-    """(rows, planes) of a field-kernel tile variant."""
+    """(rows, planes) of a field-kernel tile variant; rows = 0: the flat form, at most `planes`."""
     lib = load_gpu_library()
     f = lib.mithra_tile_shape
     f.restype, f.argtypes = C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
@@ -199,6 +199,7 @@ def _declare(lib, prefix):
         sig["set_reorder_interval"] = (C.c_int, [vp, C.c_int])
         sig["set_deterministic"] = (C.c_int, [vp, C.c_int])
         sig["set_tiles"] = (C.c_int, [vp, C.c_int, C.c_int])
+        sig["tiles"] = (C.c_int, [vp] + 3 * [C.POINTER(C.c_int)])
         sig["set_lazy_fields"] = (C.c_int, [vp, C.c_int])
         sig["autotune"] = (C.c_int, [vp, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_float)])
         sig["bunch_advance"] = (C.c_int, [vp, C.POINTER(BunchParams), C.POINTER(Undulator), C.c_int,
@@ -454,6 +455,13 @@ class Domain:
     def set_tiles(self, interior, evaluation):
         """Tile shape variants of the interior update and the E/B evaluation."""
         self._check(self.f["set_tiles"](self.h, interior, evaluation))
+
+    def tiles(self):
+        """The present tile shape variants of the interior update, the E/B evaluation and the pipelined
+        step's fused kernel."""
+        v = [C.c_int() for _ in range(3)]
+        self._check(self.f["tiles"](self.h, *map(C.byref, v)))
+        return tuple(c.value for c in v)
 
     def autotune(self, reps=3):
         """Times every tile shape of both field kernels; keeps the fastest.  Returns

@@ -792,6 +792,14 @@ int mithra_tile_shape(int variant, int* rows, int* planes) {
   return MITHRA_OK;
 }
 
+int mithra_dev_tiles(const mithra_dev* d, int* interior, int* eval, int* fused) {
+  if (!d) return MITHRA_E_ARG;
+  if (interior) *interior = d->tile_interior;
+  if (eval) *eval = d->tile_eval;
+  if (fused) *fused = d->tile_fused;
+  return MITHRA_OK;
+}
+
 int mithra_dev_set_tiles(mithra_dev* d, int interior, int eval) {
   if (!d || interior < 0 || interior >= kTileVariants || eval < 0 || eval >= kTileVariants) return MITHRA_E_ARG;
   d->tile_interior = interior;

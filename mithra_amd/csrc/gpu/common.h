@@ -399,7 +399,8 @@ hipError_t launch_stencil_eb(Domain* d);
 constexpr int kFusedVariants = 4;
 extern const int kFusedShapes[kFusedVariants][2];
 hipError_t launch_zrange(Domain* d);  // reduces what the last push left into zrange, unless a deposit has
-// Tile shapes {rows, planes} of the marched field kernels, selected by Domain::tile_*.
+// Tile shapes {rows, planes} of the marched field kernels, selected by Domain::tile_*; shape 0, the flat
+// form, has no rows of its own.
 constexpr int kTileVariants = 10;  // 7..9: LDS-staged interior update
 extern const int kTileShapes[kTileVariants][2];
 hipError_t launch_fill_zero(Domain* d, void* ptr, size_t bytes);

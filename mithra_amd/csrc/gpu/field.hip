@@ -1892,7 +1892,7 @@ hipError_t eval_impl(Domain* d, int klo, int khi, const int* zr = nullptr, int p
 
 }  // namespace
 
-extern const int kTileShapes[kTileVariants][2] = {{4, 64}, {2, 64}, {4, 32}, {4, 128}, {8, 32},
+extern const int kTileShapes[kTileVariants][2] = {{0, 8}, {2, 64}, {4, 32}, {4, 128}, {8, 32},
                                                   {8, 64}, {16, 32}, {4, 64}, {8, 64}, {16, 64}};
 
 // The shapes a domain starts with.  In FP32 the flat interior update is the fastest at every size

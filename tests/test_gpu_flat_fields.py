@@ -62,8 +62,8 @@ def test_flat_field_update_bit_exact(size, sc, solver):
                                                     ((200, 128, 320), abi.PRECISION_FP64, (7, 8)),
                                                     ((200, 180, 150), abi.PRECISION_FP32_BULK, (0, 0))])
 def test_default_shapes_match_flat(nodes, precision, shapes):
-    """A domain's starting shapes on both sides of each size in the rule compute what the flat form
-    computes (`shapes`: the ones the rule names for this mesh)."""
+    """A domain's starting shapes on both sides of sizes in the rule are the ones it names and compute what
+    the flat form computes."""
     g = grid(*nodes, 0)
     rng = np.random.default_rng(3)
     c, n = coeffs(rng), g.nodes
@@ -71,6 +71,7 @@ def test_default_shapes_match_flat(nodes, precision, shapes):
     out = []
     for tiles in (None, (0, 0), shapes):
         d = abi.Domain(g, c, precision=precision)
+        assert d.tiles()[:2] == shapes
         if tiles:
             d.set_tiles(*tiles)
         out.append(update(d, levels, [None] * 3))
