@@ -12,8 +12,10 @@ from mithra_amd import abi
 
 pytestmark = pytest.mark.gpu
 
-# The walk over the ring rounds each of its Nf additions (Nf <= 200: a bound of Nf 2^-53 < 3e-14 of
-# the largest term); P is a difference of products of such sums over the nodes.
+# The walk over the ring rounds each of its Nf additions: Nf 2^-53 < 5e-15 of the terms' sum of magnitudes for
+# the 40 slots here.  P is a difference of products of such sums, added over nodes of both signs; 1e-11 of the
+# largest P leaves room for what these cancel, a factor of 2000.  (Where nothing cancels, the samplers are held
+# to their roundings in test_gpu_power_renewal.py.)
 RTOL = 1e-11
 
 
