@@ -1746,10 +1746,13 @@ hipError_t field_variant(Domain* d, int kernel, int v, int klo, int khi, const i
 
 // Below this many nodes the flat forms are the faster ones in FP64 too.  The tiled forms with LDS
 // planes read a node's neighbours once from L2 but march serially; they win once the
-// levels no longer fit the 256 MB last-level cache and the workgroups suffice.  us, flat against
-// tiled: fused kernel 32 x 32 x 128 with phi 12 / 163, 71 x 71 x 397 60 / 182, 90 x 90 x 301
-// 77 / 165, 128 x 128 x 1024 463 / 369; interior update 64 x 64 x 1024 135 / 142, 96 x 96 x 600
-// 172 / 167, 128 x 128 x 1024 453 / 370.
+// levels no longer fit the 256 MB last-level cache and the workgroups suffice.  The line is the interior
+// update's, us flat / 4 x 64 tiles: 64 x 64 x 1024 135 / 142, 96 x 96 x 600 169 / 164, 128 x 128 x 330 158 / 157
+// (206 / 173 with phi), 128 x 128 x 500 232 / 191; ragged meshes cross later (150 x 150 x 360 218 / 257, 200 x
+// 210 x 340 370 / 405).  The fused kernel's own line would lie at some 8 million nodes: 32 x 32 x 128 with phi 12 /
+// 163, 71 x 71 x 397 60 / 182, 90 x 90 x 301 77 / 165, 131 x 147 x 260 107 / 183 (192 / 256 with phi),
+// 96 x 96 x 600 115 / 185, 150 x 150 x 360 259 / 265, 128 x 128 x 500 247 / 226, 128 x 128 x 850 406 / 354,
+// 128 x 128 x 1024 463 / 369; so that it is not the fastest shape on meshes of 5 to 8 million.
 constexpr long kFlatNodes = 5000000;
 
 template <typename R, bool NSFD, int TI, int K, bool SC>
@@ -1772,7 +1775,7 @@ template <typename R, bool NSFD, bool SC = false>
 hipError_t stencil_eb_variant(Domain* d, const int* zr, int pb0, int pb1) {
   static_assert(kFusedVariants == 4, "variant table and switch disagree");
   switch (d->tile_fused) {
-    // the flat form up to kFlatNodes, where it takes a third of the tiles' time (see there)
+    // the flat form up to kFlatNodes (see there)
     case 0:
       if (d->nodes < kFlatNodes) return stencil_eb_flat_launch<R, NSFD, SC>(d, zr, pb0, pb1);
       return stencil_eb_launch<R, NSFD, 4, 64, SC>(d, zr, pb0, pb1);
@@ -1901,6 +1904,9 @@ extern const int kTileShapes[kTileVariants][2] = {{0, 8}, {2, 64}, {4, 32}, {4, 
 // 165 us, 128 x 128 x 1024 263 / 323, 211 x 211 x 1531 1273 / 1357) and in FP32 from 16M nodes when
 // the 64-node rows of the tiles waste few lanes (128 x 128 x 1024 186 / 215; but 150 x 150 x 1000
 // 318 flat, 323 tiled).  The 8-row tiles fetch fewer halo rows, the 4-row ones suit ragged meshes.
+// The fused kernel's 4-row tiles are ahead of the 8-row ones below 12 million nodes (128 x 128 x 500 226 / 255, x 670
+// 286 / 324), behind from there where rows fill (x 850 354 / 348, x 970 376 / 368), and ahead on ragged
+// meshes (200 x 210 x 340 521 / 617).
 int default_tile(const Domain* d, int kernel) {
   const int N1 = d->g.N1;
   const bool f64 = d->precision == MITHRA_PRECISION_FP64, aligned = 10 * ((N1 + 63) / 64 * 64) < 11 * N1;
