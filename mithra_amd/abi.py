@@ -297,9 +297,9 @@ class Domain:
         return rc
 
     def close(self):
-        if self.h:
-            self._check(self.f["destroy"](self.h))
-            self.h = C.c_void_p()
+        h, self.h = self.h, None  # before the call: at the interpreter's end this may run a second time
+        if h:
+            self._check(self.f["destroy"](h))
 
     def __del__(self):
         try:
@@ -576,9 +576,9 @@ class DeviceBunch:
         return q
 
     def close(self):
-        if self.h:
-            self.lib.mithra_bunch_destroy(self.h)
-            self.h = C.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.mithra_bunch_destroy(h)
 
     def __del__(self):
         try:
@@ -667,9 +667,9 @@ class Batch:
         return out[:self.slots[i]]
 
     def close(self):
-        if self.h:
-            self.lib.mithra_batch_destroy(self.h)
-            self.h = C.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.mithra_batch_destroy(h)
 
     def __del__(self):
         try:
@@ -773,9 +773,9 @@ class MLP:
         return loss
 
     def close(self):
-        if self.h:
-            self.lib.mithra_mlp_destroy(self.h)
-            self.h = C.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.mithra_mlp_destroy(h)
 
     def __del__(self):
         try:

@@ -79,9 +79,9 @@ class Job:
         return rc
 
     def close(self):
-        if self.h:
-            self.lib.mithra_job_close(self.h)
-            self.h = C.c_void_p()
+        h, self.h = self.h, None
+        if h:
+            self.lib.mithra_job_close(h)
 
     def __del__(self):
         try:
