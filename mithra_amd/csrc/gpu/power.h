@@ -15,9 +15,10 @@
 // keeps what is left of a value far larger than those after it, however the samples are spaced.  A node whose
 // sums are not finite is summed afresh too, and plainly while its ring holds an infinity or a NaN.
 //
-// Walking the ring of 139-152 slots at every step, with one workgroup per 256 nodes, was bound by the latency of those reads on small planes and by the bytes (32 a slot
-// and node) on large ones.  A sample of one frequency, launches back to back: 32 x 32 nodes 24 -> 6.7 us,
-// 128 x 128 35 -> 7.9; in a step of 256 x 256 nodes 89 -> 19 us between events.
+// Walking the ring of 139-152 slots at every step, with one workgroup per 256 nodes, was bound by the
+// latency of those reads on small planes and by the bytes (32 a slot and node) on large ones.  A sample
+// of one frequency, launches back to back: 32 x 32 nodes 24 -> 6.7 us, 128 x 128 35 -> 7.9; in a step of
+// 256 x 256 nodes 89 -> 19 us between events.
 #pragma once
 
 #include "common.h"
