@@ -131,7 +131,10 @@ int stage_listed(HostStage* h, hipStream_t s, long n, size_t unit, long most, si
     const hipError_t idle = hipStreamSynchronize(s);
     return idle == hipSuccess ? MITHRA_OK : MITHRA_E_HIP - (int)idle;
   }
-  if (stage_first(h, (size_t)n * unit, kOnce)) return stage_pageable(h, s, n, unit, most, listed, list, put, take);
+  if (stage_first(h, (size_t)n * unit, kOnce)) {
+    const int rc = stage_pageable(h, s, n, unit, most, listed, list, put, take);
+    if (rc != MITHRA_E_NOMEM) return rc;
+  }
   const size_t want = std::min(std::max((size_t)n * unit / 4, kSlotLow), kSlotHigh);
   const long per = std::min<long>(n, std::max<long>((n + most - 1) / most, (long)(want / unit)));
   const size_t bytes = ((size_t)per * unit + 255) / 256 * 256;

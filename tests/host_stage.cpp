@@ -94,6 +94,10 @@ int main() {
     transfer("little", &h, n);
     mithra::stage_free(&h);
     device_most = 0;
+    pinned_most = ~(size_t)0;
+    transfer("full", &h, n);
+    mithra::stage_free(&h);
+    pinned_most = 0;
     transfer("none", &h, n);
     mithra::stage_free(&h);
     device_most = pinned_most = ~(size_t)0;

@@ -30,10 +30,10 @@ def of(lines, name):
 SIZES = [0, 1, 744, 745, 5957, 5958, 100001]
 
 
-@pytest.mark.parametrize("name", ["first", "pinned", "refused", "little", "granted"])
+@pytest.mark.parametrize("name", ["first", "pinned", "refused", "little", "granted", "full"])
 def test_transfer_comes_through(lines, name):
-    """With pinned memory, without any, with a device that grants 50 kB at most, and with pinned memory granted
-    again after a refusal, whose error no later launch may report."""
+    """With pinned memory, without any, with a device that grants 50 kB at most, with pinned memory granted
+    again after a refusal, whose error no later launch may report, and with pinned memory alone."""
     assert sorted({line[0] for line in of(lines, name)}) == SIZES
     for n, status, good, *_ in of(lines, name):
         assert (status, good) == (OK, 1), (name, n)
